@@ -45,6 +45,7 @@
 #include "../../include/e2.h"
 #include "../../include/e2_dispatch.h"
 #include "common.h"
+#include "gemm_args.h"
 #include "model_internal.h"
 #include "plan.h"
 #include "plan_dev.h"
@@ -161,8 +162,8 @@ struct e2mi_engine {
     std::pair<int, int> slot_shape[kFlagSlots];
     std::map<std::pair<int, int>, int> rows_seen;
     bool packed = true;
-    // (sequences, seq_len, rows, bits: packed 1, split 2, planned on the device 4)
-    std::map<std::tuple<int, int, int, int>, hipGraphExec_t> graphs;
+    // (sequences, seq_len, rows, bits: packed 1, split 2, planned on the device 4, tile_signature above)
+    std::map<std::tuple<int, int, int, long>, hipGraphExec_t> graphs;
     bool use_graph = true;
     bool fuse_qkv = true;  // E2MI_NOFUSE=1: the q|k|v GEMM and the norm/RoPE kernel run separately
     bool fuse_an = true;   // E2MI_NOFUSE_AN=1: the O and down GEMMs and their norm_add run separately
@@ -500,9 +501,9 @@ static int enqueue(e2mi_engine *g, int B, int S, int Mp, bool pk, hipStream_t s,
     return k + 1;  // the pool is two launches
 }
 
-// dev: planned on the device (est: the expected row count, sig: the GEMM tile shapes it gives)
+// dev: planned on the device (est: the expected row count, sig: the kernels it gives)
 static int run_shape(e2mi_engine *g, int B, int S, int Mp, bool pk, hipStream_t s, bool dev = false, int est = 0,
-                     int sig = 0) {
+                     long sig = 0) {
     if (!g->use_graph || g->prof_rec) {
         const int k = enqueue(g, B, S, Mp, pk, s, dev, est);
         if (k < 0) return -1;
@@ -628,29 +629,33 @@ static int plan_pack(e2mi_engine *g, const uint8_t *valid, int n, int S) {
     return Mp;
 }
 
-// The GEMM tile shapes of a device-planned forward of about `est` rows: one bit per distinct output
-// width of the forward's GEMMs whose tile shape follows the row count (gemm_half_tiles)
-static int tile_signature(const e2mi_engine *g, int est) {
-    std::vector<int> ns;
+// The kernels of a device-planned forward of about `est` rows: for every distinct GEMM of the forward
+// whose kernel follows the row count, which one takes it (gemm_small_route, gemm_half_tiles), and
+// whether the projections run with their norm_add and in how many row units per workgroup (1-5)
+static long tile_signature(const e2mi_engine *g, int est) {
+    const e2_config &c = g->cfg;
     const bool an = gemm_an_fits(est);
+    std::vector<std::tuple<int, int, int>> gemms;  // N, K, epilogue
+    auto add = [&](const e2mi_q8w &w, int epi) { gemms.emplace_back(w.N, w.K, epi); };
     for (const LayerDev &L : g->layers) {
-        if (!(L.o_an && an)) ns.push_back(L.o.N);
-        if (!(L.down_an && an)) ns.push_back(L.down.N);
-        if (!L.qkv_fused) ns.push_back(L.qkv.N);
-        if (g->cfg.ple_dim > 0) {
-            ns.push_back(L.ple_gate.N);
-            if (!(L.down_an && an)) ns.push_back(L.ple_proj.N);
+        add(L.qkv, L.qkv_fused ? EPI_QKV : EPI_F32);
+        add(L.gu, EPI_GEGLU);
+        if (!(L.o_an && an)) add(L.o, EPI_F32);
+        if (!(L.down_an && an)) add(L.down, EPI_F32);
+        if (c.ple_dim > 0) {
+            add(L.ple_gate, EPI_GELUMUL);
+            if (!(L.down_an && an)) add(L.ple_proj, EPI_F32);
         }
     }
-    if (g->cfg.ple_dim > 0) ns.push_back(g->ple_model.N);
-    if (g->cfg.out_dim > 0) ns.push_back(g->embed_proj.N);
-    std::sort(ns.begin(), ns.end());
-    ns.erase(std::unique(ns.begin(), ns.end()), ns.end());
-    int sig = 0;
-    for (size_t i = 0; i < ns.size(); i++)
-        if (gemm_half_tiles(est, ns[i])) sig |= 1 << i;
-    // whether the GEMMs with the norm_add run, and their row units per workgroup (1-5), in the bits above
-    if (!g->layers.empty() && g->layers[0].o_an && an) sig |= 1 << 15 | gemm_an_units(est) << 16;
+    if (c.ple_dim > 0) add(g->ple_model, EPI_F32);
+    if (c.out_dim > 0) add(g->embed_proj, EPI_F32);
+    std::sort(gemms.begin(), gemms.end());
+    gemms.erase(std::unique(gemms.begin(), gemms.end()), gemms.end());
+    long sig = !g->layers.empty() && g->layers[0].o_an && an ? gemm_an_units(est) : 0;
+    for (const auto &[N, K, epi] : gemms) {  // at most 14 of them, 3 bits each
+        const int small = gemm_small_route(est, N, K, epi, false);
+        sig = sig << 3 | (small ? small : gemm_half_tiles(est, N) ? 4 : 0);
+    }
     return sig;
 }
 

@@ -33,49 +33,9 @@
 #include <stddef.h>
 
 #include "common.h"
+#include "gemm_args.h"
 
 namespace e2mi {
-
-enum { EPI_F32 = 0, EPI_I8Q = 1, EPI_GEGLU = 2, EPI_GELUMUL = 3, EPI_QKV = 4 };
-
-struct GemmArgs {
-    const int8_t *A;
-    const float *as;
-    const int8_t *W;
-    const float *ws;
-    const float *bias;
-    float *Y;        // EPI_F32 output, EPI_GEGLU optional f32 g
-    int8_t *Yq;      // EPI_I8Q / EPI_GEGLU quantized output
-    float *ys;       // ... and its per-128 scales [M][ldys]
-    int32_t *accd;   // optional int32 accumulator dump [nb][M][N] (parity tests)
-    const float *mul;  // EPI_GELUMUL: the multiplier of gelu(y) [M][ldmul]
-    int ldmul;
-    int lda, ldw, ldy, ldyq, ldys;
-    int M, N, K;
-    float lo, hi;
-    // EPI_QKV: q/k gammas [256], RoPE tables [positions][256], each row's position (packed
-    // batches) or none (row % qS), f16 outputs q [M][qH*256], k [M][qKV*256] and V^T
-    // [M/qS][qKV][256][qS], optional f32 copies q, k, v [M][heads*256]
-    const float *q_gamma, *k_gamma, *cs, *sn;
-    const int32_t *pos;
-    uint16_t *q16, *k16, *vt16;
-    float *q32, *k32, *v32;
-    int qH, qKV, qS;
-    float eps;
-    // a device row count (a multiple of 256, at most M; k_gemm_p only, which takes it as its own
-    // first argument), or null: M rows
-    const int *rows;
-};
-
-
-// LDS tiles hold 128-byte K slices of consecutive rows with no padding. The LDS has 64 banks of 4
-// bytes and serves a ds_read_b128 16 lanes at a time; a 128-byte row spans 32 banks, so rows of
-// equal parity share a bank half. The 16-byte chunk c of row r sits at slot c ^ ((r >> 1) & 7):
-// the 16 consecutive rows read by one 16-lane group then cover all 64 banks once. Each
-// 1-KB direct-to-LDS load fills 8 rows of a tile: lane l writes slot l, so it fetches row l/8's
-// chunk (l % 8) ^ ((row >> 1) & 7).
-__device__ inline int swzk(int r) { return (r >> 1) & 7; }
-__device__ inline int swz(int r, int c) { return r * 128 + ((c ^ swzk(r)) << 4); }
 
 // Buffer loads straight into LDS: the per-lane offset is a VGPR fixed for the whole K loop and the
 // K step's offset a scalar, so a step costs no VALU address arithmetic. (Device functions rather
@@ -1899,6 +1859,14 @@ static bool half_tiles(const GemmArgs &p) {
     return gemm_half_tiles(est > 0 && est < p.M ? est : p.M, p.N);
 }
 
+static int expected_rows(const GemmArgs &p) {
+    const int est = p.rows ? device_rows().est : 0;
+    return est > 0 && est < p.M ? est : p.M;
+}
+// the kernels for few rows (gemm_s.hip) where they are the faster ones
+#define E2MI_TRY_SMALL(epi, tok)                                                                   \
+    if (const int rc = launch_gemm_small(s, p, epi, expected_rows(p), tok)) return rc < 0 ? -1 : 0
+
 int launch_gemm_f32(hipStream_t s, GemmArgs p, bool dump, bool tok = false) {
     if (check_args(p, "i8_gemm", !dump && !tok)) return -1;
     if (!p.Y || p.ldy < p.N) {
@@ -1912,6 +1880,7 @@ int launch_gemm_f32(hipStream_t s, GemmArgs p, bool dump, bool tok = false) {
         }
         return launch_dump(s, p);
     }
+    E2MI_TRY_SMALL(EPI_F32, tok);
     if (tok) return launch_t<EPI_F32>(s, p);
     if (half_tiles(p)) return launch_p<128, 128, 4, 1, EPI_F32>(s, p);
     return launch_p<256, 128, 8, 1, EPI_F32>(s, p);
@@ -1924,6 +1893,7 @@ int launch_gemm_i8q(hipStream_t s, GemmArgs p, bool tok = false) {
         set_error("i8_gemm_q: N must be a multiple of 128 with a 16-byte aligned int8 output");
         return -1;
     }
+    E2MI_TRY_SMALL(EPI_I8Q, tok);
     if (tok) return launch_t<EPI_I8Q>(s, p);
     if (half_tiles(p)) return launch_p<128, 128, 4, 1, EPI_I8Q>(s, p);
     return launch_p<256, 128, 8, 1, EPI_I8Q>(s, p);
@@ -1937,6 +1907,7 @@ int launch_gemm_gelumul(hipStream_t s, GemmArgs p) {
         set_error("i8_gemm_gelu_mul: N must be a multiple of 128; outputs and multiplier 16-byte aligned");
         return -1;
     }
+    E2MI_TRY_SMALL(EPI_GELUMUL, false);
     if (half_tiles(p)) return launch_p<128, 128, 4, 1, EPI_GELUMUL>(s, p);
     return launch_p<256, 128, 8, 1, EPI_GELUMUL>(s, p);
 }
@@ -1948,6 +1919,7 @@ int launch_gemm_geglu(hipStream_t s, GemmArgs p) {
         set_error("i8_gemm_geglu: N (gate|up interleaved) must be a multiple of 256, outputs aligned");
         return -1;
     }
+    E2MI_TRY_SMALL(EPI_GEGLU, false);
     // 128 x 256 tiles: a tile holds the interleaved gate|up columns of one output block
     return launch_p<128, 256, 4, 2, EPI_GEGLU>(s, p);
 }
@@ -1976,6 +1948,7 @@ int launch_gemm_qkv(hipStream_t s, GemmArgs p) {
                   p.qH > p.qKV ? p.qH : p.qKV);
         return -1;
     }
+    E2MI_TRY_SMALL(EPI_QKV, false);
     // 128 x 256 tiles: a tile is one head of 128 rows
     return launch_p<128, 256, 4, 2, EPI_QKV>(s, p);
 }

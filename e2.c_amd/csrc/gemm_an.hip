@@ -377,7 +377,19 @@ static int launch_an(hipStream_t s, const int *rows, const AnArgs &a, int grid, 
     }
 }
 
+// Whether the projection and its norm_add run as two launches (gemm_s.hip's GEMM, then the row kernel)
+// at a row count: below about a million outputs a workgroup of k_gemm_an reads the whole weight for
+// its 16 rows (0.6-1 MB at the 64 B a clock a CU loads: 5-8 us) while most CUs have none. 768 columns,
+// two launches | one: K = 768 7.1 | 12.5 us at 32 rows, 10.7 | 13.1 at 1024, 15.4 | 13.9 at 2048;
+// K = 1152 7.5 | 15.5, 12.8 | 16.4, 18.4 | 18.2; 512 columns: K = 1024 6.8 | 11.5, 9.9 | 13.2, 13.2 |
+// 13.9; K = 2048 7.8 | 18.2, 14.2 | 21.0, 17.4 | 21.5.
+bool gemm_an_split(int rows, int D) { return (long)rows * D <= 1 << 20; }
+
 bool gemm_fold_fast();
+// rowops.hip: the row kernel with k_gemm_an's byte packing
+int launch_add_norm(hipStream_t s, const float *src, const float *res, const float *gamma_add, float post_scale,
+                    const float *gamma_next, float eps, int M, int D, float *x_out, float *xn_out, int8_t *q,
+                    float *qs, bool scale);
 
 // The two entry points' checks and launch. SCALE: the norm_add of the reference checkpoint's PLE
 // layers (x scaled after the add; without gamma_next, x itself quantized).
@@ -420,6 +432,17 @@ static int gemm_add_norm(hipStream_t s, const int8_t *qa, const float *a_scales,
     a.gamma_n = gamma_next; a.x_out = x_out; a.xn_out = xn_out; a.q = q; a.qs = qs; a.y = y;
     a.lda = w->K; a.ldw = w->ld; a.M = M; a.K = w->K; a.eps = eps; a.post_scale = post_scale;
     const int est = dr.ptr && dr.est > 0 && dr.est < M ? dr.est : M;
+    if (gemm_an_split(est, D)) {
+        // the projection goes through y, or through x_out beside the residual, which the row kernel then
+        // overwrites row by row
+        const size_t n = (size_t)M * D;
+        auto apart = [&](const float *t) { return t && (t + n <= res || res + n <= t); };
+        float *t = apart(y) ? y : apart(x_out) ? x_out : nullptr;
+        if (t)
+            return e2mi_i8_gemm(s, t, D, qa, a_scales, w, M, 0, D) ||
+                           launch_add_norm(s, t, res, gamma_add, post_scale, gamma_next, eps, M, D, x_out, xn_out, q, qs, scale)
+                       ? -1 : 0;
+    }
     const int uc = gemm_an_units(est);
     const int grid = ((M + 15) / 16 + uc - 1) / uc;
     const bool fast = gemm_fold_fast();

@@ -45,6 +45,7 @@ struct RowArgs {
     float post_scale = 1.f;  // ADDNORM: x scaled after the add (layer_scalar, text.c:959)
     const int *rows = nullptr;  // device row count (times rows_mul, at most M), or null: M
     int rows_mul = 1;
+    bool magic = false;  // ADDNORM/ADDSCALE: bytes packed as k_gemm_an does (the same bytes but for NaN rows)
 };
 
 // NC = float4 chunks per lane = D / 256 (rounded up); chunk i of lane l covers elements
@@ -121,8 +122,10 @@ __global__ __launch_bounds__(256) void k_rows(RowArgs a) {
         if (c < nch) {
             const QScale s = qscale(am);
             *(uint32_t *)(a.q + (size_t)m * D + 4 * c) =
-                pack4(qbyte(v[i].x, s.inv), qbyte(v[i].y, s.inv), qbyte(v[i].z, s.inv),
-                      qbyte(v[i].w, s.inv));
+                (MODE == ROW_ADDNORM || MODE == ROW_ADDSCALE) && a.magic
+                    ? pack4_magic(v[i].x, v[i].y, v[i].z, v[i].w, s.inv)
+                    : pack4(qbyte(v[i].x, s.inv), qbyte(v[i].y, s.inv), qbyte(v[i].z, s.inv),
+                            qbyte(v[i].w, s.inv));
             if ((l & 31) == 0) a.qs[(size_t)m * nb + (4 * c) / kQBlock] = s.sc;
         }
     }
@@ -458,6 +461,16 @@ static int row_launch(hipStream_t s, int mode, const RowArgs &a) {
 }
 
 int launch_rows(hipStream_t s, int mode, const RowArgs &a) { return row_launch(s, mode, a); }
+
+// the norm_add of a projection that gemm_an.hip runs as two launches (its checks made there)
+int launch_add_norm(hipStream_t s, const float *src, const float *res, const float *gamma_add, float post_scale,
+                    const float *gamma_next, float eps, int M, int D, float *x_out, float *xn_out, int8_t *q,
+                    float *qs, bool scale) {
+    RowArgs a = {};
+    a.src = src; a.res = res; a.gamma_a = gamma_add; a.gamma_n = gamma_next; a.eps = eps; a.post_scale = post_scale;
+    a.x_out = x_out; a.xn_out = xn_out; a.q = q; a.qs = qs; a.M = M; a.D = D; a.magic = true;
+    return row_launch(s, scale ? ROW_ADDSCALE : ROW_ADDNORM, a);
+}
 
 int launch_qkv_norm_rope(hipStream_t s, const QkvArgs &qa, int D) {
     QkvArgs a = qa;
