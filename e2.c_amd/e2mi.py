@@ -255,13 +255,36 @@ def set_gemm_fold(mode: str) -> str:
 
 
 # ---- kernel wrappers over torch device tensors
+# A call on few rows takes the GPU 3-5 us, less than the host's time to make it: the stream is taken as
+# its raw handle and addresses go to ctypes as plain ints (declared c_void_p in SIGNATURES), which
+# halves a wrapper's own time (torch.cuda.current_stream() alone builds a Stream object per call).
+def _stream(stream):
+    if stream is not None:
+        return stream.cuda_stream
+    import torch
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
+def _p(t):
+    return None if t is None else t.data_ptr()
+
+
+def _gemm_out(qa, w, n0, n1):
+    """A GEMM's own output: columns outside [n0, n1) read zero."""
+    import torch
+    shape = (qa.shape[0], w.q.N)
+    if n0 == 0 and n1 == w.q.N:
+        return qa.new_empty(shape, dtype=torch.float32)
+    return torch.zeros(shape, dtype=torch.float32, device=qa.device)
+
+
 def quantize(x, block=128, q=None, scales=None, stream=None):
     import torch
     M, K = x.shape
-    q = torch.empty((M, K), dtype=torch.int8, device=x.device) if q is None else q
+    q = x.new_empty((M, K), dtype=torch.int8) if q is None else q
     nb = K // block
-    scales = torch.empty((M, nb), dtype=torch.float32, device=x.device) if scales is None else scales
-    check(load().e2mi_quantize(stream_ptr(stream), ptr(q), ptr(scales), ptr(x), M, K, x.stride(0),
+    scales = x.new_empty((M, nb), dtype=torch.float32) if scales is None else scales
+    check(load().e2mi_quantize(_stream(stream), _p(q), _p(scales), _p(x), M, K, x.stride(0),
                                block), "quantize")
     return q, scales
 
@@ -270,8 +293,9 @@ def i8_gemm(qa, as_, w: DeviceWeight, n0=0, n1=None, y=None, stream=None):
     import torch
     M = qa.shape[0]
     n1 = w.q.N if n1 is None else n1
-    y = torch.zeros((M, w.q.N), dtype=torch.float32, device=qa.device) if y is None else y
-    check(load().e2mi_i8_gemm(stream_ptr(stream), ptr(y), y.stride(0), ptr(qa), ptr(as_), w.ref, M,
+    if y is None:
+        y = _gemm_out(qa, w, n0, n1)
+    check(load().e2mi_i8_gemm(_stream(stream), _p(y), y.stride(0), _p(qa), _p(as_), w.ref, M,
                               n0, n1), "i8_gemm")
     return y
 
@@ -282,17 +306,17 @@ def i8_gemm_acc(qa, as_, w: DeviceWeight, n0=0, n1=None, stream=None):
     n1 = w.q.N if n1 is None else n1
     y = torch.zeros((M, w.q.N), dtype=torch.float32, device=qa.device)
     acc = torch.zeros((w.q.K // 128, M, n1 - n0), dtype=torch.int32, device=qa.device)
-    check(load().e2mi_i8_gemm_acc(stream_ptr(stream), ptr(y), y.stride(0), ptr(acc), ptr(qa),
-                                  ptr(as_), w.ref, M, n0, n1), "i8_gemm_acc")
+    check(load().e2mi_i8_gemm_acc(_stream(stream), _p(y), y.stride(0), _p(acc), _p(qa),
+                                  _p(as_), w.ref, M, n0, n1), "i8_gemm_acc")
     return y, acc
 
 
 def i8_gemm_q(qa, as_, w: DeviceWeight, stream=None):
     import torch
     M = qa.shape[0]
-    yq = torch.empty((M, w.q.N), dtype=torch.int8, device=qa.device)
-    ys = torch.empty((M, w.q.N // 128), dtype=torch.float32, device=qa.device)
-    check(load().e2mi_i8_gemm_q(stream_ptr(stream), ptr(yq), ptr(ys), ptr(qa), ptr(as_), w.ref, M),
+    yq = qa.new_empty((M, w.q.N), dtype=torch.int8)
+    ys = qa.new_empty((M, w.q.N // 128), dtype=torch.float32)
+    check(load().e2mi_i8_gemm_q(_stream(stream), _p(yq), _p(ys), _p(qa), _p(as_), w.ref, M),
           "i8_gemm_q")
     return yq, ys
 
@@ -302,8 +326,9 @@ def i8_gemm_tok(qa, as_, w: DeviceWeight, n0=0, n1=None, y=None, stream=None):
     import torch
     M = qa.shape[0]
     n1 = w.q.N if n1 is None else n1
-    y = torch.zeros((M, w.q.N), dtype=torch.float32, device=qa.device) if y is None else y
-    check(load().e2mi_i8_gemm_tok(stream_ptr(stream), ptr(y), y.stride(0), ptr(qa), ptr(as_), w.ref,
+    if y is None:
+        y = _gemm_out(qa, w, n0, n1)
+    check(load().e2mi_i8_gemm_tok(_stream(stream), _p(y), y.stride(0), _p(qa), _p(as_), w.ref,
                                   M, n0, n1), "i8_gemm_tok")
     return y
 
@@ -311,9 +336,9 @@ def i8_gemm_tok(qa, as_, w: DeviceWeight, n0=0, n1=None, y=None, stream=None):
 def i8_gemm_tok_q(qa, as_, w: DeviceWeight, stream=None):
     import torch
     M = qa.shape[0]
-    yq = torch.empty((M, w.q.N), dtype=torch.int8, device=qa.device)
-    ys = torch.empty((M, w.q.N // 128), dtype=torch.float32, device=qa.device)
-    check(load().e2mi_i8_gemm_tok_q(stream_ptr(stream), ptr(yq), ptr(ys), ptr(qa), ptr(as_), w.ref, M),
+    yq = qa.new_empty((M, w.q.N), dtype=torch.int8)
+    ys = qa.new_empty((M, w.q.N // 128), dtype=torch.float32)
+    check(load().e2mi_i8_gemm_tok_q(_stream(stream), _p(yq), _p(ys), _p(qa), _p(as_), w.ref, M),
           "i8_gemm_tok_q")
     return yq, ys
 
@@ -324,11 +349,11 @@ def i8_gemm_gelu_mul(qa, as_, w: DeviceWeight, mul, want_g=True, stream=None):
     import torch
     M = qa.shape[0]
     N = w.q.N
-    q = torch.empty((M, N), dtype=torch.int8, device=qa.device)
-    qs = torch.empty((M, N // 128), dtype=torch.float32, device=qa.device)
-    g = torch.empty((M, N), dtype=torch.float32, device=qa.device) if want_g else None
-    check(load().e2mi_i8_gemm_gelu_mul(stream_ptr(stream), ptr(q), ptr(qs), ptr(g), ptr(qa), ptr(as_),
-                                       w.ref, M, ptr(mul), mul.stride(0)), "i8_gemm_gelu_mul")
+    q = qa.new_empty((M, N), dtype=torch.int8)
+    qs = qa.new_empty((M, N // 128), dtype=torch.float32)
+    g = qa.new_empty((M, N), dtype=torch.float32) if want_g else None
+    check(load().e2mi_i8_gemm_gelu_mul(_stream(stream), _p(q), _p(qs), _p(g), _p(qa), _p(as_),
+                                       w.ref, M, _p(mul), mul.stride(0)), "i8_gemm_gelu_mul")
     return q, qs, g
 
 
@@ -336,10 +361,10 @@ def i8_gemm_geglu(qa, as_, w: DeviceWeight, want_g=True, stream=None):
     import torch
     M = qa.shape[0]
     F = w.q.N // 2
-    q = torch.empty((M, F), dtype=torch.int8, device=qa.device)
-    qs = torch.empty((M, F // 128), dtype=torch.float32, device=qa.device)
-    g = torch.empty((M, F), dtype=torch.float32, device=qa.device) if want_g else None
-    check(load().e2mi_i8_gemm_geglu(stream_ptr(stream), ptr(q), ptr(qs), ptr(g), ptr(qa), ptr(as_),
+    q = qa.new_empty((M, F), dtype=torch.int8)
+    qs = qa.new_empty((M, F // 128), dtype=torch.float32)
+    g = qa.new_empty((M, F), dtype=torch.float32) if want_g else None
+    check(load().e2mi_i8_gemm_geglu(_stream(stream), _p(q), _p(qs), _p(g), _p(qa), _p(as_),
                                     w.ref, M), "i8_gemm_geglu")
     return q, qs, g
 
@@ -349,10 +374,10 @@ def norm_quant(x, gamma, eps=1e-6, want_xn=True, quant=True, stream=None):
     import torch
     M, D = x.shape
     xn = torch.empty_like(x) if want_xn else None
-    q = torch.empty((M, D), dtype=torch.int8, device=x.device) if quant else None
-    qs = torch.empty((M, D // 128), dtype=torch.float32, device=x.device) if quant else None
-    check(load().e2mi_norm_quant(stream_ptr(stream), ptr(x), ptr(gamma), eps, M, D, ptr(xn), ptr(q),
-                                 ptr(qs)), "norm_quant")
+    q = x.new_empty((M, D), dtype=torch.int8) if quant else None
+    qs = x.new_empty((M, D // 128), dtype=torch.float32) if quant else None
+    check(load().e2mi_norm_quant(_stream(stream), _p(x), _p(gamma), eps, M, D, _p(xn), _p(q),
+                                 _p(qs)), "norm_quant")
     return xn, q, qs
 
 
@@ -363,11 +388,11 @@ def add_norm_quant(src, res, gamma_add, gamma_next=None, eps=1e-6, x_out=None, w
     x_out = torch.empty_like(src) if x_out is None else x_out
     has_next = gamma_next is not None
     xn = torch.empty_like(src) if (want_xn and has_next) else None
-    q = torch.empty((M, D), dtype=torch.int8, device=src.device) if (quant and has_next) else None
-    qs = torch.empty((M, D // 128), dtype=torch.float32, device=src.device) if q is not None else None
-    check(load().e2mi_add_norm_quant(stream_ptr(stream), ptr(src), ptr(res), ptr(gamma_add),
-                                     ptr(gamma_next), eps, M, D, ptr(x_out), ptr(xn), ptr(q),
-                                     ptr(qs)), "add_norm_quant")
+    q = src.new_empty((M, D), dtype=torch.int8) if (quant and has_next) else None
+    qs = src.new_empty((M, D // 128), dtype=torch.float32) if q is not None else None
+    check(load().e2mi_add_norm_quant(_stream(stream), _p(src), _p(res), _p(gamma_add),
+                                     _p(gamma_next), eps, M, D, _p(x_out), _p(xn), _p(q),
+                                     _p(qs)), "add_norm_quant")
     return x_out, xn, q, qs
 
 
@@ -380,12 +405,12 @@ def i8_gemm_add_norm_quant(qa, as_, w: DeviceWeight, res, gamma_add, gamma_next=
     x_out = torch.empty_like(res) if x_out is None else x_out
     has_next = gamma_next is not None
     xn = torch.empty_like(res) if (want_xn and has_next) else None
-    q = torch.empty((M, D), dtype=torch.int8, device=res.device) if (quant and has_next) else None
-    qs = torch.empty((M, D // 128), dtype=torch.float32, device=res.device) if q is not None else None
+    q = res.new_empty((M, D), dtype=torch.int8) if (quant and has_next) else None
+    qs = res.new_empty((M, D // 128), dtype=torch.float32) if q is not None else None
     y = torch.empty_like(res) if want_y else None
-    check(load().e2mi_i8_gemm_add_norm_quant(stream_ptr(stream), ptr(qa), ptr(as_), w.ref, M, ptr(res),
-                                             ptr(gamma_add), ptr(gamma_next), eps, ptr(x_out), ptr(xn),
-                                             ptr(q), ptr(qs), ptr(y)), "i8_gemm_add_norm_quant")
+    check(load().e2mi_i8_gemm_add_norm_quant(_stream(stream), _p(qa), _p(as_), w.ref, M, _p(res),
+                                             _p(gamma_add), _p(gamma_next), eps, _p(x_out), _p(xn),
+                                             _p(q), _p(qs), _p(y)), "i8_gemm_add_norm_quant")
     return x_out, xn, q, qs, y
 
 
@@ -398,12 +423,12 @@ def i8_gemm_add_norm_scale_quant(qa, as_, w: DeviceWeight, res, gamma_add, post_
     x_out = torch.empty_like(res) if x_out is None else x_out
     has_next = gamma_next is not None
     xn = torch.empty_like(res) if (want_xn and has_next) else None
-    q = torch.empty((M, D), dtype=torch.int8, device=res.device) if quant else None
-    qs = torch.empty((M, D // 128), dtype=torch.float32, device=res.device) if quant else None
+    q = res.new_empty((M, D), dtype=torch.int8) if quant else None
+    qs = res.new_empty((M, D // 128), dtype=torch.float32) if quant else None
     y = torch.empty_like(res) if want_y else None
-    check(load().e2mi_i8_gemm_add_norm_scale_quant(stream_ptr(stream), ptr(qa), ptr(as_), w.ref, M, ptr(res),
-                                                   ptr(gamma_add), post_scale, ptr(gamma_next), eps, ptr(x_out),
-                                                   ptr(xn), ptr(q), ptr(qs), ptr(y)),
+    check(load().e2mi_i8_gemm_add_norm_scale_quant(_stream(stream), _p(qa), _p(as_), w.ref, M, _p(res),
+                                                   _p(gamma_add), post_scale, _p(gamma_next), eps, _p(x_out),
+                                                   _p(xn), _p(q), _p(qs), _p(y)),
           "i8_gemm_add_norm_scale_quant")
     return x_out, xn, q, qs, y
 
@@ -412,11 +437,11 @@ def embed_norm_quant(table, ids, embed_scale, gamma, eps=1e-6, stream=None):
     import torch
     M = ids.shape[0]
     V, D = table.shape
-    x = torch.empty((M, D), dtype=torch.float32, device=table.device)
-    q = torch.empty((M, D), dtype=torch.int8, device=table.device)
-    qs = torch.empty((M, D // 128), dtype=torch.float32, device=table.device)
-    check(load().e2mi_embed_norm_quant(stream_ptr(stream), ptr(table), V, ptr(ids), embed_scale,
-                                       ptr(gamma), eps, M, D, ptr(x), ptr(q), ptr(qs)),
+    x = table.new_empty((M, D), dtype=torch.float32)
+    q = table.new_empty((M, D), dtype=torch.int8)
+    qs = table.new_empty((M, D // 128), dtype=torch.float32)
+    check(load().e2mi_embed_norm_quant(_stream(stream), _p(table), V, _p(ids), embed_scale,
+                                       _p(gamma), eps, M, D, _p(x), _p(q), _p(qs)),
           "embed_norm_quant")
     return x, q, qs
 
@@ -433,9 +458,9 @@ def qkv_norm_rope(qkv, S, H, KV, q_gamma, k_gamma, cos_tab, sin_tab, eps=1e-6, w
     vt16 = torch.empty((B, KV, D, S), dtype=torch.float16, device=dev)
     f = (lambda *s: torch.empty(s, dtype=torch.float32, device=dev)) if want_f32 else (lambda *s: None)
     q32, k32, v32 = f(M, H * D), f(M, KV * D), f(M, KV * D)
-    check(load().e2mi_qkv_norm_rope(stream_ptr(stream), ptr(qkv), M, S, H, KV, D, ptr(q_gamma),
-                                    ptr(k_gamma), eps, ptr(cos_tab), ptr(sin_tab), ptr(q16),
-                                    ptr(k16), ptr(vt16), ptr(q32), ptr(k32), ptr(v32)),
+    check(load().e2mi_qkv_norm_rope(_stream(stream), _p(qkv), M, S, H, KV, D, _p(q_gamma),
+                                    _p(k_gamma), eps, _p(cos_tab), _p(sin_tab), _p(q16),
+                                    _p(k16), _p(vt16), _p(q32), _p(k32), _p(v32)),
           "qkv_norm_rope")
     return q16, k16, vt16, q32, k32, v32
 
@@ -462,19 +487,19 @@ def i8_gemm_qkv(qa, as_, w: DeviceWeight, H, KV, q_gamma, k_gamma, cos_tab, sin_
     vt16 = torch.empty((M // S, KV, D, S), dtype=torch.float16, device=dev)
     f = (lambda *s: torch.empty(s, dtype=torch.float32, device=dev)) if want_f32 else (lambda *s: None)
     q32, k32, v32 = f(M, H * D), f(M, KV * D), f(M, KV * D)
-    check(load().e2mi_i8_gemm_qkv(stream_ptr(stream), ptr(qa), ptr(as_), w.ref, M, S, ptr(pos), H, KV,
-                                  ptr(q_gamma), ptr(k_gamma), eps, ptr(cos_tab), ptr(sin_tab), ptr(q16),
-                                  ptr(k16), ptr(vt16), ptr(q32), ptr(k32), ptr(v32)), "i8_gemm_qkv")
+    check(load().e2mi_i8_gemm_qkv(_stream(stream), _p(qa), _p(as_), w.ref, M, S, _p(pos), H, KV,
+                                  _p(q_gamma), _p(k_gamma), eps, _p(cos_tab), _p(sin_tab), _p(q16),
+                                  _p(k16), _p(vt16), _p(q32), _p(k32), _p(v32)), "i8_gemm_qkv")
     return q16, k16, vt16, q32, k32, v32
 
 
 def gelu_mul_quant(gate, up, write_back=True, stream=None):
     import torch
     M, D = gate.shape
-    q = torch.empty((M, D), dtype=torch.int8, device=gate.device)
-    qs = torch.empty((M, D // 128), dtype=torch.float32, device=gate.device)
-    check(load().e2mi_gelu_mul_quant(stream_ptr(stream), ptr(gate), gate.stride(0), ptr(up),
-                                     up.stride(0), M, D, ptr(q), ptr(qs), int(write_back)),
+    q = gate.new_empty((M, D), dtype=torch.int8)
+    qs = gate.new_empty((M, D // 128), dtype=torch.float32)
+    check(load().e2mi_gelu_mul_quant(_stream(stream), _p(gate), gate.stride(0), _p(up),
+                                     up.stride(0), M, D, _p(q), _p(qs), int(write_back)),
           "gelu_mul_quant")
     return q, qs
 
@@ -485,8 +510,8 @@ def pool_l2(x, valid, B, S, stream=None):
     lib = load()
     ws = torch.empty(lib.e2mi_pool_workspace_bytes(B, S, D) // 4 + 64, dtype=torch.float32,
                      device=x.device)
-    out = torch.empty((B, D), dtype=torch.float32, device=x.device)
-    check(lib.e2mi_pool_l2(stream_ptr(stream), ptr(x), ptr(valid), B, S, D, ptr(ws), ptr(out)),
+    out = x.new_empty((B, D), dtype=torch.float32)
+    check(lib.e2mi_pool_l2(_stream(stream), _p(x), _p(valid), B, S, D, _p(ws), _p(out)),
           "pool_l2")
     return out
 
@@ -499,8 +524,8 @@ def attention(q16, k16, vt16, valid, B, S, H, KV, scale=1.0, want_f32=True, stre
     cq = torch.empty((M, H * D), dtype=torch.int8, device=dev)
     cs = torch.empty((M, H * D // 128), dtype=torch.float32, device=dev)
     c32 = torch.empty((M, H * D), dtype=torch.float32, device=dev) if want_f32 else None
-    check(load().e2mi_attention(stream_ptr(stream), ptr(q16), ptr(k16), ptr(vt16), ptr(valid), B, S,
-                                H, KV, D, scale, ptr(cq), ptr(cs), ptr(c32)), "attention")
+    check(load().e2mi_attention(_stream(stream), _p(q16), _p(k16), _p(vt16), _p(valid), B, S,
+                                H, KV, D, scale, _p(cq), _p(cs), _p(c32)), "attention")
     return cq, cs, c32
 
 
@@ -530,10 +555,10 @@ def qkv_norm_rope_packed(qkv, pos, H, KV, q_gamma, k_gamma, cos_tab, sin_tab, ep
     vt16 = torch.empty((KV, D, M), dtype=torch.float16, device=dev)
     f = (lambda *s: torch.empty(s, dtype=torch.float32, device=dev)) if want_f32 else (lambda *s: None)
     q32, k32, v32 = f(M, H * D), f(M, KV * D), f(M, KV * D)
-    check(load().e2mi_qkv_norm_rope_packed(stream_ptr(stream), ptr(qkv), M, ptr(pos), H, KV, D,
-                                           ptr(q_gamma), ptr(k_gamma), eps, ptr(cos_tab),
-                                           ptr(sin_tab), ptr(q16), ptr(k16), ptr(vt16), ptr(q32),
-                                           ptr(k32), ptr(v32)), "qkv_norm_rope_packed")
+    check(load().e2mi_qkv_norm_rope_packed(_stream(stream), _p(qkv), M, _p(pos), H, KV, D,
+                                           _p(q_gamma), _p(k_gamma), eps, _p(cos_tab),
+                                           _p(sin_tab), _p(q16), _p(k16), _p(vt16), _p(q32),
+                                           _p(k32), _p(v32)), "qkv_norm_rope_packed")
     return q16, k16, vt16, q32, k32, v32
 
 
@@ -575,9 +600,9 @@ def plan_device(valid, H, window=0, div=2, ids=None, n_slots=None, stream=None):
     i32 = lambda n: torch.full((n,), -7, dtype=torch.int32, device=dev)
     rowmap, pos, start, lens, work, rows = i32(cap), i32(cap), i32(B), i32(B), i32(n_slots), i32(1)
     ids_out = i32(cap) if ids is not None else None
-    check(load().e2mi_plan_device(stream_ptr(stream), ptr(valid), ptr(ids), B, S, H, window, div, n_slots,
-                                  ptr(rowmap), ptr(pos), ptr(start), ptr(lens), ptr(ids_out), ptr(work),
-                                  ptr(rows)), "plan_device")
+    check(load().e2mi_plan_device(_stream(stream), _p(valid), _p(ids), B, S, H, window, div, n_slots,
+                                  _p(rowmap), _p(pos), _p(start), _p(lens), _p(ids_out), _p(work),
+                                  _p(rows)), "plan_device")
     M = int(rows.item())
     return (rowmap[:M], pos[:M], start, lens, M, work, None if ids_out is None else ids_out[:M])
 
@@ -604,10 +629,10 @@ def attention_packed_split(q16, k16, vt16, start, lens, max_len, H, KV, work, me
     part = torch.empty(nb // 4, dtype=torch.float32, device=dev)
     wt = torch.from_numpy(work).to(dev)
     mt = torch.from_numpy(merge).to(dev)
-    check(load().e2mi_attention_packed_split(stream_ptr(stream), ptr(q16), ptr(k16), ptr(vt16), M, ptr(start),
-                                             ptr(lens), ptr(pos), start.shape[0], max_len, H, KV, D, scale,
-                                             window, ptr(cq), ptr(cs), ptr(c32), ptr(wt), wt.shape[0], ptr(mt),
-                                             mt.shape[0], ptr(part), M), "attention_packed_split")
+    check(load().e2mi_attention_packed_split(_stream(stream), _p(q16), _p(k16), _p(vt16), M, _p(start),
+                                             _p(lens), _p(pos), start.shape[0], max_len, H, KV, D, scale,
+                                             window, _p(cq), _p(cs), _p(c32), _p(wt), wt.shape[0], _p(mt),
+                                             mt.shape[0], _p(part), M), "attention_packed_split")
     return cq, cs, c32
 
 
@@ -621,9 +646,9 @@ def attention_packed(q16, k16, vt16, start, lens, max_len, H, KV, scale=1.0, wan
     cs = torch.zeros((M, H * D // 128), dtype=torch.float32, device=dev) if cs is None else cs
     if want_f32 and c32 is None:
         c32 = torch.zeros((M, H * D), dtype=torch.float32, device=dev)
-    check(load().e2mi_attention_packed(stream_ptr(stream), ptr(q16), ptr(k16), ptr(vt16), M,
-                                       ptr(start), ptr(lens), start.shape[0], max_len, H, KV, D,
-                                       scale, ptr(cq), ptr(cs), ptr(c32), ptr(work),
+    check(load().e2mi_attention_packed(_stream(stream), _p(q16), _p(k16), _p(vt16), M,
+                                       _p(start), _p(lens), start.shape[0], max_len, H, KV, D,
+                                       scale, _p(cq), _p(cs), _p(c32), _p(work),
                                        0 if work is None else work.shape[0]), "attention_packed")
     return cq, cs, c32
 
@@ -639,9 +664,9 @@ def attention_packed_window(q16, k16, vt16, start, lens, max_len, H, KV, D, wind
     cs = torch.zeros((M, H * D // 128), dtype=torch.float32, device=dev) if cs is None else cs
     if want_f32 and c32 is None:
         c32 = torch.zeros((M, H * D), dtype=torch.float32, device=dev)
-    check(load().e2mi_attention_packed_window(stream_ptr(stream), ptr(q16), ptr(k16), ptr(vt16), M,
-                                              ptr(start), ptr(lens), ptr(pos), start.shape[0], max_len,
-                                              H, KV, D, scale, window, ptr(cq), ptr(cs), ptr(c32), ptr(work),
+    check(load().e2mi_attention_packed_window(_stream(stream), _p(q16), _p(k16), _p(vt16), M,
+                                              _p(start), _p(lens), _p(pos), start.shape[0], max_len,
+                                              H, KV, D, scale, window, _p(cq), _p(cs), _p(c32), _p(work),
                                               0 if work is None else work.shape[0]), "attention_packed_window")
     return cq, cs, c32
 
@@ -655,10 +680,10 @@ def add_norm_scale_quant(src, res, gamma_add, post_scale, gamma_next=None, eps=1
     x_out = torch.empty_like(src) if x_out is None else x_out
     has_next = gamma_next is not None
     xn = torch.empty_like(src) if (want_xn and has_next) else None
-    q = torch.empty((M, D), dtype=torch.int8, device=src.device) if quant else None
-    qs = torch.empty((M, D // 128), dtype=torch.float32, device=src.device) if quant else None
-    check(load().e2mi_add_norm_scale_quant(stream_ptr(stream), ptr(src), ptr(res), ptr(gamma_add), post_scale,
-                                           ptr(gamma_next), eps, M, D, ptr(x_out), ptr(xn), ptr(q), ptr(qs)),
+    q = src.new_empty((M, D), dtype=torch.int8) if quant else None
+    qs = src.new_empty((M, D // 128), dtype=torch.float32) if quant else None
+    check(load().e2mi_add_norm_scale_quant(_stream(stream), _p(src), _p(res), _p(gamma_add), post_scale,
+                                           _p(gamma_next), eps, M, D, _p(x_out), _p(xn), _p(q), _p(qs)),
           "add_norm_scale_quant")
     return x_out, xn, q, qs
 
@@ -668,7 +693,7 @@ def scale_norm(x, pre_scale, gamma, eps=1e-6, out=None, stream=None):
     import torch
     rows, D = x.shape
     out = torch.empty_like(x) if out is None else out
-    check(load().e2mi_scale_norm(stream_ptr(stream), ptr(x), rows, D, pre_scale, ptr(gamma), eps, ptr(out)),
+    check(load().e2mi_scale_norm(_stream(stream), _p(x), rows, D, pre_scale, _p(gamma), eps, _p(out)),
           "scale_norm")
     return out
 
@@ -690,9 +715,9 @@ def attention_i8_packed(q32, k32, v32, start, lens, max_len, H, KV, want_f32=Tru
     if want_f32 and c32 is None:
         c32 = torch.zeros((M, H * D), dtype=torch.float32, device=dev)
     wp = C.c_void_p((workspace.data_ptr() + 255) & ~255)
-    check(lib.e2mi_attention_i8_packed(stream_ptr(stream), ptr(q32), ptr(k32), ptr(v32), M, ptr(start),
-                                       ptr(lens), B, max_len, H, KV, D, wp, ptr(cq), ptr(cs), ptr(c32),
-                                       ptr(work), 0 if work is None else work.shape[0]),
+    check(lib.e2mi_attention_i8_packed(_stream(stream), _p(q32), _p(k32), _p(v32), M, _p(start),
+                                       _p(lens), B, max_len, H, KV, D, wp, _p(cq), _p(cs), _p(c32),
+                                       _p(work), 0 if work is None else work.shape[0]),
           "attention_i8_packed")
     return cq, cs, c32
 
@@ -704,9 +729,9 @@ def pool_l2_packed(x, start, lens, max_len, stream=None):
     lib = load()
     ws = torch.empty(lib.e2mi_pool_workspace_bytes(B, max_len, D) // 4 + 64, dtype=torch.float32,
                      device=x.device)
-    out = torch.empty((B, D), dtype=torch.float32, device=x.device)
-    check(lib.e2mi_pool_l2_packed(stream_ptr(stream), ptr(x), ptr(start), ptr(lens), B, max_len, D,
-                                  ptr(ws), ptr(out)), "pool_l2_packed")
+    out = x.new_empty((B, D), dtype=torch.float32)
+    check(lib.e2mi_pool_l2_packed(_stream(stream), _p(x), _p(start), _p(lens), B, max_len, D,
+                                  _p(ws), _p(out)), "pool_l2_packed")
     return out
 
 
@@ -714,7 +739,7 @@ def gather_ids(ids, rowmap, stream=None):
     import torch
     M = rowmap.shape[0]
     out = torch.empty(M, dtype=torch.int32, device=rowmap.device)
-    check(load().e2mi_gather_ids(stream_ptr(stream), ptr(ids), ptr(rowmap), M, ptr(out)), "gather_ids")
+    check(load().e2mi_gather_ids(_stream(stream), _p(ids), _p(rowmap), M, _p(out)), "gather_ids")
     return out
 
 
@@ -871,8 +896,8 @@ class Engine:
 
     def embed_batch_device(self, ids, valid, out, stream=None):
         B, S = ids.shape
-        check(load().e2mi_text_embed_batch_device(self.h, ptr(ids), ptr(valid), B, S, ptr(out),
-                                                  stream_ptr(stream)), "text_embed_batch_device")
+        check(load().e2mi_text_embed_batch_device(self.h, _p(ids), _p(valid), B, S, _p(out), _stream(stream)),
+              "text_embed_batch_device")
         return out
 
     def stats(self):
