@@ -198,6 +198,12 @@ bool gemm_half_tiles(int M, int N);
 // whether one round of the CUs covers that count
 int gemm_an_units(int rows);
 bool gemm_an_fits(int rows);
+// gemm_an.hip: the projection and its norm_add in one launch (e2mi_i8_gemm_add_norm_quant, scale:
+// _scale_quant), and whether two launches are faster at a row count
+int launch_gemm_add_norm(hipStream_t s, const int8_t *qa, const float *a_scales, const e2mi_q8w *w, int M,
+                         const float *res, const float *gamma_add, float post_scale, const float *gamma_next,
+                         float eps, float *x_out, float *xn_out, int8_t *q, float *qs, bool scale);
+bool gemm_an_split(int rows, int D);
 
 template <class T>
 static int dalloc(e2mi_engine *g, T **p, size_t count) {
@@ -340,14 +346,34 @@ static bool reference_geometry(const e2_config &c) {
 // the shortest sequence the int8 attention takes (text.c:873-875: its blocked kernels need 32 rows)
 constexpr int kI8MinKeys = 32;
 
-// attention workgroups of a packed chunk of n sequences in M rows: at most H (M / 128 + n)
-static int work_slots(const e2mi_engine *g, int n, int M) { return g->cfg.n_heads * (M / 128 + n); }
+// attention workgroups of a packed chunk of n sequences in M rows: at most H (ceil(M / 128) + n)
+static int work_slots(const e2mi_engine *g, int n, int M) { return g->cfg.n_heads * ((M + 127) / 128 + n); }
+
+// The rows a packed forward computes for `rows` planned ones (each sequence's rounded up to 8): up to 256
+// a multiple of 32, the small kernels' tile, so that a query's forward is not mostly filler rows (19
+// tokens, reference geometry: 1.50 ms with 256 rows); above, of 256, as the public planner rounds them.
+static int forward_rows(long rows) { return (int)(rows <= 256 ? (rows + 31) & ~31L : (rows + 255) & ~255L); }
 
 // split key ranges: a 128-query block whose keys span more than 8 tiles of 32 is split into
 // ceil(tiles / 8) parts (at most kMaxAttnParts), so the longest blocks no longer set the
 // attention's time alone; the parts depend only on the sequence's own length and the window
 // (block_parts, plan.cpp). The attention work lists are dealt to the XCDs (xcd_deal, plan.cpp).
 constexpr int kAttnPartTiles = 8, kMaxAttnParts = 4;
+
+// How a forward of about `rows` rows runs each projection (O, down, PLE) and its norm_add: separately,
+// fused (the norm_add in the projection's epilogue, one workgroup holding whole rows), or, at few rows,
+// ahead: the projection in many small tiles to memory and the norm_add in the workgroups of the GEMM
+// that reads it (NormIn). Fused needs one round of the CUs to cover the rows: past that each
+// workgroup's weight fetch costs more than the f32 round trip. Ahead while 32-row tiles of the GeGLU
+// GEMM, the widest reader, fit one round (a 19-token query, reference geometry: 2.10 ms fused, 1.21
+// ahead); between the two, up to gemm_an_split, two launches beat the fused one.
+enum NormForm { NORM_SEPARATE, NORM_FUSED, NORM_AHEAD };
+static NormForm norm_form(const e2mi_engine *g, int rows) {
+    const e2_config &c = g->cfg;
+    if (!g->fuse_an || (c.hidden != 768 && c.hidden != 512) || !gemm_an_fits(rows)) return NORM_SEPARATE;
+    if (gemm_small_route(rows, 2 * c.ffn, c.hidden, EPI_GEGLU, false) == GEMM_S32) return NORM_AHEAD;
+    return gemm_an_split(rows, c.hidden) ? NORM_SEPARATE : NORM_FUSED;
+}
 
 // every kernel of one forward over B sequences of S tokens (M rows: B * S padded, or the packed
 // row count), on stream s; returns the launch count or -1
@@ -357,9 +383,10 @@ static int enqueue(e2mi_engine *g, int B, int S, int Mp, bool pk, hipStream_t s,
     const DeviceRowsScope dev_rows(dev ? g->d_rows : nullptr, 1, est);
     const e2_config &c = g->cfg;
     const int M = pk ? Mp : B * S, Dm = c.hidden, H = c.n_heads, P = c.ple_dim;
-    // the projections with their norm_add in the epilogue when one round of the CUs covers the
-    // (expected) rows; past that each workgroup's weight fetch costs more than the f32 round trip
-    const bool an = gemm_an_fits(dev && est > 0 ? est : M);
+    const NormForm form = norm_form(g, dev && est > 0 ? est : M);
+    const bool an = form == NORM_FUSED;
+    // form ahead: x moves between two buffers, each norm_add reading one and writing the other
+    float *x = g->x, *x_other = g->xn;
     if (M <= 0 || M > g->R) {
         set_error("forward: %d rows for a %d-row workspace", M, g->R);
         return -1;
@@ -395,6 +422,18 @@ static int enqueue(e2mi_engine *g, int B, int S, int Mp, bool pk, hipStream_t s,
     } while (0)
     RUN("embed", launch_embed_checked(s, g->embed, c.vocab, g->ids, c.embed_scale, g->layers[0].ln_in, eps, M, Dm,
                              g->x, g->qa, g->as, nullptr));
+    // a GEMM whose activations come from the pending norm_add of tmp (form ahead)
+    NormIn pend;
+#define RUN_NORMED(name, call)                    \
+    do {                                          \
+        const NormInScope norm_scope(pend);       \
+        RUN(name, call);                          \
+        if (pend.y) std::swap(x, x_other);        \
+        pend.y = nullptr;                         \
+    } while (0)
+    auto ahead = [&](const float *gamma_a, float post_scale, const float *gamma_n) {
+        pend = NormIn{g->tmp, x, gamma_a, gamma_n, x_other, post_scale, eps};
+    };
     if (P > 0) {  // the per-layer inputs from the scaled embeddings (text.c:929-932)
         const int NP = c.n_layers * P;
         RUN("ple_quant", e2mi_quantize(s, g->qg, g->gs, g->x, M, Dm, Dm, 128));
@@ -407,11 +446,11 @@ static int enqueue(e2mi_engine *g, int B, int S, int Mp, bool pk, hipStream_t s,
         const int D = L.geo.D, KV = L.geo.KV, qd = H * D;
         const float *cs = L.geo.full ? g->cos_full : g->cos_tab, *sn = L.geo.full ? g->sin_full : g->sin_tab;
         if (L.qkv_fused)
-            RUN("qkv_norm_rope_gemm", e2mi_i8_gemm_qkv(s, g->qa, g->as, &L.qkv, M, pk ? M : S, pk ? g->pos : nullptr, H, KV, L.q_norm,
+            RUN_NORMED("qkv_norm_rope_gemm", e2mi_i8_gemm_qkv(s, g->qa, g->as, &L.qkv, M, pk ? M : S, pk ? g->pos : nullptr, H, KV, L.q_norm,
                                  L.k_norm, eps, cs, sn, g->q16, g->k16, g->vt16, g->attn_i8 ? g->q32 : nullptr,
                                  g->attn_i8 ? g->k32 : nullptr, g->attn_i8 ? g->v32 : nullptr));
         else
-            RUN("qkv", e2mi_i8_gemm(s, g->qkv, qd + 2 * KV * D, g->qa, g->as, &L.qkv, M, 0, L.qkv.N));
+            RUN_NORMED("qkv", e2mi_i8_gemm(s, g->qkv, qd + 2 * KV * D, g->qa, g->as, &L.qkv, M, 0, L.qkv.N));
         if (pk) {
             if (!L.qkv_fused)
                 RUN("qkv_norm_rope", e2mi_qkv_norm_rope_packed(s, g->qkv, M, g->pos, H, KV, D, L.q_norm, L.k_norm, eps, cs, sn,
@@ -441,34 +480,57 @@ static int enqueue(e2mi_engine *g, int B, int S, int Mp, bool pk, hipStream_t s,
             RUN("attention", e2mi_attention(s, g->q16, g->k16, g->vt16, g->valid, B, S, H, KV, D, c.attn_scale,
                                g->cq, g->cs, nullptr));
         }
-        if (L.o_an && an) {
-            RUN("o_proj+add_norm", e2mi_i8_gemm_add_norm_quant(s, g->cq, g->cs, &L.o, M, g->x, L.ln_attn, L.ln_pre, eps,
-                                                               g->x, nullptr, g->qa, g->as, nullptr));
+        if (form == NORM_AHEAD) {
+            RUN("o_proj+add_norm", e2mi_i8_gemm(s, g->tmp, Dm, g->cq, g->cs, &L.o, M, 0, Dm));
+            ahead(L.ln_attn, 1.0f, L.ln_pre);
+        } else if (L.o_an && an) {
+            RUN("o_proj+add_norm", launch_gemm_add_norm(s, g->cq, g->cs, &L.o, M, g->x, L.ln_attn, 1.0f, L.ln_pre, eps,
+                                                        g->x, nullptr, g->qa, g->as, false));
         } else {
             RUN("o_proj", e2mi_i8_gemm(s, g->tmp, Dm, g->cq, g->cs, &L.o, M, 0, Dm));
             RUN("add_norm", e2mi_add_norm_quant(s, g->tmp, g->x, L.ln_attn, L.ln_pre, eps, M, Dm, g->x, nullptr,
                                                 g->qa, g->as));
         }
-        RUN("gate_up_geglu", e2mi_i8_gemm_geglu(s, g->qg, g->gs, nullptr, g->qa, g->as, &L.gu, M));
+        RUN_NORMED("gate_up_geglu", e2mi_i8_gemm_geglu(s, g->qg, g->gs, nullptr, g->qa, g->as, &L.gu, M));
         const bool last = l + 1 == nl;
         const float *gnext = last ? g->final_norm : g->layers[l + 1].ln_in;
+        if (form == NORM_AHEAD) {
+            // the last norm_add has no GEMM after it that takes it: fused, into g->x and g->xn
+            if (P > 0 || !last) RUN("down+add_norm", e2mi_i8_gemm(s, g->tmp, Dm, g->qg, g->gs, &L.down, M, 0, Dm));
+            if (P > 0) {
+                ahead(L.ln_ffn, 1.0f, nullptr);
+                RUN_NORMED("ple_gate", e2mi_i8_gemm_gelu_mul(s, g->qg, g->gs, nullptr, g->qa, g->as, &L.ple_gate, M,
+                                                             g->ple32 + (size_t)l * P, c.n_layers * P));
+                if (!last) RUN("ple_proj+add_norm", e2mi_i8_gemm(s, g->tmp, Dm, g->qg, g->gs, &L.ple_proj, M, 0, Dm));
+            }
+            if (!last) {
+                ahead(P > 0 ? L.ple_norm : L.ln_ffn, P > 0 ? L.layer_scalar : 1.0f, gnext);
+            } else if (P > 0) {
+                RUN("ple_proj+add_norm", launch_gemm_add_norm(s, g->qg, g->gs, &L.ple_proj, M, x, L.ple_norm,
+                                                              L.layer_scalar, gnext, eps, g->x, g->xn, g->qa, g->as, true));
+            } else {
+                const bool quant = c.out_dim > 0;
+                RUN("down+add_norm", launch_gemm_add_norm(s, g->qg, g->gs, &L.down, M, x, L.ln_ffn, 1.0f, gnext, eps, g->x,
+                                                          g->xn, quant ? g->qa : nullptr, quant ? g->as : nullptr, false));
+            }
+            continue;
+        }
         if (L.down_an && an && P > 0) {
             // post_ffn norm_add in the down projection, x itself quantized for the PLE gate; the PLE
             // block, its norm_add and the layer scale in the PLE projection
-            RUN("down+add_norm", e2mi_i8_gemm_add_norm_scale_quant(s, g->qg, g->gs, &L.down, M, g->x, L.ln_ffn, 1.0f,
-                                                                   nullptr, eps, g->x, nullptr, g->qa, g->as, nullptr));
+            RUN("down+add_norm", launch_gemm_add_norm(s, g->qg, g->gs, &L.down, M, g->x, L.ln_ffn, 1.0f, nullptr, eps,
+                                                      g->x, nullptr, g->qa, g->as, true));
             RUN("ple_gate", e2mi_i8_gemm_gelu_mul(s, g->qg, g->gs, nullptr, g->qa, g->as, &L.ple_gate, M,
                                                   g->ple32 + (size_t)l * P, c.n_layers * P));
-            RUN("ple_proj+add_norm", e2mi_i8_gemm_add_norm_scale_quant(s, g->qg, g->gs, &L.ple_proj, M, g->x, L.ple_norm,
-                                                                       L.layer_scalar, gnext, eps, g->x,
-                                                                       last ? g->xn : nullptr, g->qa, g->as, nullptr));
+            RUN("ple_proj+add_norm", launch_gemm_add_norm(s, g->qg, g->gs, &L.ple_proj, M, g->x, L.ple_norm,
+                                                          L.layer_scalar, gnext, eps, g->x, last ? g->xn : nullptr,
+                                                          g->qa, g->as, true));
             continue;
         }
         if (L.down_an && an) {
-            RUN("down+add_norm", e2mi_i8_gemm_add_norm_quant(s, g->qg, g->gs, &L.down, M, g->x, L.ln_ffn, gnext, eps, g->x,
-                                                             last ? g->xn : nullptr,
-                                                             !last || c.out_dim > 0 ? g->qa : nullptr,
-                                                             !last || c.out_dim > 0 ? g->as : nullptr, nullptr));
+            RUN("down+add_norm", launch_gemm_add_norm(s, g->qg, g->gs, &L.down, M, g->x, L.ln_ffn, 1.0f, gnext, eps, g->x,
+                                                      last ? g->xn : nullptr, !last || c.out_dim > 0 ? g->qa : nullptr,
+                                                      !last || c.out_dim > 0 ? g->as : nullptr, false));
             continue;
         }
         RUN("down", e2mi_i8_gemm(s, g->tmp, Dm, g->qg, g->gs, &L.down, M, 0, Dm));
@@ -497,6 +559,7 @@ static int enqueue(e2mi_engine *g, int B, int S, int Mp, bool pk, hipStream_t s,
         RUN("pool", e2mi_pool_l2_packed(s, rows, g->seq_start, g->seq_len, B, S, g->dout, g->pool_ws, g->out));
     else
         RUN("pool", e2mi_pool_l2(s, rows, g->valid, B, S, g->dout, g->pool_ws, g->out));
+#undef RUN_NORMED
 #undef RUN
     return k + 1;  // the pool is two launches
 }
@@ -567,6 +630,7 @@ struct PlanLayout {
 static bool has_full_list(const e2mi_engine *g) { return g->split_factor > 1 && g->cfg.full_period > 0; }
 static PlanLayout plan_layout(const e2mi_engine *g, int n, int Mp) {
     auto up = [](size_t x) { return (x + 63) & ~(size_t)63; };
+    Mp = (Mp + 255) & ~255;  // the planners' row count
     const size_t slots = (size_t)work_slots(g, n, Mp);
     PlanLayout L;
     size_t o = 0;
@@ -600,7 +664,8 @@ static int plan_pack(e2mi_engine *g, const uint8_t *valid, int n, int S) {
     long rows = 0;
     for (int b = 0; b < n; b++) rows += seq_rows(valid ? valid + (size_t)b * S : nullptr, S);
     plan_bind(g, plan_layout(g, n, (int)((rows + 255) & ~255L)));
-    const int Mp = pack_rows(valid, n, S, g->h_rowmap, g->h_pos, g->h_start, g->h_len);
+    pack_rows(valid, n, S, g->h_rowmap, g->h_pos, g->h_start, g->h_len);
+    const int Mp = forward_rows(rows);
     const int H = g->cfg.n_heads, slots = work_slots(g, n, Mp);
     // split long blocks' keys only where the unsplit blocks leave most of the device idle (few
     // sequences; mode 2): a full batch's blocks already fill it, and the parts' partial states then
@@ -631,10 +696,11 @@ static int plan_pack(e2mi_engine *g, const uint8_t *valid, int n, int S) {
 
 // The kernels of a device-planned forward of about `est` rows: for every distinct GEMM of the forward
 // whose kernel follows the row count, which one takes it (gemm_small_route, gemm_half_tiles), and
-// whether the projections run with their norm_add and in how many row units per workgroup (1-5)
+// how the projections run their norm_add (fused: in how many row units per workgroup, 1-5)
 static long tile_signature(const e2mi_engine *g, int est) {
     const e2_config &c = g->cfg;
-    const bool an = gemm_an_fits(est);
+    const NormForm form = norm_form(g, est);
+    const bool an = form == NORM_FUSED;
     std::vector<std::tuple<int, int, int>> gemms;  // N, K, epilogue
     auto add = [&](const e2mi_q8w &w, int epi) { gemms.emplace_back(w.N, w.K, epi); };
     for (const LayerDev &L : g->layers) {
@@ -651,7 +717,7 @@ static long tile_signature(const e2mi_engine *g, int est) {
     if (c.out_dim > 0) add(g->embed_proj, EPI_F32);
     std::sort(gemms.begin(), gemms.end());
     gemms.erase(std::unique(gemms.begin(), gemms.end()), gemms.end());
-    long sig = !g->layers.empty() && g->layers[0].o_an && an ? gemm_an_units(est) : 0;
+    long sig = an ? gemm_an_units(est) : form == NORM_AHEAD ? 6 : 0;
     for (const auto &[N, K, epi] : gemms) {  // at most 14 of them, 3 bits each
         const int small = gemm_small_route(est, N, K, epi, false);
         sig = sig << 3 | (small ? small : gemm_half_tiles(est, N) ? 4 : 0);
@@ -660,13 +726,13 @@ static long tile_signature(const e2mi_engine *g, int est) {
 }
 
 // The device entry plans on the device (plan_dev.hip) when the whole batch is one chunk whatever its
-// mask (every token valid: n ceil8(S) rows, rounded up to 256, within the workspace) and its lists fit
+// mask (every token valid: n ceil8(S) rows, rounded up (forward_rows), within the workspace) and its lists fit
 // the planner's workgroup, with the unsplit f16 lists (no int8 attention, no split mode) and no
 // workspace dump (which writes the host plan). Returns the rows the forward is sized for, or 0.
 static int device_plan_rows(const e2mi_engine *g, int n, int S) {
     if (!g->device_plan || !g->packed || g->attn_i8 || g->split_mode != 0 || !g->dump_dir.empty() || n > g->bmax)
         return 0;
-    const long cap = ((long)n * ((S + 7) & ~7) + 255) & ~255L;
+    const long cap = forward_rows((long)n * ((S + 7) & ~7));
     if (cap > g->R || !plan_device_fits(n, S, g->cfg.n_heads, work_slots(g, n, (int)cap))) return 0;
     return (int)cap;
 }
@@ -1214,7 +1280,7 @@ extern "C" int e2mi_text_embed_batch_device(e2mi_engine *g, const int32_t *ids, 
         // the GEMM tiles follow the row count of this shape's latest finished call (the capacity
         // before one has finished): the same embeddings either way, one recorded forward per choice
         const auto seen = g->rows_seen.find(std::make_pair(batch, seq_len));
-        const int est = seen != g->rows_seen.end() ? seen->second : cap;
+        const int est = seen != g->rows_seen.end() ? std::min(seen->second, cap) : cap;
         if (launch_plan_packed(s, pa) ||
             run_shape(g, batch, seq_len, cap, true, s, true, est, tile_signature(g, est)) ||
             check_hip(hipMemcpyAsync(out, g->out, (size_t)batch * g->dout * 4, hipMemcpyDeviceToDevice, s),

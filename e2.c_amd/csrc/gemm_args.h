@@ -37,6 +37,25 @@ struct GemmArgs {
     const int *rows;
 };
 
+// The norm_add that makes a GEMM's activations, run in the GEMM's own workgroups (gemm_s.hip; the
+// engine at few rows): x' = (rmsnorm(y) * gamma_a + x) * post_scale -> x_out (another buffer than x),
+// then rmsnorm(x') * gamma_n (without gamma_n: x' itself) quantized per 128. Rows of K columns.
+// Set for the GEMMs that the thread launches while a NormInScope lives; they take no quantized
+// activations then.
+struct NormIn {
+    const float *y = nullptr, *x = nullptr, *gamma_a = nullptr, *gamma_n = nullptr;
+    float *x_out = nullptr;
+    float post_scale = 1.f, eps = 0.f;
+};
+const NormIn &norm_in();
+class NormInScope {
+  public:
+    explicit NormInScope(const NormIn &n);
+    ~NormInScope();
+    NormInScope(const NormInScope &) = delete;
+    NormInScope &operator=(const NormInScope &) = delete;
+};
+
 // gemm_s.hip: the kernels for few rows, and which one (0: none) takes an M x N x K GEMM with the
 // epilogue `epi` (tok: per-token activation scales); launch_gemm_small runs it at the expected row
 // count and returns 1, or returns 0 for the caller's kernels and -1 on error

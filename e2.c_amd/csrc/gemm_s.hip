@@ -55,8 +55,13 @@ struct Small {
 // rest as their slots are read. Weight blocks are private to a wave: no barrier in the K loop, only
 // its own load counts. The folded tile goes through LDS once, so that a row is held by 32 or 64
 // lanes in the epilogue.
-template <int EPI, int NW, int RU, int CU, int FOLD>
-__global__ __launch_bounds__(NW * 64, 1) void k_gemm_s(const int *rows, GemmArgs p, int tiles_m, int tiles) {
+//
+// NC > 0: the activations are made here from the norm_add before the GEMM (NormIn, rows of 256 NC), each
+// column tile's workgroup norming the tile's rows again: 2 x 4 K bytes a row more to load, under the
+// weight loads, against a row kernel's launch (3.3-3.9 us at 32-256 rows). The row kernel's steps
+// (rowops.hip, ROW_ADDNORM / ROW_ADDSCALE) with k_gemm_an's byte packing: the same bits.
+template <int EPI, int NW, int RU, int CU, int FOLD, int NC = 0>
+__global__ __launch_bounds__(NW * 64, 1) void k_gemm_s(const int *rows, GemmArgs p, int tiles_m, int tiles, NormIn ni) {
     using S = Small<NW, RU, CU>;
     constexpr int R = S::R, CPW = S::CPW, BN = S::BN, BM = S::BM, FP = S::FP, NT = NW * 64;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -78,13 +83,31 @@ __global__ __launch_bounds__(NW * 64, 1) void k_gemm_s(const int *rows, GemmArgs
     // (l % 8) ^ swzk(row), which depends on j's parity. Rows past M (N) read as zero.
     const uint32_t ch[2] = {(uint32_t)((lane & 7) ^ (lane >> 4)) << 4, (uint32_t)((lane & 7) ^ (4 + (lane >> 4))) << 4};
     const uint32_t lr = (uint32_t)lane >> 3;
-    for (int i = wave; i < nb * RU * 2; i += NW) {
-        const int b = i / (RU * 2), j = i % (RU * 2);
-        dma16(rA, lds0 + (uint32_t)i * 1024u, (uint32_t)(m0 + 8 * j + lr) * (uint32_t)p.lda + ((j & 1) ? ch[1] : ch[0]),
-              (uint32_t)b * kQBlock);
+    constexpr int NR = BM / NW, ND = NC > 0 ? NC : 1;  // rows a wave norms, float4 chunks per lane of a row
+    float4 ny[NR][ND], nx[NR][ND], ga[ND], gn[ND];
+    if constexpr (NC > 0) {
+#pragma unroll
+        for (int j = 0; j < NR; j++)
+#pragma unroll
+            for (int i = 0; i < NC; i++) {
+                const size_t o = (size_t)min(m0 + wave * NR + j, p.M - 1) * (256 * NC) + 4 * (lane + 64 * i);
+                ny[j][i] = ld4(ni.y + o);
+                nx[j][i] = ld4(ni.x + o);
+            }
+#pragma unroll
+        for (int i = 0; i < NC; i++) {
+            ga[i] = ld4(ni.gamma_a + 4 * (lane + 64 * i));
+            gn[i] = ni.gamma_n ? ld4(ni.gamma_n + 4 * (lane + 64 * i)) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    } else {
+        for (int i = wave; i < nb * RU * 2; i += NW) {
+            const int b = i / (RU * 2), j = i % (RU * 2);
+            dma16(rA, lds0 + (uint32_t)i * 1024u, (uint32_t)(m0 + 8 * j + lr) * (uint32_t)p.lda + ((j & 1) ? ch[1] : ch[0]),
+                  (uint32_t)b * kQBlock);
+        }
+        for (int b = wave; b < nsb; b += NW)
+            dma4(rS, lds0 + oS + (uint32_t)b * 256u, (uint32_t)(m0 + lane) * (uint32_t)nsb * 4u, (uint32_t)b * 4u);
     }
-    for (int b = wave; b < nsb; b += NW)
-        dma4(rS, lds0 + oS + (uint32_t)b * 256u, (uint32_t)(m0 + lane) * (uint32_t)nsb * 4u, (uint32_t)b * 4u);
     if (wave < BN / 64) dma4(rV, lds0 + oV + wave * 256u, (uint32_t)(n0 + wave * 64 + lane) * 4u, 0);
     const uint32_t ring = oW + wave * R * CU * 2048;
     auto issue_w = [&](int b) {
@@ -143,8 +166,45 @@ __global__ __launch_bounds__(NW * 64, 1) void k_gemm_s(const int *rows, GemmArgs
             }
         }
     };
-    wait_items(ahead);
-    asm volatile("s_barrier" ::: "memory");  // every wave's part of A and the scales has landed
+    if constexpr (NC > 0) {
+#pragma unroll
+        for (int j = 0; j < NR; j++) {
+            const int r = wave * NR + j, m = m0 + r;
+            float ss = 0.f;
+#pragma unroll
+            for (int i = 0; i < NC; i++) ss += sumsq4(ny[j][i]);
+            float inv = rms_inv(group_sum<64>(ss), 256 * NC, ni.eps);
+            ss = 0.f;
+#pragma unroll
+            for (int i = 0; i < NC; i++) {
+                const float4 y = scale4(ny[j][i], inv, ga[i]), x = nx[j][i];
+                const float4 v = make_float4(__fmul_rn(y.x + x.x, ni.post_scale), __fmul_rn(y.y + x.y, ni.post_scale),
+                                             __fmul_rn(y.z + x.z, ni.post_scale), __fmul_rn(y.w + x.w, ni.post_scale));
+                ny[j][i] = v;
+                if (n0 == 0 && m < p.M) st4(ni.x_out + (size_t)m * (256 * NC) + 4 * (lane + 64 * i), v);
+                ss += sumsq4(v);
+            }
+            if (ni.gamma_n) {
+                inv = rms_inv(group_sum<64>(ss), 256 * NC, ni.eps);
+#pragma unroll
+                for (int i = 0; i < NC; i++) ny[j][i] = scale4(ny[j][i], inv, gn[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < NC; i++) {  // chunk l + 64 i: block 2 i + l / 32, its bytes 4 (l % 32) .. + 3
+                const float4 v = ny[j][i];
+                const QScale q = qscale(group_max<32>(amax4(v)));
+                const int blk = 2 * i + hh;
+                *(uint32_t *)(smem + blk * (RU * 2048) + (r >> 4) * 2048 + swz(r & 15, c >> 2) + (c & 3) * 4) =
+                    pack4_magic(v.x, v.y, v.z, v.w, q.inv);
+                if (c == 0) *(float *)(smem + oS + blk * 256 + r * 4) = q.sc;
+            }
+        }
+        wait_items(ahead);
+        lds_barrier();
+    } else {
+        wait_items(ahead);
+        asm volatile("s_barrier" ::: "memory");  // every wave's part of A and the scales has landed
+    }
 
     float f[RU][CU][4];
 #pragma unroll
@@ -500,17 +560,18 @@ int set_lds(K kern) {
 
 int grid_of(int tiles) { return (tiles + 7) / 8 * 8; }
 
-template <int EPI, int NW, int RU, int CU, int FOLD>
+template <int EPI, int NW, int RU, int CU, int FOLD, int NC = 0>
 int launch_s1(hipStream_t s, const GemmArgs &p) {
     using T = Small<NW, RU, CU>;
-    auto kern = k_gemm_s<EPI, NW, RU, CU, FOLD>;
+    auto kern = k_gemm_s<EPI, NW, RU, CU, FOLD, NC>;
     static bool attr = false;
     if (!attr) {
         if (set_lds(kern)) return -1;
         attr = true;
     }
     const int tm = (p.M + T::BM - 1) / T::BM, tiles = tm * ((p.N + T::BN - 1) / T::BN);
-    hipLaunchKernelGGL(kern, dim3(grid_of(tiles)), dim3(NW * 64), T::lds(p.K / kQBlock), s, p.rows, p, tm, tiles);
+    hipLaunchKernelGGL(kern, dim3(grid_of(tiles)), dim3(NW * 64), T::lds(p.K / kQBlock), s, p.rows, p, tm, tiles,
+                       norm_in());
     return check_hip(hipGetLastError(), "gemm launch");
 }
 template <int EPI, int NW, int RU, int CU>
@@ -534,7 +595,35 @@ int launch_sk(hipStream_t s, const GemmArgs &p) {
 
 constexpr int kLds = 160 * 1024;
 
+// with the norm_add before it (NormInScope): 32-row tiles, rows of 512 or 768
+template <int EPI, int NW>
+int launch_norm1(hipStream_t s, const GemmArgs &p) {
+    const bool fast = gemm_fold_fast();
+    if (p.K == 768)
+        return fast ? launch_s1<EPI, NW, 2, 1, FOLD_FAST, 3>(s, p) : launch_s1<EPI, NW, 2, 1, FOLD_EXACT, 3>(s, p);
+    return fast ? launch_s1<EPI, NW, 2, 1, FOLD_FAST, 2>(s, p) : launch_s1<EPI, NW, 2, 1, FOLD_EXACT, 2>(s, p);
+}
+int launch_norm(hipStream_t s, const GemmArgs &p, int epi) {
+    if (p.K != 512 && p.K != 768) {
+        set_error("gemm: a norm_add before the GEMM needs rows of 512 or 768 (K=%d)", p.K);
+        return -1;
+    }
+    switch (epi) {
+    case EPI_F32: return launch_norm1<EPI_F32, 8>(s, p);
+    case EPI_GELUMUL: return launch_norm1<EPI_GELUMUL, 8>(s, p);
+    case EPI_GEGLU: return launch_norm1<EPI_GEGLU, 16>(s, p);
+    case EPI_QKV: return launch_norm1<EPI_QKV, 16>(s, p);
+    default: set_error("gemm: no norm_add before this GEMM"); return -1;
+    }
+}
+
+thread_local NormIn t_norm;
+
 }  // namespace
+
+const NormIn &norm_in() { return t_norm; }
+NormInScope::NormInScope(const NormIn &n) { t_norm = n; }
+NormInScope::~NormInScope() { t_norm = NormIn{}; }
 
 // Which kernel takes an M x N x K GEMM. The outputs are the same bits whichever it is; the lines lie
 // where the measured times cross (us per launch, weights not in L2, gemm.hip's kernel last).
@@ -579,6 +668,7 @@ int gemm_small_route(int M, int N, int K, int epi, bool tok) {
 // Runs the GEMM here when gemm_small_route takes it at the expected row count: 1 when it was launched,
 // 0 when the caller's kernels take it, -1 on error.
 int launch_gemm_small(hipStream_t s, const GemmArgs &p, int epi, int est, bool tok) {
+    if (norm_in().y) return launch_norm(s, p, epi) ? -1 : 1;
     const int route = gemm_small_route(est, p.N, p.K, epi, tok);
     if (!route) return 0;
     int rc;
