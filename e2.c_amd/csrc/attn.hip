@@ -16,6 +16,8 @@
 // B-operand slots must carry, once the A operand (V^T) is read in the same key order. K tile rows
 // are stored with bits 2 and 3 of the key index exchanged, which makes those keys consecutive
 // (16 j + 8 half + 0..7 for MFMA j), so a lane's V^T operand is 8 consecutive keys of one row.
+#include <algorithm>
+
 #include "common.h"
 
 namespace e2mi {
@@ -756,6 +758,276 @@ __global__ __launch_bounds__(512, 1) void k_attn_packed_d512(AttnArgs a) {
     }
 }
 
+// ---- the same attention in blocks of 32 queries, one 4-wave workgroup each: for grids that leave CUs
+// idle in 128-query blocks, where a block's time is its serial walk over the key tiles. The waves
+// take NT = 4 (head_dim 512: 2) key tiles at once: wave w computes the logits of tile w (head_dim
+// 512: of tile w % 2 over dims 256 (w / 2) .. + 255, the two partial sums added as in
+// k_attn_packed_d512), then the context's dims D/4 w .. + D/4 - 1 over all NT tiles. The tiles' row
+// maxima, probabilities and row sums go through LDS (two barriers a group, three at 512), and every
+// wave walks the running max over the NT tiles in order, so each query sees the arithmetic of
+// k_attn_packed (k_attn_packed_d512) bit for bit: the same MFMA chains, rescales and sums; tiles with
+// no key for a query change nothing there, and are skipped here.
+// K and V^T fragments are private to a wave (16 KB each), loaded straight to LDS with no barrier: the
+// next group's K while this group's softmax and context run, its V^T under the next logits.
+template <int D>
+struct GroupTile {
+    static constexpr int ND = D / 256, NT = 4 / ND, DW = D / 4;  // dim halves, tiles a group, dims a wave
+    static constexpr int kW = 32 * 1024;                         // a wave's K (16 KB) and V^T (16 KB)
+    static constexpr int kP = 4 * kW, kX = kP + NT * 2048, kM = kX + (ND > 1 ? 16384 : 0), kS = kM + NT * 128;
+    static constexpr size_t kLds = kS + NT * 256 + 4 * 128;
+};
+
+template <int D, bool WIN>
+__global__ __launch_bounds__(256, 1) void k_attn_group(AttnArgs a, int n_work) {
+    using T = GroupTile<D>;
+    constexpr int ND = T::ND, NT = T::NT, DW = T::DW, NO = DW / 32;
+    extern __shared__ __align__(16) unsigned char pk_smem[];
+    // work entry i's four blocks on the XCD of workgroup i of a 128-query grid (i % 8)
+    int q0 = blockIdx.x * 32, h = blockIdx.y, b = blockIdx.z;
+    if (a.work) {
+        const int i = (blockIdx.x >> 5) * 8 + (blockIdx.x & 7);
+        const int item = i < n_work ? a.work[i] : -1;
+        if (item < 0) return;
+        b = item & 0xffff;
+        h = (item >> 16) & 0xf;
+        q0 = (item >> 24) * 128 + ((blockIdx.x >> 3) & 3) * 32;
+    }
+    const int Sk = a.seq_len[b];
+    if (q0 >= Sk) return;
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, ql = lane & 31;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tw = w % NT, dh = w / NT;  // this wave's tile of a group and dim half
+    const int S = a.S, HD = a.H * D, kvh = h / (a.H / a.KV);
+    const size_t row0 = (size_t)a.seq_start[b];
+    const int qi = q0 + ql;
+    const int qc = min(qi, Sk - 1);
+    h8 qf[16];
+    {
+        const uint16_t *qp = a.q + (row0 + qc) * HD + h * D + dh * 256 + 8 * half;
+#pragma unroll
+        for (int s = 0; s < 16; s++) qf[s] = *(const h8 *)(qp + 16 * s);
+    }
+    const int W = WIN ? a.window : 0;
+    int kt0 = 0, kt1 = (Sk + kKT - 1) / kKT;
+    int pq0 = 0, pq1 = 0, pqi = qc;
+    if constexpr (WIN) {
+        const int q1 = min(q0 + 31, Sk - 1);
+        kt0 = max(q0 - W, 0) / kKT;
+        kt1 = min((min(q1 + W, Sk - 1)) / kKT + 1, kt1);
+        pq0 = a.pos ? a.pos[row0 + q0] : q0;
+        pq1 = a.pos ? a.pos[row0 + q1] : q1;
+        pqi = a.pos ? a.pos[row0 + qc] : qc;
+    }
+    const uint32_t rowB = (uint32_t)a.KV * D * 2;
+    const v4u rK = rsrc_words(a.k + row0 * a.KV * D + kvh * D, (uint32_t)Sk * rowB);
+    const uint16_t *vslab = a.vt + (size_t)kvh * D * S + row0;
+    const v4u rV = rsrc_words(vslab, (uint32_t)((size_t)D * S * 2));
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const lds_void *)pk_smem);
+    const uint32_t kbase = w * T::kW, vbase = kbase + 16384;
+    // K: load i fills rows 2 i, 2 i + 1 of the wave's tile (row r: key swap23(r), chunk x at x ^ (r & 7)),
+    // offsets past the sequence read as zero. V^T: rows of NT * 64 bytes (NT * 32 keys), chunk c of row
+    // d at c ^ (d & 15) (NT = 4) or c ^ ((d >> 1) & 7) (NT = 2), chunks past the sequence as zero.
+    auto issue_k = [&](int kt) {
+        const int k0 = kt * kKT + tw * kKT;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int r = 2 * i + half;
+            dma16(rK, lds0 + kbase + i * 1024u,
+                  (uint32_t)(swap23(2 * i) + half + k0) * rowB + dh * 512u + (uint32_t)((ql ^ (r & 7)) << 4), 0u);
+        }
+    };
+    constexpr int LPR = NT * 4;  // lanes (16-byte chunks) a V^T row
+    const int vr0 = lane / LPR;
+    auto issue_v = [&](int kt) {
+        const int k0 = kt * kKT;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int r = (64 / LPR) * i + vr0;
+            const int cx = (lane % LPR) ^ (NT == 4 ? (r & 15) : ((r >> 1) & 7));
+            dma16(rV, lds0 + vbase + i * 1024u,
+                  k0 + 8 * cx < Sk ? (uint32_t)(((w * DW + r) * S + k0 + 8 * cx) * 2) : 0x80000000u, 0u);
+        }
+    };
+    uint32_t krd[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) krd[u] = kbase + (uint32_t)(ql * 512 + (((2 * u + half) ^ (ql & 7)) << 4));
+    // V^T fragment of o tile tt, group tile t, key half j
+    auto vfrag = [&](int tt, int t, int j) {
+        const int d = 32 * tt + ql, c = 4 * t + 2 * j + half;
+        const int sw = NT == 4 ? (d & 15) : ((d >> 1) & 7);
+        return *(const h8 *)(pk_smem + vbase + d * (NT * 64) + ((c ^ sw) << 4));
+    };
+    float *mx = (float *)(pk_smem + T::kM), *ps = (float *)(pk_smem + T::kS);
+
+    f16v o[NO];
+#pragma unroll
+    for (int t = 0; t < NO; t++) o[t] = (f16v){};
+    float mrun = -INFINITY, lrun = 0.f;
+    const float c2 = a.scale * 1.44269504088896341f;  // logits in base-2 units
+    issue_k(kt0);
+    issue_v(kt0);
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // the Q loads, after the first tiles' (see k_attn_packed)
+    for (int kg = kt0; kg < kt1; kg += NT) {
+        const int kt = kg + tw, k0 = kt * kKT;
+        const bool next = kg + NT < kt1;
+        asm volatile("s_waitcnt vmcnt(16)" ::: "memory");  // K of this group (V^T was issued after it)
+        f16v st = (f16v){};
+        h8 kr[PFK];
+#pragma unroll
+        for (int s = 0; s < PFK; s++) kr[s] = *(const h8 *)(pk_smem + krd[s & 3] + (s >> 2) * 128);
+#pragma unroll
+        for (int s = 0; s < 16; s++) {
+            st = __builtin_amdgcn_mfma_f32_32x32x16_f16(kr[s % PFK], qf[s], st, 0, 0, 0);
+            if (s + PFK < 16) kr[s % PFK] = *(const h8 *)(pk_smem + krd[(s + PFK) & 3] + ((s + PFK) >> 2) * 128);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (next) issue_k(kg + NT);  // (this wave's K reads have completed: the MFMAs took them)
+        float tv[16];
+        if constexpr (ND > 1) {
+            float *xw = (float *)(pk_smem + T::kX) + (w * 64 + lane) * 4;
+            const float *xp = (const float *)(pk_smem + T::kX) + ((w ^ NT) * 64 + lane) * 4;
+#pragma unroll
+            for (int r = 0; r < 16; r += 4) *(float4 *)(xw + r * 256) = make_float4(st[r], st[r + 1], st[r + 2], st[r + 3]);
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+            for (int r = 0; r < 16; r += 4) {
+                const float4 x = *(const float4 *)(xp + r * 256);
+                tv[r] = st[r] + x.x;
+                tv[r + 1] = st[r + 1] + x.y;
+                tv[r + 2] = st[r + 2] + x.z;
+                tv[r + 3] = st[r + 3] + x.w;
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; r++) tv[r] = st[r];
+        }
+        bool edge = k0 + kKT > Sk || kt >= kt1;
+        if constexpr (WIN) {
+            if (!edge) {
+                const int pka = a.pos ? a.pos[row0 + k0] : k0, pkb = a.pos ? a.pos[row0 + k0 + kKT - 1] : k0 + kKT - 1;
+                edge = pkb - pq0 > W || pq1 - pka > W;
+            }
+        }
+        if (edge) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int key = 16 * (r >> 3) + 8 * half + 4 * ((r >> 2) & 1) + (r & 3);
+                bool keep = k0 + key < Sk && kt < kt1;
+                if constexpr (WIN) {
+                    if (keep) {
+                        const int pk = a.pos ? a.pos[row0 + k0 + key] : k0 + key;
+                        keep = pk - pqi <= W && pqi - pk <= W;
+                    }
+                }
+                if (!keep) tv[r] = -INFINITY;
+            }
+        }
+        // softmax_tile over the group's tiles in order
+        float mloc = tv[0];
+#pragma unroll
+        for (int r = 1; r < 16; r++) mloc = fmaxf(mloc, tv[r]);
+        mloc = fmaxf(mloc, xor_lane<32>(mloc));
+        if (half == 0 && dh == 0) mx[tw * 32 + ql] = mloc;
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        float alpha[NT], mine = 0.f;
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            const float mc = mx[t * 32 + ql] * c2;
+            alpha[t] = 1.f;
+            if (mc > mrun + kTau) {
+                alpha[t] = __builtin_amdgcn_exp2f(mrun - mc);
+                mrun = mc;
+            }
+            if (t == tw) mine = mrun;
+        }
+        const float ms = mine == -INFINITY ? 0.f : mine;
+        float psum = 0.f;
+        h8 pb[2];
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const float pr = __builtin_amdgcn_exp2f(__builtin_fmaf(tv[r], c2, -ms));
+            psum += pr;
+            pb[r >> 3][r & 7] = (_Float16)pr;
+        }
+        if (dh == 0) {
+            *(h8 *)(pk_smem + T::kP + tw * 2048 + lane * 16) = pb[0];
+            *(h8 *)(pk_smem + T::kP + tw * 2048 + 1024 + lane * 16) = pb[1];
+            ps[tw * 64 + lane] = psum;
+        }
+        if (next) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");  // V^T of this group
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            if (kg + t >= kt1) break;
+            lrun = lrun * alpha[t] + ps[t * 64 + lane];
+            h8 pt[2], vf[NO][2];
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                pt[j] = *(const h8 *)(pk_smem + T::kP + t * 2048 + j * 1024 + lane * 16);
+#pragma unroll
+                for (int tt = 0; tt < NO; tt++) vf[tt][j] = vfrag(tt, t, j);
+            }
+            if (__any(alpha[t] != 1.f)) {
+#pragma unroll
+                for (int tt = 0; tt < NO; tt++) o[tt] *= alpha[t];
+            }
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int tt = 0; tt < NO; tt++) o[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[tt][j], pt[j], o[tt], 0, 0, 0);
+        }
+        if (next) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            issue_v(kg + NT);
+        }
+    }
+    const float ltot = lrun + xor_lane<32>(lrun);
+    const float inv = (qi < Sk && ltot > 0.f) ? __fdiv_rn(1.0f, ltot) : 0.f;
+    float am = 0.f;
+#pragma unroll
+    for (int t = 0; t < NO; t++) {
+        o[t] *= inv;
+#pragma unroll
+        for (int r = 0; r < 16; r++) am = fmaxf(am, fabsf(o[t][r]));
+    }
+    am = fmaxf(am, xor_lane<32>(am));
+    if constexpr (ND == 1) {  // a 128-dim block is two waves'
+        float *xm = (float *)(pk_smem + T::kS + NT * 256);
+        if (half == 0) xm[w * 32 + ql] = am;
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        am = fmaxf(am, xm[(w ^ 1) * 32 + ql]);
+    }
+    const QScale qs = qscale(am);
+    // the bytes through the wave's own K area (pitch DW + 16: rows off each other's banks), out as
+    // 16-byte lane stores
+    unsigned char *stg = pk_smem + kbase;
+    constexpr int PT = DW + 16;
+    const size_t orow = row0 + qi;
+#pragma unroll
+    for (int t = 0; t < NO; t++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const int d = 32 * t + 8 * g + 4 * half;
+            *(uint32_t *)(stg + ql * PT + d) = pack4_magic(o[t][4 * g], o[t][4 * g + 1], o[t][4 * g + 2], o[t][4 * g + 3], qs.inv);
+            if (a.c32 && qi < Sk)
+                *(float4 *)(a.c32 + orow * HD + h * D + w * DW + d) =
+                    make_float4(o[t][4 * g], o[t][4 * g + 1], o[t][4 * g + 2], o[t][4 * g + 3]);
+        }
+    if (half == 0 && qi < Sk && (ND > 1 || (w & 1) == 0)) a.cs[orow * (HD / kQBlock) + h * (D / 128) + w * DW / 128] = qs.sc;
+    constexpr int CPR = DW / 16;
+    const bool al = ((uintptr_t)a.cq & 15) == 0;
+#pragma unroll
+    for (int k = 0; k < 32 * CPR / 64; k++) {
+        const int r = (64 * k + lane) / CPR, ch = lane % CPR, q = q0 + r;
+        const uint4 v = *(const uint4 *)(stg + r * PT + 16 * ch);
+        if (q >= Sk) continue;
+        int8_t *dst = a.cq + (row0 + q) * HD + h * D + w * DW + 16 * ch;
+        if (al) *(uint4 *)dst = v;
+        else *(uint32_t *)dst = v.x, *(uint32_t *)(dst + 4) = v.y, *(uint32_t *)(dst + 8) = v.z, *(uint32_t *)(dst + 12) = v.w;
+    }
+}
+
 // Merge of split key ranges (k_attn_packed with parts > 1; head_dim 256), for the entries of the
 // merge list (work_entry with part 0 and the block's part count): per query row, M = max_p m_p,
 // w_p = 2^(m_p - M) (row maxima in base-2 units, see softmax_tile), ctx = (sum_p w_p o_p) * RN(1 / sum_p w_p l_p), parts in order, then the
@@ -819,6 +1091,31 @@ __global__ __launch_bounds__(256) void k_attn_merge(AttnArgs a, const int32_t *m
         if (a.c32) *(float4 *)(a.c32 + row * HD + h * D + d) = o;
         if ((lane & 31) == 0) a.cs[row * (HD / kQBlock) + h * 2 + half] = qs.sc;
     }
+}
+
+// 32-query blocks while the sequences' blocks (at most H (rows / 32 + B) of them) fit one round of the
+// CUs, one workgroup each: past that their four times larger K and V^T traffic costs more than the idle
+// CUs. us per launch, 128-query | 32-query blocks (32-query blocks in brackets): head_dim 256, 3 heads,
+// 1 x 100 tokens 10.9 | 8.6 [12], 2 x 90-301 18.1 | 13.0 [51], 8 x 64-512 24.5 | 19.6 [237], 16 x 64-512 25.7
+// | 32.0 [459]; 4 heads, window 512, 1 x 2048 65.5 | 34.5 [256], 2 x 1024-2048 70.6 | 66.8 [464]; head_dim
+// 512, 1 x 300 37.2 | 20.9 [40], 1 x 2048 159.6 | 91.6 [256], 2 x 700-1500 123.4 | 120.7 [340], 4 x
+// 1024-2048 168.9 | 303.2 [864]. A sequence of one or two key tiles gains nothing (19 tokens: 7.1 | 7.4 at
+// head_dim 256, 9.5 | 8.2 at 512).
+static bool attn_group_fits(int rows, int B, int max_len, int H, int D) {
+    return (D == 512 || max_len > 64) && (long)H * ((rows + 31) / 32 + B) <= num_cus();
+}
+
+template <int D, bool WIN>
+static int launch_attn_group(hipStream_t s, const AttnArgs &a, dim3 grid, int n_work) {
+    static bool done = false;
+    if (!done) {
+        if (check_hip(hipFuncSetAttribute((const void *)k_attn_group<D, WIN>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          (int)GroupTile<D>::kLds), "attention lds attribute"))
+            return -1;
+        done = true;
+    }
+    hipLaunchKernelGGL((k_attn_group<D, WIN>), grid, dim3(256), GroupTile<D>::kLds, s, a, n_work);
+    return check_hip(hipGetLastError(), "attention launch");
 }
 
 template <int D, bool WIN>
@@ -896,6 +1193,15 @@ static int attention_packed(const char *who, e2mi_stream stream, const uint16_t 
     const bool direct = M % 2 == 0 && (size_t)KV * D * M * 2 < 0x7fffffffu &&
                         (size_t)M * KV * D * 2 < 0x7fffffffu && ((uintptr_t)vt16 & 3) == 0;
     const dim3 grid = work ? dim3(n_work) : dim3((max_len + 127) / 128, H, B);
+    const DeviceRows dr = device_rows();
+    const int rows = dr.ptr && dr.est > 0 ? std::min(dr.est, M) : M;
+    if (direct && !merge && attn_group_fits(rows, B, max_len, H, D)) {
+        const hipStream_t st = (hipStream_t)stream;
+        const dim3 gg = work ? dim3((n_work + 7) / 8 * 32) : dim3((max_len + 31) / 32, H, B);
+        if (D == 512)
+            return window > 0 ? launch_attn_group<512, true>(st, a, gg, n_work) : launch_attn_group<512, false>(st, a, gg, n_work);
+        return window > 0 ? launch_attn_group<256, true>(st, a, gg, n_work) : launch_attn_group<256, false>(st, a, gg, n_work);
+    }
     if (direct && D == 256 && window > 0) {
         if (attn_packed_attr<256, true>()) return -1;
         hipLaunchKernelGGL((k_attn_packed<256, true>), grid, dim3(256), PackedTile<256>::kLds, (hipStream_t)stream, a);

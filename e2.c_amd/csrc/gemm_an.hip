@@ -396,7 +396,7 @@ int launch_add_norm(hipStream_t s, const float *src, const float *res, const flo
 static int gemm_add_norm(hipStream_t s, const int8_t *qa, const float *a_scales, const e2mi_q8w *w, int M,
                          const float *res, const float *gamma_add, float post_scale, const float *gamma_next,
                          float eps, float *x_out, float *xn_out, int8_t *q, float *qs, float *y, bool scale,
-                         const char *who, bool may_split = true) {
+                         const char *who, bool engine = false, float *tmp = nullptr) {
     if (!w || !w->w || !w->scale || (w->N != 512 && w->N != 768) || w->K <= 0 || w->K % kQBlock ||
         w->ld < w->K || w->ld % 16) {
         set_error("%s: the weight must have N = 512 or 768 rows of K = a multiple of 128", who);
@@ -432,12 +432,12 @@ static int gemm_add_norm(hipStream_t s, const int8_t *qa, const float *a_scales,
     a.gamma_n = gamma_next; a.x_out = x_out; a.xn_out = xn_out; a.q = q; a.qs = qs; a.y = y;
     a.lda = w->K; a.ldw = w->ld; a.M = M; a.K = w->K; a.eps = eps; a.post_scale = post_scale;
     const int est = dr.ptr && dr.est > 0 && dr.est < M ? dr.est : M;
-    if (may_split && gemm_an_split(est, D)) {
-        // the projection goes through y, or through x_out beside the residual, which the row kernel then
-        // overwrites row by row
+    if (engine ? tmp != nullptr : gemm_an_split(est, D)) {
+        // the projection goes through the engine's scratch, y, or x_out beside the residual, which the row
+        // kernel then overwrites row by row
         const size_t n = (size_t)M * D;
         auto apart = [&](const float *t) { return t && (t + n <= res || res + n <= t); };
-        float *t = apart(y) ? y : apart(x_out) ? x_out : nullptr;
+        float *t = tmp ? tmp : apart(y) ? y : apart(x_out) ? x_out : nullptr;
         if (t)
             return e2mi_i8_gemm(s, t, D, qa, a_scales, w, M, 0, D) ||
                            launch_add_norm(s, t, res, gamma_add, post_scale, gamma_next, eps, M, D, x_out, xn_out, q, qs, scale)
@@ -453,12 +453,12 @@ static int gemm_add_norm(hipStream_t s, const int8_t *qa, const float *a_scales,
     return fast ? launch_an<768, false, true>(s, dr.ptr, a, grid, uc) : launch_an<768, false, false>(s, dr.ptr, a, grid, uc);
 }
 
-// the engine's: always one launch
+// the engine's: two launches through tmp (M x D floats), or one without it
 int launch_gemm_add_norm(hipStream_t s, const int8_t *qa, const float *a_scales, const e2mi_q8w *w, int M,
                          const float *res, const float *gamma_add, float post_scale, const float *gamma_next,
-                         float eps, float *x_out, float *xn_out, int8_t *q, float *qs, bool scale) {
+                         float eps, float *x_out, float *xn_out, int8_t *q, float *qs, bool scale, float *tmp) {
     return gemm_add_norm(s, qa, a_scales, w, M, res, gamma_add, post_scale, gamma_next, eps, x_out, xn_out, q, qs,
-                         nullptr, scale, "i8_gemm_add_norm", false);
+                         nullptr, scale, "i8_gemm_add_norm", true, tmp);
 }
 
 }  // namespace e2mi

@@ -108,3 +108,40 @@ def test_split_sliding_window(gpu, oracle, rng, holes):
         valid[0, 200:260] = 0
         valid[1, rng.random(S) < 0.2] = 0
     _case(gpu, oracle, rng, valid, 4, 2, 512, 1.0 / 16, "engine")
+
+
+@pytest.mark.parametrize("D,H,KV,window", [(256, 3, 1, 0), (256, 4, 2, 96), (512, 4, 1, 0), (512, 2, 1, 70)])
+@pytest.mark.parametrize("lens", [[1], [33, 127], [129, 31, 64], [300], [65, 200, 8]])
+def test_few_blocks_match_a_full_grid(gpu, rng, D, H, KV, window, lens):
+    """32-query blocks (k_attn_group, few sequences) against the same sequences among enough others
+    that the 128-query kernels take them: bit for bit, with and without a work list, positions with
+    holes, and a context buffer aligned to 4 bytes only."""
+    import e2mi
+    import torch
+    fill = [256] * 24
+    start, r = [], 0
+    for L in lens + fill:
+        start.append(r)
+        r += (L + 7) & ~7
+    M = (r + 255) & ~255
+    g = torch.Generator(device=gpu).manual_seed(sum(lens) + D)
+    t = lambda *s: torch.randn(s, generator=g, device=gpu).half()
+    q, k, v = t(M, H * D) * 0.2, t(M, KV * D), t(KV, D, M)
+    pos = torch.zeros(M, dtype=torch.int32)
+    for s0, L in zip(start, lens + fill):
+        pos[s0:s0 + L] = torch.cumsum(torch.from_numpy(rng.integers(1, 3, L)), 0).int()
+    pos = pos.to(gpu)
+    ti = lambda a: torch.tensor(a, dtype=torch.int32, device=gpu)
+    run = lambda n, m, w, **kw: e2mi.attention_packed_window(
+        q[:m], k[:m], v[..., :m].contiguous(), ti(start[:n]), ti((lens + fill)[:n]), 320, H, KV, D, window=window,
+        pos=pos[:m].contiguous(), work=w, **kw)
+    full = run(len(start), M, None)
+    n, rows = len(lens), start[len(lens) - 1] + lens[-1]
+    m = (rows + 7) & ~7
+    work = torch.from_numpy(e2mi.attention_work(lens, H, window)).to(gpu)
+    odd = torch.zeros(m * H * D + 4, dtype=torch.int8, device=gpu)[4:].view(m, H * D)
+    for got in (run(n, m, None), run(n, m, work), run(n, m, work, cq=odd)):
+        for s0, L in zip(start, lens):
+            for a, b in zip(got, full):
+                a, b = a[s0:s0 + L], b[s0:s0 + L]
+                assert torch.equal(a.view(torch.int8), b.view(torch.int8)), (lens, s0)
