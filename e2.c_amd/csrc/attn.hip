@@ -758,8 +758,8 @@ __global__ __launch_bounds__(512, 1) void k_attn_packed_d512(AttnArgs a) {
     }
 }
 
-// ---- the same attention in blocks of 32 queries, one 4-wave workgroup each: for grids that leave CUs
-// idle in 128-query blocks, where a block's time is its serial walk over the key tiles. The waves
+// ---- the same attention in blocks of 32 QS queries (QS = 1, 2), four waves per 32: for grids that leave
+// CUs idle in 128-query blocks, where a block's time is its serial walk over the key tiles. The waves
 // take NT = 4 (head_dim 512: 2) key tiles at once: wave w computes the logits of tile w (head_dim
 // 512: of tile w % 2 over dims 256 (w / 2) .. + 255, the two partial sums added as in
 // k_attn_packed_d512), then the context's dims D/4 w .. + D/4 - 1 over all NT tiles. The tiles' row
@@ -767,39 +767,47 @@ __global__ __launch_bounds__(512, 1) void k_attn_packed_d512(AttnArgs a) {
 // wave walks the running max over the NT tiles in order, so each query sees the arithmetic of
 // k_attn_packed (k_attn_packed_d512) bit for bit: the same MFMA chains, rescales and sums; tiles with
 // no key for a query change nothing there, and are skipped here.
-// K and V^T fragments are private to a wave (16 KB each), loaded straight to LDS with no barrier: the
-// next group's K while this group's softmax and context run, its V^T under the next logits.
-template <int D>
+// With QS = 1 the K and V^T fragments are private to a wave (16 KB each), loaded straight to LDS with no
+// barrier: the next group's K while this group's softmax and context run, its V^T under the next
+// logits. With QS = 2 two waves share and load a half each (half the traffic a query, one more barrier a
+// group).
+template <int D, int QS>
 struct GroupTile {
     static constexpr int ND = D / 256, NT = 4 / ND, DW = D / 4;  // dim halves, tiles a group, dims a wave
     static constexpr int kW = 32 * 1024;                         // a wave's K (16 KB) and V^T (16 KB)
-    static constexpr int kP = 4 * kW, kX = kP + NT * 2048, kM = kX + (ND > 1 ? 16384 : 0), kS = kM + NT * 128;
-    static constexpr size_t kLds = kS + NT * 256 + 4 * 128;
+    // per 32 queries: the probabilities, at 512 the exchanged logits (with QS = 2 in the same place: a
+    // barrier lies between a group's last probability read and the next logits), the tiles' row maxima
+    // and row sums, the waves' context maxima
+    static constexpr int kX = QS == 1 ? NT * 2048 : 0, kM = ND > 1 ? kX + 8192 : NT * 2048, kS = kM + NT * 128, kC = kS + NT * 256, kQ = kC + 512;
+    static constexpr size_t kLds = 4 * kW + QS * kQ;
+    static_assert(kLds <= 160 * 1024, "LDS budget");
 };
 
-template <int D, bool WIN>
-__global__ __launch_bounds__(256, 1) void k_attn_group(AttnArgs a, int n_work) {
-    using T = GroupTile<D>;
+template <int D, bool WIN, int QS>
+__global__ __launch_bounds__(256 * QS, 1) void k_attn_group(AttnArgs a, int n_work) {
+    using T = GroupTile<D, QS>;
     constexpr int ND = T::ND, NT = T::NT, DW = T::DW, NO = DW / 32;
     extern __shared__ __align__(16) unsigned char pk_smem[];
-    // work entry i's four blocks on the XCD of workgroup i of a 128-query grid (i % 8)
-    int q0 = blockIdx.x * 32, h = blockIdx.y, b = blockIdx.z;
+    // work entry i's 4 / QS blocks on the XCD of workgroup i of a 128-query grid (i % 8)
+    constexpr int NBK = 4 / QS;
+    int q0 = blockIdx.x * (32 * QS), h = blockIdx.y, b = blockIdx.z;
     if (a.work) {
-        const int i = (blockIdx.x >> 5) * 8 + (blockIdx.x & 7);
+        const int i = (blockIdx.x / (8 * NBK)) * 8 + (blockIdx.x & 7);
         const int item = i < n_work ? a.work[i] : -1;
         if (item < 0) return;
         b = item & 0xffff;
         h = (item >> 16) & 0xf;
-        q0 = (item >> 24) * 128 + ((blockIdx.x >> 3) & 3) * 32;
+        q0 = (item >> 24) * 128 + ((blockIdx.x >> 3) % NBK) * (32 * QS);
     }
     const int Sk = a.seq_len[b];
     if (q0 >= Sk) return;
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, ql = lane & 31;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), w = wv & 3, sub = wv >> 2;
+    const int qw = q0 + 32 * sub;  // this wave's queries
     const int tw = w % NT, dh = w / NT;  // this wave's tile of a group and dim half
     const int S = a.S, HD = a.H * D, kvh = h / (a.H / a.KV);
     const size_t row0 = (size_t)a.seq_start[b];
-    const int qi = q0 + ql;
+    const int qi = qw + ql;
     const int qc = min(qi, Sk - 1);
     h8 qf[16];
     {
@@ -811,7 +819,7 @@ __global__ __launch_bounds__(256, 1) void k_attn_group(AttnArgs a, int n_work) {
     int kt0 = 0, kt1 = (Sk + kKT - 1) / kKT;
     int pq0 = 0, pq1 = 0, pqi = qc;
     if constexpr (WIN) {
-        const int q1 = min(q0 + 31, Sk - 1);
+        const int q1 = min(q0 + 32 * QS - 1, Sk - 1);
         kt0 = max(q0 - W, 0) / kKT;
         kt1 = min((min(q1 + W, Sk - 1)) / kKT + 1, kt1);
         pq0 = a.pos ? a.pos[row0 + q0] : q0;
@@ -830,8 +838,8 @@ __global__ __launch_bounds__(256, 1) void k_attn_group(AttnArgs a, int n_work) {
     auto issue_k = [&](int kt) {
         const int k0 = kt * kKT + tw * kKT;
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int r = 2 * i + half;
+        for (int ii = 0; ii < 16 / QS; ii++) {
+            const int i = 16 / QS * sub + ii, r = 2 * i + half;
             dma16(rK, lds0 + kbase + i * 1024u,
                   (uint32_t)(swap23(2 * i) + half + k0) * rowB + dh * 512u + (uint32_t)((ql ^ (r & 7)) << 4), 0u);
         }
@@ -841,8 +849,8 @@ __global__ __launch_bounds__(256, 1) void k_attn_group(AttnArgs a, int n_work) {
     auto issue_v = [&](int kt) {
         const int k0 = kt * kKT;
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int r = (64 / LPR) * i + vr0;
+        for (int ii = 0; ii < 16 / QS; ii++) {
+            const int i = 16 / QS * sub + ii, r = (64 / LPR) * i + vr0;
             const int cx = (lane % LPR) ^ (NT == 4 ? (r & 15) : ((r >> 1) & 7));
             dma16(rV, lds0 + vbase + i * 1024u,
                   k0 + 8 * cx < Sk ? (uint32_t)(((w * DW + r) * S + k0 + 8 * cx) * 2) : 0x80000000u, 0u);
@@ -857,7 +865,8 @@ __global__ __launch_bounds__(256, 1) void k_attn_group(AttnArgs a, int n_work) {
         const int sw = NT == 4 ? (d & 15) : ((d >> 1) & 7);
         return *(const h8 *)(pk_smem + vbase + d * (NT * 64) + ((c ^ sw) << 4));
     };
-    float *mx = (float *)(pk_smem + T::kM), *ps = (float *)(pk_smem + T::kS);
+    unsigned char *const sq = pk_smem + 4 * T::kW + sub * T::kQ;
+    float *mx = (float *)(sq + T::kM), *ps = (float *)(sq + T::kS);
 
     f16v o[NO];
 #pragma unroll
@@ -865,12 +874,19 @@ __global__ __launch_bounds__(256, 1) void k_attn_group(AttnArgs a, int n_work) {
     float mrun = -INFINITY, lrun = 0.f;
     const float c2 = a.scale * 1.44269504088896341f;  // logits in base-2 units
     issue_k(kt0);
-    issue_v(kt0);
+    if constexpr (QS == 1) issue_v(kt0);
     __builtin_amdgcn_s_waitcnt(0x0F70);  // the Q loads, after the first tiles' (see k_attn_packed)
     for (int kg = kt0; kg < kt1; kg += NT) {
         const int kt = kg + tw, k0 = kt * kKT;
         const bool next = kg + NT < kt1;
-        asm volatile("s_waitcnt vmcnt(16)" ::: "memory");  // K of this group (V^T was issued after it)
+        // K of this group (QS = 1: V^T was issued after it; QS = 2: the barrier shows both waves' halves, and
+        // ends every wave's V^T reads of the previous group)
+        if constexpr (QS == 1) {
+            asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+        } else {
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            issue_v(kg);
+        }
         f16v st = (f16v){};
         h8 kr[PFK];
 #pragma unroll
@@ -881,21 +897,23 @@ __global__ __launch_bounds__(256, 1) void k_attn_group(AttnArgs a, int n_work) {
             if (s + PFK < 16) kr[s % PFK] = *(const h8 *)(pk_smem + krd[(s + PFK) & 3] + ((s + PFK) >> 2) * 128);
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (next) issue_k(kg + NT);  // (this wave's K reads have completed: the MFMAs took them)
+        if (QS == 1 && next) issue_k(kg + NT);  // (this wave's K reads have completed: the MFMAs took them)
         float tv[16];
         if constexpr (ND > 1) {
-            float *xw = (float *)(pk_smem + T::kX) + (w * 64 + lane) * 4;
-            const float *xp = (const float *)(pk_smem + T::kX) + ((w ^ NT) * 64 + lane) * 4;
+            // the upper dim half's partial logits to the lower half's wave, which runs the tile's softmax
+            float *x = (float *)(sq + T::kX) + tw * 1024 + lane * 4;
+            if (dh == 1) {
 #pragma unroll
-            for (int r = 0; r < 16; r += 4) *(float4 *)(xw + r * 256) = make_float4(st[r], st[r + 1], st[r + 2], st[r + 3]);
+                for (int r = 0; r < 16; r += 4) *(float4 *)(x + r * 64) = make_float4(st[r], st[r + 1], st[r + 2], st[r + 3]);
+            }
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
             for (int r = 0; r < 16; r += 4) {
-                const float4 x = *(const float4 *)(xp + r * 256);
-                tv[r] = st[r] + x.x;
-                tv[r + 1] = st[r + 1] + x.y;
-                tv[r + 2] = st[r + 2] + x.z;
-                tv[r + 3] = st[r + 3] + x.w;
+                const float4 y = *(const float4 *)(x + r * 64);
+                tv[r] = st[r] + y.x;
+                tv[r + 1] = st[r + 1] + y.y;
+                tv[r + 2] = st[r + 2] + y.z;
+                tv[r + 3] = st[r + 3] + y.w;
             }
         } else {
 #pragma unroll
@@ -929,6 +947,7 @@ __global__ __launch_bounds__(256, 1) void k_attn_group(AttnArgs a, int n_work) {
         mloc = fmaxf(mloc, xor_lane<32>(mloc));
         if (half == 0 && dh == 0) mx[tw * 32 + ql] = mloc;
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (QS > 1 && next) issue_k(kg + NT);  // (every wave is past its K reads)
         float alpha[NT], mine = 0.f;
 #pragma unroll
         for (int t = 0; t < NT; t++) {
@@ -941,20 +960,21 @@ __global__ __launch_bounds__(256, 1) void k_attn_group(AttnArgs a, int n_work) {
             if (t == tw) mine = mrun;
         }
         const float ms = mine == -INFINITY ? 0.f : mine;
-        float psum = 0.f;
-        h8 pb[2];
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const float pr = __builtin_amdgcn_exp2f(__builtin_fmaf(tv[r], c2, -ms));
-            psum += pr;
-            pb[r >> 3][r & 7] = (_Float16)pr;
-        }
         if (dh == 0) {
-            *(h8 *)(pk_smem + T::kP + tw * 2048 + lane * 16) = pb[0];
-            *(h8 *)(pk_smem + T::kP + tw * 2048 + 1024 + lane * 16) = pb[1];
+            float psum = 0.f;
+            h8 pb[2];
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const float pr = __builtin_amdgcn_exp2f(__builtin_fmaf(tv[r], c2, -ms));
+                psum += pr;
+                pb[r >> 3][r & 7] = (_Float16)pr;
+            }
+            *(h8 *)(sq + tw * 2048 + lane * 16) = pb[0];
+            *(h8 *)(sq + tw * 2048 + 1024 + lane * 16) = pb[1];
             ps[tw * 64 + lane] = psum;
         }
-        if (next) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");  // V^T of this group
+        // V^T of this group (the next K was issued after it)
+        if (next) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(16 / QS) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
@@ -964,7 +984,7 @@ __global__ __launch_bounds__(256, 1) void k_attn_group(AttnArgs a, int n_work) {
             h8 pt[2], vf[NO][2];
 #pragma unroll
             for (int j = 0; j < 2; j++) {
-                pt[j] = *(const h8 *)(pk_smem + T::kP + t * 2048 + j * 1024 + lane * 16);
+                pt[j] = *(const h8 *)(sq + t * 2048 + j * 1024 + lane * 16);
 #pragma unroll
                 for (int tt = 0; tt < NO; tt++) vf[tt][j] = vfrag(tt, t, j);
             }
@@ -977,7 +997,7 @@ __global__ __launch_bounds__(256, 1) void k_attn_group(AttnArgs a, int n_work) {
 #pragma unroll
                 for (int tt = 0; tt < NO; tt++) o[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[tt][j], pt[j], o[tt], 0, 0, 0);
         }
-        if (next) {
+        if (QS == 1 && next) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             issue_v(kg + NT);
         }
@@ -993,16 +1013,16 @@ __global__ __launch_bounds__(256, 1) void k_attn_group(AttnArgs a, int n_work) {
     }
     am = fmaxf(am, xor_lane<32>(am));
     if constexpr (ND == 1) {  // a 128-dim block is two waves'
-        float *xm = (float *)(pk_smem + T::kS + NT * 256);
+        float *xm = (float *)(sq + T::kC);
         if (half == 0) xm[w * 32 + ql] = am;
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         am = fmaxf(am, xm[(w ^ 1) * 32 + ql]);
     }
     const QScale qs = qscale(am);
-    // the bytes through the wave's own K area (pitch DW + 16: rows off each other's banks), out as
-    // 16-byte lane stores
-    unsigned char *stg = pk_smem + kbase;
+    // the bytes through an area of the wave's own in the K space (its last reads were before the last
+    // barriers; pitch DW + 16: rows off each other's banks), out as 16-byte lane stores
     constexpr int PT = DW + 16;
+    unsigned char *stg = pk_smem + kbase + sub * (32 * PT);
     const size_t orow = row0 + qi;
 #pragma unroll
     for (int t = 0; t < NO; t++)
@@ -1019,7 +1039,7 @@ __global__ __launch_bounds__(256, 1) void k_attn_group(AttnArgs a, int n_work) {
     const bool al = ((uintptr_t)a.cq & 15) == 0;
 #pragma unroll
     for (int k = 0; k < 32 * CPR / 64; k++) {
-        const int r = (64 * k + lane) / CPR, ch = lane % CPR, q = q0 + r;
+        const int r = (64 * k + lane) / CPR, ch = lane % CPR, q = qw + r;
         const uint4 v = *(const uint4 *)(stg + r * PT + 16 * ch);
         if (q >= Sk) continue;
         int8_t *dst = a.cq + (row0 + q) * HD + h * D + w * DW + 16 * ch;
@@ -1093,29 +1113,40 @@ __global__ __launch_bounds__(256) void k_attn_merge(AttnArgs a, const int32_t *m
     }
 }
 
-// 32-query blocks while the sequences' blocks (at most H (rows / 32 + B) of them) fit one round of the
-// CUs, one workgroup each: past that their four times larger K and V^T traffic costs more than the idle
-// CUs. us per launch, 128-query | 32-query blocks (32-query blocks in brackets): head_dim 256, 3 heads,
-// 1 x 100 tokens 10.9 | 8.6 [12], 2 x 90-301 18.1 | 13.0 [51], 8 x 64-512 24.5 | 19.6 [237], 16 x 64-512 25.7
-// | 32.0 [459]; 4 heads, window 512, 1 x 2048 65.5 | 34.5 [256], 2 x 1024-2048 70.6 | 66.8 [464]; head_dim
-// 512, 1 x 300 37.2 | 20.9 [40], 1 x 2048 159.6 | 91.6 [256], 2 x 700-1500 123.4 | 120.7 [340], 4 x
-// 1024-2048 168.9 | 303.2 [864]. A sequence of one or two key tiles gains nothing (19 tokens: 7.1 | 7.4 at
-// head_dim 256, 9.5 | 8.2 at 512).
-static bool attn_group_fits(int rows, int B, int max_len, int H, int D) {
-    return (D == 512 || max_len > 64) && (long)H * ((rows + 31) / 32 + B) <= num_cus();
+// Blocks of 32 (1), 64 (2) or 128 (0) queries by how many of them the sequences have, about H (rows / 32 +
+// B / 2) and H (rows / 64 + B / 2): 32 while those leave a fifth of the CUs idle, 64 while they fit one round
+// of the CUs, one workgroup each; past that the larger K and V^T traffic of small blocks costs more than
+// idle CUs. us per launch at 128 | 64 | 32 queries (32-query blocks in brackets): head_dim 256, 3 heads, 1 x
+// 100 tokens 10.9 | 10.3 | 8.7 [12], 2 x 90-301 18.0 | 15.1 | 13.0 [51], 8 x 64-512 24.7 | 18.2 | 20.1 [237], 16
+// x 64-512 26.1 | 21.4 | 32.8 [459], 32 x 64-512 28.8 | 39.4 | 57.7 [930]; 4 heads, window 512, 1 x 2048 64.8 |
+// 34.6 | 34.5 [256], 2 x 1024-2048 71.5 | 37.6 | 65.6 [464], 4 x 1024-2048 76.3 | 70.9 | 108.3 [864], 8 x
+// 1024-2048 89.0 | 108.7 | 175.4; head_dim 512, 1 x 300 36.5 | 21.6 | 19.6 [40], 1 x 2048 158.8 | 95.3 | 87.0 [256],
+// 2 x 700-1500 122.9 | 73.7 | 115.4 [340], 4 x 1024-2048 166.2 | 185.8 | 289.9. At head_dim 256 a sequence of one
+// or two key tiles gains nothing (19 tokens: 7.1 | 7.8 | 7.4).
+static int attn_group_blocks(int rows, int B, int max_len, int H, int D) {
+    if (D == 256 && max_len <= 64) return 0;
+    const double C = num_cus();
+    if (H * (rows / 32.0 + B / 2.0) <= 0.8 * C) return 1;
+    return H * (rows / 64.0 + B / 2.0) <= C ? 2 : 0;
 }
 
-template <int D, bool WIN>
-static int launch_attn_group(hipStream_t s, const AttnArgs &a, dim3 grid, int n_work) {
+template <int D, bool WIN, int QS>
+static int launch_attn_group(hipStream_t s, const AttnArgs &a, int max_len, int n_work) {
+    using T = GroupTile<D, QS>;
     static bool done = false;
     if (!done) {
-        if (check_hip(hipFuncSetAttribute((const void *)k_attn_group<D, WIN>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                          (int)GroupTile<D>::kLds), "attention lds attribute"))
+        if (check_hip(hipFuncSetAttribute((const void *)k_attn_group<D, WIN, QS>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          (int)T::kLds), "attention lds attribute"))
             return -1;
         done = true;
     }
-    hipLaunchKernelGGL((k_attn_group<D, WIN>), grid, dim3(256), GroupTile<D>::kLds, s, a, n_work);
+    const dim3 grid = a.work ? dim3((n_work + 7) / 8 * 8 * (4 / QS)) : dim3((max_len + 32 * QS - 1) / (32 * QS), a.H, a.B);
+    hipLaunchKernelGGL((k_attn_group<D, WIN, QS>), grid, dim3(256 * QS), T::kLds, s, a, n_work);
     return check_hip(hipGetLastError(), "attention launch");
+}
+template <int D, bool WIN>
+static int launch_attn_group(hipStream_t s, const AttnArgs &a, int max_len, int n_work, int qs) {
+    return qs == 1 ? launch_attn_group<D, WIN, 1>(s, a, max_len, n_work) : launch_attn_group<D, WIN, 2>(s, a, max_len, n_work);
 }
 
 template <int D, bool WIN>
@@ -1195,12 +1226,14 @@ static int attention_packed(const char *who, e2mi_stream stream, const uint16_t 
     const dim3 grid = work ? dim3(n_work) : dim3((max_len + 127) / 128, H, B);
     const DeviceRows dr = device_rows();
     const int rows = dr.ptr && dr.est > 0 ? std::min(dr.est, M) : M;
-    if (direct && !merge && attn_group_fits(rows, B, max_len, H, D)) {
+    const int qs = merge ? 0 : attn_group_blocks(rows, B, max_len, H, D);
+    if (direct && qs) {
         const hipStream_t st = (hipStream_t)stream;
-        const dim3 gg = work ? dim3((n_work + 7) / 8 * 32) : dim3((max_len + 31) / 32, H, B);
         if (D == 512)
-            return window > 0 ? launch_attn_group<512, true>(st, a, gg, n_work) : launch_attn_group<512, false>(st, a, gg, n_work);
-        return window > 0 ? launch_attn_group<256, true>(st, a, gg, n_work) : launch_attn_group<256, false>(st, a, gg, n_work);
+            return window > 0 ? launch_attn_group<512, true>(st, a, max_len, n_work, qs)
+                              : launch_attn_group<512, false>(st, a, max_len, n_work, qs);
+        return window > 0 ? launch_attn_group<256, true>(st, a, max_len, n_work, qs)
+                          : launch_attn_group<256, false>(st, a, max_len, n_work, qs);
     }
     if (direct && D == 256 && window > 0) {
         if (attn_packed_attr<256, true>()) return -1;

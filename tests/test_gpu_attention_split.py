@@ -111,14 +111,14 @@ def test_split_sliding_window(gpu, oracle, rng, holes):
 
 
 @pytest.mark.parametrize("D,H,KV,window", [(256, 3, 1, 0), (256, 4, 2, 96), (512, 4, 1, 0), (512, 2, 1, 70)])
-@pytest.mark.parametrize("lens", [[1], [33, 127], [129, 31, 64], [300], [65, 200, 8]])
+@pytest.mark.parametrize("lens", [[1], [33, 127], [129, 31, 64], [300], [65, 200, 8], [700, 650, 129, 700, 690, 577]])
 def test_few_blocks_match_a_full_grid(gpu, rng, D, H, KV, window, lens):
-    """32-query blocks (k_attn_group, few sequences) against the same sequences among enough others
-    that the 128-query kernels take them: bit for bit, with and without a work list, positions with
-    holes, and a context buffer aligned to 4 bytes only."""
+    """Blocks of 32 and (the last lengths) 64 queries (k_attn_group, few sequences) against the same
+    sequences among enough others that the 128-query kernels take them: bit for bit, with and without
+    a work list, positions with holes, and a context buffer aligned to 4 bytes only."""
     import e2mi
     import torch
-    fill = [256] * 24
+    fill = [256] * 40
     start, r = [], 0
     for L in lens + fill:
         start.append(r)
@@ -133,7 +133,7 @@ def test_few_blocks_match_a_full_grid(gpu, rng, D, H, KV, window, lens):
     pos = pos.to(gpu)
     ti = lambda a: torch.tensor(a, dtype=torch.int32, device=gpu)
     run = lambda n, m, w, **kw: e2mi.attention_packed_window(
-        q[:m], k[:m], v[..., :m].contiguous(), ti(start[:n]), ti((lens + fill)[:n]), 320, H, KV, D, window=window,
+        q[:m], k[:m], v[..., :m].contiguous(), ti(start[:n]), ti((lens + fill)[:n]), 704, H, KV, D, window=window,
         pos=pos[:m].contiguous(), work=w, **kw)
     full = run(len(start), M, None)
     n, rows = len(lens), start[len(lens) - 1] + lens[-1]
