@@ -13,16 +13,13 @@
 // The context is then quantized per (row, 128 dims) for the O-projection GEMM, as in attn.hip.
 //
 // Kernels:
-//   k_i8_qk_prep   one wave per (row, q head | k head): Q per 128, K per row (float4 per lane)
-//   k_i8_vmax      per (sequence, kv head, 64-row chunk): column maxima of V
+//   k_i8_prep      one wave per (row, q head | k head): Q per 128, K per row (float4 per lane); and
+//                  per (sequence, kv head, 64-row chunk): column maxima of V
 //   k_i8_vquant    per (sequence, kv head, 32-row chunk): V^T bytes (thread d writes 32 bytes of
 //                  row d of V^T [KV][D][M]) and the per-dim scales
-//   k_attn_i8      a workgroup is (sequence, head, 128 queries), 4 waves of 32 queries, one wave
-//                  per SIMD (the two f32 context sets need 256 registers). Pass 1 walks the key
-//                  tiles for each query's softmax max and sum (online); pass 2 walks them again per
-//                  128-key block: the block's probabilities (recomputed, bit-identical scores),
-//                  their quantization with the block's scale (the largest probability is the one of
-//                  the largest score: exp and the multiply by 1/sum are monotone), then
+//   k_attn_i8      a workgroup is (sequence, head, 32 queries). Pass 1 walks the key tiles for each
+//                  query's softmax max and sum (online); pass 2 walks them again per 128-key block:
+//                  the block's probabilities, their quantization with the block's scale, then
 //                  O^T += V^T P^T on int8 MFMA with int32 accumulators folded into f32 once per
 //                  block. S^T = K Q^T as in attn.hip: K tile rows are permuted so a lane's 16
 //                  logits are 16 consecutive keys of its query, exactly its P^T operand bytes.
@@ -31,10 +28,8 @@
 namespace e2mi {
 
 constexpr int kI8D = 256;                           // head dim
-constexpr int kI8Tile = 8192;                       // K [32 keys][256] or V^T [256 d][32 keys]
+constexpr int kI8Tile = 8192;                       // K [32 keys][256] or V^T [64 d][128 keys]
 constexpr int kI8Buf = kI8Tile + 256;               // + the tile's key scales (64 loaded, 32 used)
-constexpr int kI8Ring = 3;                          // tile buffers: loads two tiles ahead
-constexpr int kAttnI8Lds = kI8Ring * kI8Buf + kI8D * 4;  // + the sequence's V scales
 
 // ---------------------------------------------------------------- Q and K quantization
 struct I8PrepArgs {
@@ -48,11 +43,34 @@ struct I8PrepArgs {
     float *vs;                     // [B][KV][D]
     const int32_t *seq_start, *seq_len;
     int M, H, KV, nch;
+    int nbk, nv;  // B KV, and its workgroups of the first launch (nbk nch)
 };
 
-__global__ __launch_bounds__(256) void k_i8_qk_prep(I8PrepArgs a) {
+// V's part of the launch: workgroup c B KV + (b, kv) takes the column maxima of rows [64 c, 64 c + 64)
+// of the sequence, thread = dim
+__device__ inline void i8_vmax(const I8PrepArgs &a, int blk) {
+    const int bk = blk % a.nbk, c = blk / a.nbk, b = bk / a.KV, kv = bk % a.KV, d = threadIdx.x;
+    const int L = a.seq_len[b], r0 = 64 * c;
+    if (r0 >= L) return;
+    const int r1 = min(L, r0 + 64);
+    const size_t st = (size_t)a.KV * kI8D;
+    const float *src = a.v32 + ((size_t)a.seq_start[b] + r0) * st + kv * kI8D + d;
+    float m8[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    int r = r0;
+    for (; r + 8 <= r1; r += 8, src += 8 * st)
+#pragma unroll
+        for (int e = 0; e < 8; e++) m8[e] = fmaxf(m8[e], fabsf(src[e * st]));
+    for (; r < r1; r++, src += st) m8[0] = fmaxf(m8[0], fabsf(*src));
+    float am = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; e++) am = fmaxf(am, m8[e]);
+    a.vpart[((size_t)bk * a.nch + c) * kI8D + d] = am;
+}
+
+__global__ __launch_bounds__(256) void k_i8_prep(I8PrepArgs a) {
+    if ((int)blockIdx.x < a.nv) return i8_vmax(a, blockIdx.x);
     const int lane = threadIdx.x & 63;
-    const long item = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const long item = (long)(blockIdx.x - a.nv) * 4 + (threadIdx.x >> 6);
     const int per = a.H + a.KV;
     if (item >= (long)a.M * per) return;
     const int row = (int)(item / per), j = (int)(item % per);
@@ -75,26 +93,6 @@ __global__ __launch_bounds__(256) void k_i8_qk_prep(I8PrepArgs a) {
 }
 
 // ---------------------------------------------------------------- V^T quantization
-// grid (B * KV, nch): column maxima of rows [64 c, 64 c + 64) of the sequence, thread = dim
-__global__ __launch_bounds__(256) void k_i8_vmax(I8PrepArgs a) {
-    const int b = blockIdx.x / a.KV, kv = blockIdx.x % a.KV, c = blockIdx.y, d = threadIdx.x;
-    const int L = a.seq_len[b], r0 = 64 * c;
-    if (r0 >= L) return;
-    const int r1 = min(L, r0 + 64);
-    const size_t st = (size_t)a.KV * kI8D;
-    const float *src = a.v32 + ((size_t)a.seq_start[b] + r0) * st + kv * kI8D + d;
-    float m8[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    int r = r0;
-    for (; r + 8 <= r1; r += 8, src += 8 * st)
-#pragma unroll
-        for (int e = 0; e < 8; e++) m8[e] = fmaxf(m8[e], fabsf(src[e * st]));
-    for (; r < r1; r++, src += st) m8[0] = fmaxf(m8[0], fabsf(*src));
-    float am = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; e++) am = fmaxf(am, m8[e]);
-    a.vpart[((size_t)blockIdx.x * a.nch + c) * kI8D + d] = am;
-}
-
 // grid (B * KV, ceil(max_len / 32)): thread d reduces its column's chunk maxima, then quantizes rows
 // [32 c, 32 c + 32) of the sequence into 32 bytes of V^T row d
 __global__ __launch_bounds__(256) void k_i8_vquant(I8PrepArgs a) {
@@ -145,24 +143,42 @@ struct AttnI8Args {
     int M, H, KV;
 };
 
-__global__ __launch_bounds__(256, 1) void k_attn_i8(AttnI8Args a) {
+// A block is 32 queries, four waves each on a key tile of its own. Pass 1 takes four tiles at once:
+// wave w the scores of tile w; the tiles' maxima and partial sums are exchanged through LDS and folded
+// in tile order by every wave. Pass 2 quantizes a 128-key block's four tiles in the four waves,
+// exchanges the bytes, and each wave computes 64 of the 256 dims over the block. A wave's K tiles and
+// V^T pieces (8 KB each: [32 keys][256], [64 dims][128 keys]) share a ring of two buffers, loaded a
+// step ahead. KEEP (no sequence longer than 512 keys): a wave keeps its four tiles' scores in
+// registers for pass 2, else they are computed again.
+// What bounds it is the chain of a block: load, scores, exchange, probabilities, exchange, context. A
+// workgroup of four waves that walk the tiles together, 32 queries each, has one wave on a SIMD and
+// a chain four times as long; here two workgroups share a CU. us per call with the quantization (about
+// 16), such workgroups -> these: 3 heads, 1 x 100 tokens 26.8 -> 16.4, 12 x 64-512 70.8 -> 36.4, 64 x 64-512 125.2
+// -> 98.1; 4 heads, 2 x 1024-2048 217.7 -> 102.4, 16 x 1024-2048 661.7 -> 447.7. KEEP against computing the scores
+// again: 36.4 | 41.0 and 98.1 | 111.9. Blocks of 64 queries on eight waves: 36.6, 103.8, 93.9 and 451.4.
+constexpr int kI8Keep = 512;
+constexpr int kI8P = 0, kI8M = 4096, kI8L = kI8M + 1024, kI8X = kI8L + 2048;  // bytes, maxima, partial sums
+constexpr int kI8V = 8 * kI8Buf, kI8S = kI8V + kI8D * 4, kAttnI8Lds = kI8S + kI8X;
+
+template <bool KEEP>
+__global__ __launch_bounds__(256, 2) void k_attn_i8(AttnI8Args a, int n_work) {
     extern __shared__ __align__(16) unsigned char smem[];
-    int qb = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-    if (a.work) {
-        const int item = a.work[blockIdx.x];
+    int q0 = blockIdx.x * 32, h = blockIdx.y, b = blockIdx.z;
+    if (a.work) {  // work entry i's four blocks on one XCD (i % 8)
+        const int i = (blockIdx.x >> 5) * 8 + (blockIdx.x & 7);
+        const int item = i < n_work ? a.work[i] : -1;
         if (item < 0) return;
         b = item & 0xffff;
-        h = (item >> 16) & 0xf;  // (one part: work_entry(b, h, 0, 1, qb))
-        qb = item >> 24;
+        h = (item >> 16) & 0xf;  // (one part: work_entry(b, h, 0, 1, query block))
+        q0 = (item >> 24) * 128 + ((blockIdx.x >> 3) & 3) * 32;
     }
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, half = lane >> 5;
+    const int Sk = a.seq_len[b];
+    if (q0 >= Sk) return;
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, ql = lane & 31;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int HD = a.H * kI8D, kvh = h / (a.H / a.KV);
     const size_t row0 = (size_t)a.seq_start[b];
-    const int Sk = a.seq_len[b];
-    if (qb * 128 >= Sk) return;
-
-    const int qi = qb * 128 + w * 32 + (lane & 31);  // this lane's query
-    const int qc = min(qi, Sk - 1);
+    const int qi = q0 + ql, qc = min(qi, Sk - 1);  // this lane's query
     // Q^T operand (B of S^T = K Q^T): the query's d = 32 kk + 16 half .. + 16
     v4i qf[8];
     {
@@ -171,100 +187,65 @@ __global__ __launch_bounds__(256, 1) void k_attn_i8(AttnI8Args a) {
         for (int kk = 0; kk < 8; kk++) qf[kk] = *(const v4i *)(qp + 32 * kk);
     }
     const float qs0 = a.qs[(row0 + qc) * a.H * 2 + h * 2], qs1 = a.qs[(row0 + qc) * a.H * 2 + h * 2 + 1];
-    float *vs_l = (float *)(smem + kI8Ring * kI8Buf);
+    float *vs_l = (float *)(smem + kI8V);
     vs_l[tid] = a.vs[((size_t)b * a.KV + kvh) * kI8D + tid];
     // the loads above complete here, under a wait the compiler sees: otherwise its wait would sit
-    // inside the tile loop and also cover the tile loads in flight
+    // inside a loop and also cover the tile loads in flight
     __builtin_amdgcn_s_waitcnt(0x0F70);
 
     const int ntiles = (Sk + 31) / 32, nblk = (ntiles + 3) / 4;
-    const uint32_t rowB = (uint32_t)a.KV * kI8D;
+    const uint32_t rowB = (uint32_t)a.KV * kI8D, vpitch = 2u * (uint32_t)a.M;
     const v4u rK = rsrc_words(a.k8 + row0 * rowB + kvh * kI8D, (uint32_t)Sk * rowB);
     const v4u rKS = rsrc_words(a.ks + row0 * a.KV + kvh, (uint32_t)Sk * a.KV * 4);
     const v4u rV = rsrc_words(a.vt8 + (size_t)kvh * kI8D * 2 * a.M, (uint32_t)((size_t)kI8D * 2 * a.M));
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const lds_void *)smem);
-    const int wu = __builtin_amdgcn_readfirstlane(w);
-    // K tile: load i (wave w issues 2 w, 2 w + 1) fills physical rows rho = 4 i + lane / 16, 16-byte
-    // position lane % 16 holding chunk (lane % 16) ^ (rho % 16), of key kappa(rho) =
-    // 16 ((rho / 4) % 2) + 4 (rho / 8) + rho % 4 = 16 (i % 2) + 4 (i / 2) + lane / 16
-    uint32_t kvo[2];
+    // K: load i fills physical rows rho = 4 i + lane / 16, 16-byte position lane % 16 holding chunk
+    // (lane % 16) ^ (rho % 16), of key 16 ((rho / 4) % 2) + 4 (rho / 8) + rho % 4 = 16 (i % 2) + 4 (i / 2) + lane / 16;
+    // keys past the sequence are out of the buffer's range and read as 0
+    auto issue_k = [&](int g, int buf) __attribute__((always_inline)) {
+        const int k0 = (4 * g + w) * 32;
+        const uint32_t base = lds0 + (uint32_t)((2 * w + buf) * kI8Buf);
 #pragma unroll
-    for (int e = 0; e < 2; e++) {
-        const int i = 2 * wu + e;
-        kvo[e] = (uint32_t)(lane >> 4) * rowB + (uint32_t)(((lane & 15) ^ ((4 * i + (lane >> 4)) & 15)) << 4);
-    }
-    // V^T tile: load i (wave w issues 2 w, 2 w + 1) fills rows d = 32 i + lane / 2, position lane % 2
-    // holding chunk (lane % 2) ^ ((d / 8) % 2) = (lane % 2) ^ ((lane / 16) % 2)
-    const uint32_t vpitch = 2u * (uint32_t)a.M;
-    const uint32_t vvo = (uint32_t)(lane >> 1) * vpitch + (uint32_t)(((lane & 1) ^ ((lane >> 4) & 1)) << 4);
-    // every tile costs each wave 3 loads (K: 2 row loads + the key scales, which all waves load
-    // into the same place; V^T: 2 row loads + a spare scale load), so a wait for "all but the
-    // next tile's loads" is vmcnt(3)
-    auto issue = [&](bool isk, int kt, int buf) {
-        const int k0 = kt * 32;
-        const uint32_t base = lds0 + (uint32_t)(buf * kI8Buf);
-        if (isk) {
+        for (int i = 0; i < 8; i++)
+            dma16(rK, base + i * 1024, (uint32_t)(k0 + 16 * (i & 1) + 4 * (i >> 1) + (lane >> 4)) * rowB +
+                  (uint32_t)(((lane & 15) ^ ((4 * i + (lane >> 4)) & 15)) << 4), 0u);
+        dma4(rKS, base + kI8Tile, (uint32_t)(k0 + lane) * a.KV * 4, 0u);
+    };
+    // V^T: load i fills rows d = 8 i + lane / 8 of the wave's 64, position lane % 8 holding keys
+    // 16 c .. + 15 of the block, c = (lane % 8) ^ (lane / 8)
+    auto issue_v = [&](int g, int buf) __attribute__((always_inline)) {
+        const uint32_t base = lds0 + (uint32_t)((2 * w + buf) * kI8Buf);
 #pragma unroll
-            for (int e = 0; e < 2; e++) {
-                const int i = 2 * wu + e;
-                dma16(rK, base + i * 1024, kvo[e], (uint32_t)(k0 + 16 * (i & 1) + 4 * (i >> 1)) * rowB);
-            }
-        } else {
-#pragma unroll
-            for (int e = 0; e < 2; e++) {
-                const int i = 2 * wu + e;
-                dma16(rV, base + i * 1024, vvo, (uint32_t)(32 * i) * vpitch + (uint32_t)(2 * row0 + k0));
-            }
-        }
-        dma4(rKS, base + kI8Tile, (uint32_t)lane * a.KV * 4, (uint32_t)k0 * a.KV * 4);
+        for (int i = 0; i < 8; i++)
+            dma16(rV, base + i * 1024, (uint32_t)(64 * w + 8 * i + (lane >> 3)) * vpitch +
+                  (uint32_t)(2 * row0 + 128 * g + (((lane & 7) ^ (lane >> 3)) << 4)), 0u);
     };
-    // the tile stream: pass 1's K tiles, then per 128-key block its K tiles and its V^T tiles
-    const int NS = 3 * ntiles;
-    auto desc = [&](int n, bool &isk, int &kt) {
-        if (n < ntiles) {
-            isk = true;
-            kt = n;
-            return;
-        }
-        const int m = n - ntiles, full = 8 * (nblk - 1);
-        if (m < full) {
-            isk = (m & 7) < 4;
-            kt = 4 * (m >> 3) + (m & 3);
-            return;
-        }
-        const int ntl = ntiles - 4 * (nblk - 1), j = m - full;
-        isk = j < ntl;
-        kt = 4 * (nblk - 1) + (isk ? j : j - ntl);
+    // the ring's stream: pass 1's K tiles, then KEEP ? V^T blocks : K tiles and V^T of each block in turn
+    auto issue = [&](int n) __attribute__((always_inline)) {
+        if (n < nblk) return issue_k(n, n & 1);
+        const int m = n - nblk;
+        if (KEEP ? m >= nblk : m >= 2 * nblk) return;
+        if (KEEP) issue_v(m, n & 1);
+        else if (m & 1) issue_v(m >> 1, n & 1);
+        else issue_k(m >> 1, n & 1);
     };
-    int sn = 0;  // stream position of the step being computed
-    // wait for step sn's tile (every wave's), release the buffer of step sn - 1 and refill it with
-    // step sn + 2's tile; returns step sn's buffer
-    auto begin_step = [&]() -> const unsigned char * {
-        if (sn + 1 < NS) asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (sn + 2 < NS) {
-            bool isk;
-            int kt;
-            desc(sn + 2, isk, kt);
-            issue(isk, kt, (sn + 2) % kI8Ring);
-        }
-        const unsigned char *sb = smem + (sn % kI8Ring) * kI8Buf;
-        ++sn;
-        return sb;
+    // every wave is past its reads of step n's buffer and its loads of step n + 1 have arrived; step n + 2's
+    // go into the buffer of step n
+    auto step_done = [&](int n) __attribute__((always_inline)) {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        issue(n + 2);
     };
-    // fragment offsets: K row rho = lane % 32, chunk 2 kk + half at position (2 kk + half) ^ (rho % 16);
-    // V^T row d = 32 dt + lane % 32, chunk half at position half ^ ((d / 8) % 2)
-    const int rho = lane & 31;
-    const int vrd = rho * 32 + ((half ^ ((rho >> 3) & 1)) << 4);
+    auto sync = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    unsigned char *const pq8 = smem + kI8S + kI8P;
+    float *ml = (float *)(smem + kI8S + kI8M), *pl = (float *)(smem + kI8S + kI8L);
 
     // one K tile: S^T (8 MFMAs, two 128-d blocks), folded like the reference's GEMM, keys past the
-    // sequence at -inf. s[r] is key 16 half + r of the tile.
-    auto scores = [&](const unsigned char *sb, int k0, float (&s)[16]) {
+    // sequence at -inf. s[r] is key 16 half + r of the tile (K row ql, chunk 2 kk + half).
+    auto scores = [&](const unsigned char *sb, int k0, float (&s)[16]) __attribute__((always_inline)) {
         v16i acc0 = (v16i){}, acc1 = (v16i){};
 #pragma unroll
         for (int kk = 0; kk < 8; kk++) {
-            const v4i kf = *(const v4i *)(sb + rho * 256 + (((2 * kk + half) ^ (rho & 15)) << 4));
+            const v4i kf = *(const v4i *)(sb + ql * 256 + (((2 * kk + half) ^ (ql & 15)) << 4));
             if (kk < 4) acc0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf, qf[kk], acc0, 0, 0, 0);
             else acc1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf, qf[kk], acc1, 0, 0, 0);
         }
@@ -283,124 +264,174 @@ __global__ __launch_bounds__(256, 1) void k_attn_i8(AttnI8Args a) {
         }
     };
 
-    for (int n = 0; n < 2 && n < NS; n++) {
-        bool isk;
-        int kt;
-        desc(n, isk, kt);
-        issue(isk, kt, n);
-    }
-    float mrun = -INFINITY, lrun = 0.f;
-    for (int kt = 0; kt < ntiles; kt++) {
-        const unsigned char *sb = begin_step();
-        float s[16];
-        scores(sb, kt * 32, s);
-        float mloc = -INFINITY;
+    issue(0);
+    issue(1);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    float keep[KEEP ? 4 : 1][16];
+    float mrun = -INFINITY, mfold = -INFINITY, lrun = 0.f, mt[4];
+    int nprev = 0;
+    // the partial sums of the group before (its tiles' maxima in mt), in tile order
+    auto fold = [&](int g) __attribute__((always_inline)) {
 #pragma unroll
-        for (int r = 0; r < 16; r++) mloc = fmaxf(mloc, s[r]);
-        mloc = fmaxf(mloc, xor_lane<32>(mloc));
-        const float mnew = fmaxf(mrun, mloc);
-        if (mnew > -INFINITY) {
+        for (int t = 0; t < 4; t++) {
+            if (t < nprev) {
+                const float mnew = fmaxf(mfold, mt[t]);
+                if (mnew > -INFINITY) {
+                    lrun = (mfold == -INFINITY ? 0.f : lrun * __expf(mfold - mnew)) + pl[(g & 1) * 256 + t * 64 + lane];
+                    mfold = mnew;
+                }
+            }
+        }
+    };
+    auto pass1 = [&](int g, float (&s)[16]) __attribute__((always_inline)) {
+        const int nt = min(4, ntiles - 4 * g);
+        float mloc = -INFINITY;
+        if (w < nt) {
+            scores(smem + (2 * w + (g & 1)) * kI8Buf, (4 * g + w) * 32, s);
+#pragma unroll
+            for (int r = 0; r < 16; r++) mloc = fmaxf(mloc, s[r]);
+            mloc = fmaxf(mloc, xor_lane<32>(mloc));
+            if (half == 0) ml[(g & 1) * 128 + w * 32 + ql] = mloc;
+        }
+        step_done(g);
+        fold(g - 1);
+        float mine = mrun;
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            if (t < nt) {
+                mt[t] = ml[(g & 1) * 128 + t * 32 + ql];
+                mrun = fmaxf(mrun, mt[t]);
+                if (t == w) mine = mrun;
+            }
+        }
+        nprev = nt;
+        if (w < nt) {
             float ps = 0.f;
 #pragma unroll
-            for (int r = 0; r < 16; r++) ps += s[r] == -INFINITY ? 0.f : __expf(s[r] - mnew);
-            lrun = (mrun == -INFINITY ? 0.f : lrun * __expf(mrun - mnew)) + ps;
-            mrun = mnew;
+            for (int r = 0; r < 16; r++) ps += s[r] == -INFINITY ? 0.f : __expf(s[r] - mine);
+            pl[(g & 1) * 256 + w * 64 + lane] = ps;
         }
+    };
+    if constexpr (KEEP) {
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+            if (g < nblk) pass1(g, keep[g]);
+    } else {
+        for (int g = 0; g < nblk; g++) pass1(g, keep[0]);
     }
+    sync();
+    fold(nblk - 1);
     const float ltot = lrun + xor_lane<32>(lrun);
     const float inv_l = ltot > 0.f ? __fdiv_rn(1.0f, ltot) : 0.f;
 
-    v16i acco[8];
-    float of[8][16];
+    float of[2][16];
 #pragma unroll
-    for (int dt = 0; dt < 8; dt++) {
-        acco[dt] = (v16i){};
+    for (int dt = 0; dt < 2; dt++)
 #pragma unroll
         for (int r = 0; r < 16; r++) of[dt][r] = 0.f;
-    }
-    for (int blk = 0; blk < nblk; blk++) {
-        const int nt = min(4, ntiles - 4 * blk);
-        float pv[4][16];
-        float am = 0.f;
+    auto pass2 = [&](int g, float (&s)[16]) __attribute__((always_inline)) {
+        const int nt = min(4, ntiles - 4 * g), nv = KEEP ? nblk + g : nblk + 2 * g + 1;  // this block's V^T step
+        float pv[16], am = 0.f;
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            if (t < nt) {
-                const unsigned char *sb = begin_step();
-                float s[16];
-                scores(sb, (4 * blk + t) * 32, s);
+        for (int r = 0; r < 16; r++) pv[r] = 0.f;
+        if (w < nt) {
+            if (!KEEP) scores(smem + (2 * w + ((nv - 1) & 1)) * kI8Buf, (4 * g + w) * 32, s);
 #pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    const float e = s[r] == -INFINITY ? 0.f : __expf(s[r] - mrun);
-                    pv[t][r] = __fmul_rn(e, inv_l);
-                    am = fmaxf(am, pv[t][r]);
-                }
-            } else {
-#pragma unroll
-                for (int r = 0; r < 16; r++) pv[t][r] = 0.f;
+            for (int r = 0; r < 16; r++) {
+                const float e = s[r] == -INFINITY ? 0.f : __expf(s[r] - mrun);
+                pv[r] = __fmul_rn(e, inv_l);
+                am = fmaxf(am, pv[r]);
             }
         }
         am = fmaxf(am, xor_lane<32>(am));
+        if (half == 0) ml[w * 32 + ql] = am;
+        if (KEEP && g == 0) sync();  // (step nblk - 1 was done in pass 1)
+        else step_done(nv - 1);
+#pragma unroll
+        for (int t = 0; t < 4; t++) am = fmaxf(am, ml[t * 32 + ql]);
         const QScale ps = qscale(am);
-        v4i pq[4];
+        v4i mine;
 #pragma unroll
-        for (int t = 0; t < 4; t++)
-#pragma unroll
-            for (int g = 0; g < 4; g++)
-                pq[t][g] = (int)pack4_magic(pv[t][4 * g], pv[t][4 * g + 1], pv[t][4 * g + 2], pv[t][4 * g + 3], ps.inv);
+        for (int q = 0; q < 4; q++)
+            mine[q] = (int)pack4_magic(pv[4 * q], pv[4 * q + 1], pv[4 * q + 2], pv[4 * q + 3], ps.inv);
+        *(v4i *)(pq8 + w * 1024 + lane * 16) = mine;
+        sync();
+        v16i acc[2] = {(v16i){}, (v16i){}};
+        const unsigned char *vb = smem + (2 * w + (nv & 1)) * kI8Buf;
 #pragma unroll
         for (int t = 0; t < 4; t++) {
             if (t < nt) {
-                const unsigned char *sb = begin_step();
+                const v4i pq = *(const v4i *)(pq8 + t * 1024 + lane * 16);
 #pragma unroll
-                for (int dt = 0; dt < 8; dt++) {
-                    const v4i vf = *(const v4i *)(sb + dt * 32 * 32 + vrd);
-                    acco[dt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf, pq[t], acco[dt], 0, 0, 0);
+                for (int dt = 0; dt < 2; dt++) {
+                    const v4i vf = *(const v4i *)(vb + (32 * dt + ql) * 128 + (((2 * t + half) ^ (ql & 7)) << 4));
+                    acc[dt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf, pq, acc[dt], 0, 0, 0);
                 }
             }
         }
-        // fold the block: d = 32 dt + 8 (r / 4) + 4 half + r % 4
+        // d = 64 w + 32 dt + 8 (r / 4) + 4 half + r % 4
 #pragma unroll
-        for (int dt = 0; dt < 8; dt++) {
+        for (int dt = 0; dt < 2; dt++)
 #pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const float4 v4 = *(const float4 *)(vs_l + 32 * dt + 8 * g + 4 * half);
+            for (int q = 0; q < 4; q++) {
+                const float4 v4 = *(const float4 *)(vs_l + 64 * w + 32 * dt + 8 * q + 4 * half);
                 const float vv[4] = {v4.x, v4.y, v4.z, v4.w};
 #pragma unroll
                 for (int e = 0; e < 4; e++)
-                    of[dt][4 * g + e] = __builtin_fmaf((float)acco[dt][4 * g + e], __fmul_rn(ps.sc, vv[e]), of[dt][4 * g + e]);
+                    of[dt][4 * q + e] = __builtin_fmaf((float)acc[dt][4 * q + e], __fmul_rn(ps.sc, vv[e]), of[dt][4 * q + e]);
             }
-            acco[dt] = (v16i){};
-        }
+        if (!KEEP) step_done(nv);
+    };
+    if constexpr (KEEP) {
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+            if (g < nblk) pass2(g, keep[g]);
+    } else {
+        for (int g = 0; g < nblk; g++) pass2(g, keep[0]);
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
+    // a 128-dim block is two waves'
+    float am = 0.f;
+#pragma unroll
+    for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) am = fmaxf(am, fabsf(of[dt][r]));
+    am = fmaxf(am, xor_lane<32>(am));
+    if (half == 0) ml[128 + w * 32 + ql] = am;
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    am = fmaxf(am, ml[128 + (w ^ 1) * 32 + ql]);
+    const QScale qs = qscale(am);
     if (qi >= Sk) return;  // rows past the sequence belong to the next one
     const size_t orow = row0 + qi;
 #pragma unroll
-    for (int blk = 0; blk < 2; blk++) {
-        float am = 0.f;
+    for (int dt = 0; dt < 2; dt++)
 #pragma unroll
-        for (int dt = 4 * blk; dt < 4 * blk + 4; dt++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) am = fmaxf(am, fabsf(of[dt][r]));
-        am = fmaxf(am, xor_lane<32>(am));
-        const QScale qs = qscale(am);
-#pragma unroll
-        for (int dt = 4 * blk; dt < 4 * blk + 4; dt++)
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const int d = 32 * dt + 8 * g + 4 * half;
-                *(uint32_t *)(a.cq + orow * HD + h * kI8D + d) =
-                    pack4_magic(of[dt][4 * g], of[dt][4 * g + 1], of[dt][4 * g + 2], of[dt][4 * g + 3], qs.inv);
-                if (a.c32)
-                    *(float4 *)(a.c32 + orow * HD + h * kI8D + d) =
-                        make_float4(of[dt][4 * g], of[dt][4 * g + 1], of[dt][4 * g + 2], of[dt][4 * g + 3]);
-            }
-        if (half == 0) a.cs[orow * (HD / kQBlock) + h * 2 + blk] = qs.sc;
-    }
+        for (int q = 0; q < 4; q++) {
+            const int d = 64 * w + 32 * dt + 8 * q + 4 * half;
+            *(uint32_t *)(a.cq + orow * HD + h * kI8D + d) =
+                pack4_magic(of[dt][4 * q], of[dt][4 * q + 1], of[dt][4 * q + 2], of[dt][4 * q + 3], qs.inv);
+            if (a.c32)
+                *(float4 *)(a.c32 + orow * HD + h * kI8D + d) =
+                    make_float4(of[dt][4 * q], of[dt][4 * q + 1], of[dt][4 * q + 2], of[dt][4 * q + 3]);
+        }
+    if (half == 0 && !(w & 1)) a.cs[orow * (HD / kQBlock) + h * 2 + (w >> 1)] = qs.sc;
 }
 
 static size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
+
+template <bool KEEP>
+static int launch_attn_i8(hipStream_t s, const AttnI8Args &a, int B, int max_len, int n_work) {
+    static bool attr = false;
+    if (!attr) {
+        if (check_hip(hipFuncSetAttribute((const void *)k_attn_i8<KEEP>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          kAttnI8Lds), "attention_i8 lds attribute"))
+            return -1;
+        attr = true;
+    }
+    const dim3 grid = a.work ? dim3((n_work + 7) / 8 * 32) : dim3((max_len + 31) / 32, a.H, B);
+    hipLaunchKernelGGL(k_attn_i8<KEEP>, grid, dim3(256), kAttnI8Lds, s, a, n_work);
+    return check_hip(hipGetLastError(), "attention_i8 launch");
+}
 
 struct I8Ws {
     size_t q8, qs, k8, ks, vt8, vpart, vs, total;
@@ -458,21 +489,11 @@ extern "C" int e2mi_attention_i8_packed(e2mi_stream stream, const float *q32, co
     unsigned char *ws = (unsigned char *)workspace;
     I8PrepArgs p = {q32, k32, v32, (int8_t *)(ws + wo.q8), (float *)(ws + wo.qs), (int8_t *)(ws + wo.k8),
                     (float *)(ws + wo.ks), (int8_t *)(ws + wo.vt8), (float *)(ws + wo.vpart),
-                    (float *)(ws + wo.vs), seq_start, seq_len, M, H, KV, (max_len + 63) / 64};
+                    (float *)(ws + wo.vs), seq_start, seq_len, M, H, KV, (max_len + 63) / 64, B * KV, B * KV * ((max_len + 63) / 64)};
     hipStream_t s = (hipStream_t)stream;
     const long items = (long)M * (H + KV);
-    hipLaunchKernelGGL(k_i8_qk_prep, dim3((unsigned)((items + 3) / 4)), dim3(256), 0, s, p);
-    hipLaunchKernelGGL(k_i8_vmax, dim3(B * KV, p.nch), dim3(256), 0, s, p);
+    hipLaunchKernelGGL(k_i8_prep, dim3((unsigned)(p.nv + (items + 3) / 4)), dim3(256), 0, s, p);
     hipLaunchKernelGGL(k_i8_vquant, dim3(B * KV, (max_len + 31) / 32), dim3(256), 0, s, p);
-    static bool attr = false;
-    if (!attr) {
-        if (check_hip(hipFuncSetAttribute((const void *)k_attn_i8, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                          kAttnI8Lds), "attention_i8 lds attribute"))
-            return -1;
-        attr = true;
-    }
-    AttnI8Args a = {p.q8, p.qs, p.k8, p.ks, p.vt8, p.vs, ctx_q, ctx_s, ctx32, seq_start, seq_len, work, M, H, KV};
-    const dim3 grid = work ? dim3(n_work) : dim3((max_len + 127) / 128, H, B);
-    hipLaunchKernelGGL(k_attn_i8, grid, dim3(256), kAttnI8Lds, s, a);
-    return check_hip(hipGetLastError(), "attention_i8 launch");
+    const AttnI8Args a = {p.q8, p.qs, p.k8, p.ks, p.vt8, p.vs, ctx_q, ctx_s, ctx32, seq_start, seq_len, work, M, H, KV};
+    return max_len <= kI8Keep ? launch_attn_i8<true>(s, a, B, max_len, n_work) : launch_attn_i8<false>(s, a, B, max_len, n_work);
 }

@@ -208,3 +208,21 @@ def test_engine_int8_attention_vs_oracle(gpu, rng):
     assert np.array_equal(f16, eng.embed_batch(ids, valid))  # switched back
     with pytest.raises(Exception):
         e2mi.Engine(e2mi.Model.synthetic(small_config(e2mi, n_layers=1), 1), max_rows=512).set_attention("f32")
+
+
+def test_attention_i8_kept_scores_match_recomputed(gpu, rng):
+    """Sequences of at most 512 keys at a max_len up to 512 (scores kept in registers) and above it
+    (computed twice): bit for bit, with and without a work list, at the edges of 32-key tiles and
+    128-key blocks."""
+    import torch
+    import e2mi
+    H, KV, lens = 4, 2, [512, 1, 31, 32, 33, 127, 128, 129, 257, 385, 511]
+    rowmap, pos, start, plen, M = _packed(rng, e2mi, lens, 512)
+    q, k, v = (_t(x, gpu) for x in _inputs(rng, M, H, KV))
+    sd, ld = _t(start, gpu), _t(plen, gpu)
+    work = _t(e2mi.attention_work(plen, H), gpu)
+    want = e2mi.attention_i8_packed(q, k, v, sd, ld, 512, H, KV)
+    for max_len, wk in ((512, work), (513, None), (513, work)):
+        got = e2mi.attention_i8_packed(q, k, v, sd, ld, max_len, H, KV, work=wk)
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
