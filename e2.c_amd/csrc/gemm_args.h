@@ -59,7 +59,7 @@ class NormInScope {
 // gemm_s.hip: the kernels for few rows, and which one (0: none) takes an M x N x K GEMM with the
 // epilogue `epi` (tok: per-token activation scales); launch_gemm_small runs it at the expected row
 // count and returns 1, or returns 0 for the caller's kernels and -1 on error
-enum { GEMM_SK = 1, GEMM_S32 = 2, GEMM_S64 = 3 };
+enum { GEMM_SK = 1, GEMM_S32 = 2, GEMM_S64 = 3, GEMM_RING = 5 };  // (4 is tile_signature's)
 int gemm_small_route(int M, int N, int K, int epi, bool tok);
 int launch_gemm_small(hipStream_t s, const GemmArgs &p, int epi, int est, bool tok);
 

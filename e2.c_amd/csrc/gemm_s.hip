@@ -552,12 +552,128 @@ __global__ __launch_bounds__(512, 1) void k_gemm_sk(const int *rows, GemmArgs p,
     }
 }
 
+// 64 x 128 output tiles between the tiles above and gemm.hip's: A and W stream through an LDS ring of
+// three 128-wide K blocks (24 KB each), loaded two ahead by all eight waves with one barrier a block, so no K
+// is too long and two workgroups share a CU. A wave computes 32 x 32 outputs (4 v_mfma_i32_32x32x32_i8 and 8
+// LDS reads a block; k_gemm_s's 64 x 16 read the whole A tile in every wave) and folds a block's products
+// while the next block's fragments arrive. What bounds it is that chain, 0.5 us a block for one workgroup a
+// CU (gemm.hip's 128 x 128 tiles with one wave a SIMD: 1.05). 3072 -> 768, 2520 rows: 31.3 -> 19.1 us
+// (620 TOP/s); 2048 -> 512, 4096 rows: 22.9 -> 15.0. A ring of six blocks, one workgroup a CU, measured
+// 19.7 and 15.5, and 33.9 against 26.4 at 3072 -> 768, 4096 rows.
+constexpr int kRing = 3;  // K blocks
+template <int FOLD>
+__global__ __launch_bounds__(512, 4) void k_gemm_ring(const int *rows, GemmArgs p, int tiles_m, int tiles) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int t = xcd_tile(blockIdx.x, tiles);
+    if (t < 0) return;
+    const int m0 = (t % tiles_m) * 64, n0 = (t / tiles_m) * 128;
+    const int tid = threadIdx.x, lane = tid & 63, hh = lane >> 5, c = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave & 1, wn = wave >> 1;
+    const int nb = p.K / kQBlock;
+    const v4u rA = rsrc_words(p.A, (uint32_t)((size_t)p.M * p.lda));
+    const v4u rW = rsrc_words(p.W, (uint32_t)((size_t)p.N * p.ldw));
+    const v4u rS = rsrc_words(p.as, (uint32_t)((size_t)p.M * nb * 4));
+    const v4u rV = rsrc_words(p.ws, (uint32_t)((size_t)p.N * 4));
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const lds_void *)smem);
+    constexpr int R = kRing;
+    constexpr uint32_t kSlot = 24 * 1024, oS = R * kSlot;  // slot: A 8 KB, W 16 KB; then the scales
+    const uint32_t oV = oS + (uint32_t)nb * 256u;
+    if (rows && m0 >= *rows) return;  // planned on the device: no row here
+    for (int b = wave; b < nb; b += 8)
+        dma4(rS, lds0 + oS + (uint32_t)b * 256u, (uint32_t)(m0 + lane) * (uint32_t)nb * 4u, (uint32_t)b * 4u);
+    if (wave < 2) dma4(rV, lds0 + oV + wave * 256u, (uint32_t)(n0 + wave * 64 + lane) * 4u, 0);
+    // load j of a tile fills its rows 8 j .. + 7; every wave loads one of A's and two of W's a block
+    const uint32_t lr = (uint32_t)lane >> 3, x = (uint32_t)(lane & 7);
+    const uint32_t chA = (x ^ (((wave & 1) << 2) + (lane >> 4))) << 4, ch0 = (x ^ (lane >> 4)) << 4, ch1 = (x ^ (4 + (lane >> 4))) << 4;
+    const uint32_t vA = (uint32_t)(m0 + 8 * wave + lr) * (uint32_t)p.lda + chA;
+    const uint32_t vW0 = (uint32_t)(n0 + 16 * wave + lr) * (uint32_t)p.ldw + ch0;
+    const uint32_t vW1 = (uint32_t)(n0 + 16 * wave + 8 + lr) * (uint32_t)p.ldw + ch1;
+    auto issue = [&](int b) {
+        const uint32_t st = lds0 + (uint32_t)(b % R) * kSlot, ko = (uint32_t)b * kQBlock;
+        dma16(rA, st + wave * 1024u, vA, ko);
+        dma16(rW, st + 8192u + wave * 2048u, vW0, ko);
+        dma16(rW, st + 8192u + wave * 2048u + 1024u, vW1, ko);
+    };
+    for (int b = 0; b < min(nb, R - 1); b++) issue(b);
+    // this wave's part of every block but the last n has landed and its own fragment reads are done; past
+    // the barrier that holds for every wave
+    auto sync = [&](int n) {
+        if (n >= 1) asm volatile("s_waitcnt vmcnt(3) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    };
+    static_assert(R == 3, "sync leaves one block in flight");
+    uint32_t fo[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) fo[k] = (uint32_t)swz(c, 2 * k + hh);
+    float f[16], ws = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) f[i] = 0.f;
+    v4i af[4], wf[4];
+    auto fetch = [&](int b) {  // block b's fragments; its ring predecessor's slot takes block b + R - 1
+        sync(min(nb - 1, b + R - 2) - b);
+        if (b + R - 1 < nb) issue(b + R - 1);
+        const unsigned char *st = smem + (uint32_t)(b % R) * kSlot;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            af[k] = *(const v4i *)(st + wm * 4096 + fo[k]);
+            wf[k] = *(const v4i *)(st + 8192 + wn * 4096 + fo[k]);
+        }
+    };
+    auto mul = [&](v16i &acc) {
+        acc = (v16i){};
+#pragma unroll
+        for (int k = 0; k < 4; k++) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[k], wf[k], acc, 0, 0, 0);
+    };
+    auto fold = [&](int b, const v16i &acc) {
+        const float *sb = (const float *)(smem + oS + b * 256) + wm * 32 + 4 * hh;
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const float4 a4 = ld4(sb + 8 * g);
+            const float av[4] = {a4.x, a4.y, a4.z, a4.w};
+#pragma unroll
+            for (int i = 0; i < 4; i++)  // the reference's order (FOLD_FAST: ws once, below)
+                f[4 * g + i] = __builtin_fmaf((float)acc[4 * g + i], FOLD == FOLD_FAST ? av[i] : __fmul_rn(av[i], ws), f[4 * g + i]);
+        }
+    };
+    v16i acc0, acc1;
+    fetch(0);
+    ws = *(const float *)(smem + oV + (wn * 32 + c) * 4);
+    mul(acc0);
+    int b = 1;
+    for (; b + 1 < nb; b += 2) {
+        fetch(b);
+        fold(b - 1, acc0);
+        mul(acc1);
+        fetch(b + 1);
+        fold(b, acc1);
+        mul(acc0);
+    }
+    if (b < nb) {
+        fetch(b);
+        fold(b - 1, acc0);
+        mul(acc0);
+    }
+    fold(nb - 1, acc0);
+    const int n = n0 + wn * 32 + c;
+    const bool post = p.bias != nullptr || p.lo > -1e30f || p.hi < 1e30f;
+    const float bias = p.bias ? p.bias[min(n, p.N - 1)] : 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const int m = m0 + wm * 32 + 8 * (i >> 2) + 4 * hh + (i & 3);
+        float v = f[i];
+        if constexpr (FOLD == FOLD_FAST) v = __fmul_rn(v, ws);
+        if (post) v = fminf(fmaxf(v + bias, p.lo), p.hi);
+        if (m < p.M && n < p.N) p.Y[(size_t)m * p.ldy + n] = v;
+    }
+}
+
 template <class K>
 int set_lds(K kern) {
     return check_hip(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024),
                      "gemm lds attribute");
 }
 
+int ring_lds(int nb) { return kRing * 24 * 1024 + nb * 256 + 512; }
 int grid_of(int tiles) { return (tiles + 7) / 8 * 8; }
 
 template <int EPI, int NW, int RU, int CU, int FOLD, int NC = 0>
@@ -590,6 +706,19 @@ int launch_sk(hipStream_t s, const GemmArgs &p) {
     }
     const int tm = (p.M + 31) / 32, tiles = tm * ((p.N + 31) / 32);
     hipLaunchKernelGGL(kern, dim3(grid_of(tiles)), dim3(512), p.K / kQBlock * 8448, s, p.rows, p, tm, tiles);
+    return check_hip(hipGetLastError(), "gemm launch");
+}
+
+template <int FOLD>
+int launch_ring(hipStream_t s, const GemmArgs &p) {
+    auto kern = k_gemm_ring<FOLD>;
+    static bool attr = false;
+    if (!attr) {
+        if (set_lds(kern)) return -1;
+        attr = true;
+    }
+    const int tiles = ((p.M + 63) / 64) * ((p.N + 127) / 128);
+    hipLaunchKernelGGL(kern, dim3(grid_of(tiles)), dim3(512), ring_lds(p.K / kQBlock), s, p.rows, p, (p.M + 63) / 64, tiles);
     return check_hip(hipGetLastError(), "gemm launch");
 }
 
@@ -634,13 +763,17 @@ NormInScope::~NormInScope() { t_norm = NormIn{}; }
 // 16.0 at 2048; q|k|v 768 -> 1280: 7.7 | 11.7 | 16.5 at 32, 9.6 | 13.0 | 17.5 at 1024, 17.2 | 15.1 | 19.3
 // at 3008, 24.4 | 26.0 | 19.6 at 4096.
 //
-// 128-column tiles and the K-split 32 x 32 tiles: the least of four fitted times. A K-split tile keeps
+// 128-column tiles and the K-split 32 x 32 tiles: the least of five fitted times. A K-split tile keeps
 // 8.25 KB of LDS a block, so up to 9 blocks two or more of them share a CU. 768 -> 768, K-split | 32 |
 // 64 | gemm.hip: 3.4 | 5.3 | 6.3 | 9.8 at 32 rows, 6.1 | 6.7 | 8.6 | 10.8 at 1024, 11.7 | 16.1 | 16.3 |
 // 12.0 at 3008, 15.2 | 17.2 | 17.0 | 12.6 at 4096; 2048 -> 512: 5.1 | 9.3 | - | 20.0 at 32, 18.8 | 12.4 |
 // - | 21.5 at 2048, 27.0 | 20.6 | - | 22.0 at 3008; 512 -> 512 with the PLE gate's epilogue: 4.7 | 6.1 |
 // 10.9 at 32 rows (32 | 64 | gemm.hip), 6.2 | 7.4 | 12.4 at 2048, 10.3 | 8.8 | 12.9 at 4096; per token
 // 768 -> 1152: 3.4 | 5.1 | 5.7 | 8.0 at 32, 7.9 | 9.7 | 8.0 | 9.0 at 1024, 11.1 | 14.1 | 14.2 | 9.0 at 2048.
+// The ring up to two workgroups a CU, ring | the best of the others: 768 -> 768 8.0 | 5.7 at 1024 rows, 9.3 |
+// 9.7 at 2048, 9.7 | 10.7 at 2520, 12.6 | 12.8 at 4096; 1152 -> 768 9.7 | 8.5, 10.7 | 12.1, 11.1 | 13.0, 14.8 |
+// 16.1; 2048 -> 512 12.9 | 10.4, 13.6 | 12.7, 13.7 | 21.8, 15.0 | 22.9, 21.6 | 25.7 at 8192; 3072 -> 768 16.6 |
+// 29.0 at 256, 26.4 | 32.6 at 4096, then 41.6 | 42.4 at 8192, 97.9 | 88.5 at 17408 (three and seven rounds).
 int gemm_small_route(int M, int N, int K, int epi, bool tok) {
     const int C = num_cus(), nb = K / kQBlock;
     auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
@@ -650,8 +783,8 @@ int gemm_small_route(int M, int N, int K, int epi, bool tok) {
         return 0;
     }
     auto rounds = [&](long t) { return (double)((t + C - 1) / C); };
-    const double fill = (double)tiles(128, 128) / C;
-    double best = tok ? 5.0 + 0.6 * nb : 4.2 + 1.05 * nb + (epi == EPI_GELUMUL ? 2.5 : 0.0) + (fill > 0.5 ? 4.0 * (fill - 0.5) : 0.0);
+    const double fill = (double)tiles(128, 128) / C, fr = (double)tiles(64, 128) / C;
+    double best = tok ? 5.0 + 0.6 * nb : (epi == EPI_F32 ? 5.3 : 4.2) + 1.05 * nb + (epi == EPI_GELUMUL ? 2.5 : 0.0) + (fill > 0.5 ? 4.0 * (fill - 0.5) : 0.0);
     int route = 0;
     auto offer = [&](bool ok, double t, int r) {
         if (ok && t < best) {
@@ -662,6 +795,8 @@ int gemm_small_route(int M, int N, int K, int epi, bool tok) {
     offer(epi == EPI_F32 && nb * 8448 <= kLds, 3.0 + (nb <= 9 ? 0.69e-3 : 1.0e-3) * nb * (double)tiles(32, 32) * 256 / C, GEMM_SK);
     offer(Small<8, 2, 1>::lds(nb) <= kLds, 1.2 + rounds(tiles(32, 128)) * (2.2 + 0.5 * nb), GEMM_S32);
     offer(Small<8, 4, 1>::lds(nb) <= kLds, 1.2 + rounds(tiles(64, 128)) * (3.4 + 0.85 * nb), GEMM_S64);
+    offer(epi == EPI_F32 && !tok && fr <= (ring_lds(nb) <= kLds / 2 ? 2.0 : 1.0),
+          fr <= 1.0 ? 4.2 + 0.52 * nb + 2.4 * fr : 6.4 + 0.77 * nb + fr, GEMM_RING);
     return route;
 }
 
@@ -672,7 +807,9 @@ int launch_gemm_small(hipStream_t s, const GemmArgs &p, int epi, int est, bool t
     const int route = gemm_small_route(est, p.N, p.K, epi, tok);
     if (!route) return 0;
     int rc;
-    if (route == GEMM_SK) {
+    if (route == GEMM_RING) {
+        rc = gemm_fold_fast() ? launch_ring<FOLD_FAST>(s, p) : launch_ring<FOLD_EXACT>(s, p);
+    } else if (route == GEMM_SK) {
         rc = tok ? launch_sk<FOLD_TOK>(s, p) : gemm_fold_fast() ? launch_sk<FOLD_FAST>(s, p) : launch_sk<FOLD_EXACT>(s, p);
     } else {
         const bool s64 = route == GEMM_S64;

@@ -150,3 +150,35 @@ def test_small_add_norm(gpu, rng, K, N, scale):
     want = f(qa[:8], qa2[:8].contiguous(), W, r, ga, gn, x_out=r)
     got = f(qa[:8], qa2[:8].contiguous(), W, res[:8], ga, gn)
     _same(got[2:4], want[2:4], "NaN row")
+
+
+# k_gemm_ring (64 x 128 tiles): odd and even block counts, rows at its tiles' edges
+# and at one and two workgroups a CU, an N inside a tile, bias, clamp, column range and both folds; the large call of
+# each shape is gemm.hip's
+@pytest.mark.parametrize("K,N,rows", [(3072, 256, (1, 63, 64, 65, 300)), (2944, 520, (257, 1000)), (3072, 768, (2520, 2731, 4096)),
+                                      (2048, 512, (2520, 4096, 8192)), (1152, 768, (2048, 2730, 2731)),
+                                      (896, 768, (2500, 2520))])
+def test_ring_f32(gpu, oracle, rng, K, N, rows):
+    import e2mi
+    import torch
+    qa, as_, w, ws, b, W = _ops(rng, gpu, K, N, True)
+    for mode in ("exact", "fast"):
+        prev = e2mi.set_gemm_fold(mode)
+        try:
+            W.set_clamp(-3e38, 3e38)
+            full = e2mi.i8_gemm(qa, as_, W)
+            for M in rows:
+                y = torch.full((M + 1, N), 7.0, device=gpu)
+                e2mi.i8_gemm(qa[:M], as_[:M], W, y=y)
+                _same([y[:M]], [full[:M]], f"{mode} M={M}")
+                assert bool((y[M] == 7.0).all()), f"{mode} M={M}: a row past the count was written"
+            if mode == "exact":
+                want = oracle.i8_gemm(qa[:65].cpu().numpy(), as_[:65].cpu().numpy(), w, ws, bias=b)
+                assert np.array_equal(full[:65].cpu().numpy().view(np.uint32), want.view(np.uint32))
+            W.set_clamp(-1.5, 2.0)
+            full = e2mi.i8_gemm(qa, as_, W, n0=33, n1=N - 19)
+            for M in rows:
+                y = e2mi.i8_gemm(qa[:M], as_[:M], W, n0=33, n1=N - 19)
+                _same([y], [full[:M]], f"{mode} M={M}, clamped columns")
+        finally:
+            e2mi.set_gemm_fold(prev)
