@@ -199,11 +199,11 @@ bool gemm_half_tiles(int M, int N);
 int gemm_an_units(int rows);
 bool gemm_an_fits(int rows);
 // gemm_an.hip: the projection and its norm_add (e2mi_i8_gemm_add_norm_quant, scale: _scale_quant) in one
-// launch or, through tmp, in two, and whether two are faster at a row count
+// launch or, through tmp and where that is faster, in two, and whether two are
 int launch_gemm_add_norm(hipStream_t s, const int8_t *qa, const float *a_scales, const e2mi_q8w *w, int M,
                          const float *res, const float *gamma_add, float post_scale, const float *gamma_next,
                          float eps, float *x_out, float *xn_out, int8_t *q, float *qs, bool scale, float *tmp);
-bool gemm_an_split(int rows, int D);
+bool gemm_an_split(int rows, int K);
 
 template <class T>
 static int dalloc(e2mi_engine *g, T **p, size_t count) {
@@ -364,17 +364,17 @@ constexpr int kAttnPartTiles = 8, kMaxAttnParts = 4;
 // two launches), fused (the norm_add in the projection's epilogue, one workgroup holding whole rows), or, at few rows,
 // ahead: the projection in many small tiles to memory and the norm_add in the workgroups of the GEMM
 // that reads it (NormIn). Fused needs one round of the CUs to cover the rows: past that each
-// workgroup's weight fetch costs more than the f32 round trip. Up to gemm_an_split rows two launches
-// beat the fused one, and up to 256 rows ahead is as good as two or better. One sequence, us per call,
+// workgroup's weight fetch costs more than the f32 round trip; a fused projection runs as two launches
+// through tmp where those are faster (gemm_an_split), and up to 256 rows ahead is as good as two or
+// better. One sequence, us per call,
 // ahead | separate | fused: reference geometry 1282 | 1317 | 1628 at 19 tokens, 1470 | 1488 | 1895 at
 // 100, 1899 | 1852 | 2216 at 300; BASELINE geometry 1003 | 1007 | 1226, 1122 | 1120 | 1366, 1455 | 1334 |
 // 1510.
-enum NormForm { NORM_SEPARATE, NORM_FUSED, NORM_TWO, NORM_AHEAD };
+enum NormForm { NORM_SEPARATE, NORM_FUSED, NORM_AHEAD };
 static NormForm norm_form(const e2mi_engine *g, int rows) {
     const e2_config &c = g->cfg;
     if (!g->fuse_an || (c.hidden != 768 && c.hidden != 512) || !gemm_an_fits(rows)) return NORM_SEPARATE;
-    if (rows <= 256) return NORM_AHEAD;
-    return gemm_an_split(rows, c.hidden) ? NORM_TWO : NORM_FUSED;
+    return rows <= 256 ? NORM_AHEAD : NORM_FUSED;
 }
 
 // every kernel of one forward over B sequences of S tokens (M rows: B * S padded, or the packed
@@ -386,9 +386,9 @@ static int enqueue(e2mi_engine *g, int B, int S, int Mp, bool pk, hipStream_t s,
     const e2_config &c = g->cfg;
     const int M = pk ? Mp : B * S, Dm = c.hidden, H = c.n_heads, P = c.ple_dim;
     const NormForm form = norm_form(g, dev && est > 0 ? est : M);
-    const bool an = form == NORM_FUSED || form == NORM_TWO;
-    float *an_tmp = form == NORM_TWO ? g->tmp : nullptr;
-    const int an_extra = form == NORM_TWO ? 1 : 0;
+    const bool an = form == NORM_FUSED;
+    // launches of a projection with its norm_add past the first
+    auto an_extra = [&](const e2mi_q8w &w) { return gemm_an_split(dev && est > 0 ? est : M, w.K) ? 1 : 0; };
     // form ahead: x moves between two buffers, each norm_add reading one and writing the other
     float *x = g->x, *x_other = g->xn;
     if (M <= 0 || M > g->R) {
@@ -489,8 +489,8 @@ static int enqueue(e2mi_engine *g, int B, int S, int Mp, bool pk, hipStream_t s,
             ahead(L.ln_attn, 1.0f, L.ln_pre);
         } else if (L.o_an && an) {
             RUN("o_proj+add_norm", launch_gemm_add_norm(s, g->cq, g->cs, &L.o, M, g->x, L.ln_attn, 1.0f, L.ln_pre, eps,
-                                                        g->x, nullptr, g->qa, g->as, false, an_tmp));
-            k += an_extra;
+                                                        g->x, nullptr, g->qa, g->as, false, g->tmp));
+            k += an_extra(L.o);
         } else {
             RUN("o_proj", e2mi_i8_gemm(s, g->tmp, Dm, g->cq, g->cs, &L.o, M, 0, Dm));
             RUN("add_norm", e2mi_add_norm_quant(s, g->tmp, g->x, L.ln_attn, L.ln_pre, eps, M, Dm, g->x, nullptr,
@@ -526,20 +526,20 @@ static int enqueue(e2mi_engine *g, int B, int S, int Mp, bool pk, hipStream_t s,
             // post_ffn norm_add in the down projection, x itself quantized for the PLE gate; the PLE
             // block, its norm_add and the layer scale in the PLE projection
             RUN("down+add_norm", launch_gemm_add_norm(s, g->qg, g->gs, &L.down, M, g->x, L.ln_ffn, 1.0f, nullptr, eps,
-                                                      g->x, nullptr, g->qa, g->as, true, an_tmp));
+                                                      g->x, nullptr, g->qa, g->as, true, g->tmp));
             RUN("ple_gate", e2mi_i8_gemm_gelu_mul(s, g->qg, g->gs, nullptr, g->qa, g->as, &L.ple_gate, M,
                                                   g->ple32 + (size_t)l * P, c.n_layers * P));
             RUN("ple_proj+add_norm", launch_gemm_add_norm(s, g->qg, g->gs, &L.ple_proj, M, g->x, L.ple_norm,
                                                           L.layer_scalar, gnext, eps, g->x, last ? g->xn : nullptr,
-                                                          g->qa, g->as, true, an_tmp));
-            k += 2 * an_extra;
+                                                          g->qa, g->as, true, g->tmp));
+            k += an_extra(L.down) + an_extra(L.ple_proj);
             continue;
         }
         if (L.down_an && an) {
             RUN("down+add_norm", launch_gemm_add_norm(s, g->qg, g->gs, &L.down, M, g->x, L.ln_ffn, 1.0f, gnext, eps, g->x,
                                                       last ? g->xn : nullptr, !last || c.out_dim > 0 ? g->qa : nullptr,
-                                                      !last || c.out_dim > 0 ? g->as : nullptr, false, an_tmp));
-            k += an_extra;
+                                                      !last || c.out_dim > 0 ? g->as : nullptr, false, g->tmp));
+            k += an_extra(L.down);
             continue;
         }
         RUN("down", e2mi_i8_gemm(s, g->tmp, Dm, g->qg, g->gs, &L.down, M, 0, Dm));
@@ -705,33 +705,41 @@ static int plan_pack(e2mi_engine *g, const uint8_t *valid, int n, int S) {
 
 // The kernels of a device-planned forward of about `est` rows: for every distinct GEMM of the forward
 // whose kernel follows the row count, which one takes it (gemm_small_route, gemm_half_tiles), and
-// how the projections run their norm_add (fused: in how many row units per workgroup, 1-5)
+// how the projections run their norm_add (fused: in how many row units per workgroup, 1-5, and how many
+// of them in two launches, those of larger K first)
 static long tile_signature(const e2mi_engine *g, int est) {
     const e2_config &c = g->cfg;
     const NormForm form = norm_form(g, est);
-    const bool an = form == NORM_FUSED;  // (the other forms run the projections as plain GEMMs)
+    // whether a projection runs as a GEMM of its own, and how many fused ones run in two launches
+    int split = 0;
+    auto alone = [&](const e2mi_q8w &w, bool with_an) {
+        if (!with_an || form != NORM_FUSED) return true;
+        const bool two = gemm_an_split(est, w.K);
+        split += two;
+        return two;
+    };
     std::vector<std::tuple<int, int, int>> gemms;  // N, K, epilogue
     auto add = [&](const e2mi_q8w &w, int epi) { gemms.emplace_back(w.N, w.K, epi); };
     for (const LayerDev &L : g->layers) {
         add(L.qkv, L.qkv_fused ? EPI_QKV : EPI_F32);
         add(L.gu, EPI_GEGLU);
-        if (!(L.o_an && an)) add(L.o, EPI_F32);
-        if (!(L.down_an && an)) add(L.down, EPI_F32);
+        if (alone(L.o, L.o_an)) add(L.o, EPI_F32);
+        if (alone(L.down, L.down_an)) add(L.down, EPI_F32);
         if (c.ple_dim > 0) {
             add(L.ple_gate, EPI_GELUMUL);
-            if (!(L.down_an && an)) add(L.ple_proj, EPI_F32);
+            if (alone(L.ple_proj, L.down_an)) add(L.ple_proj, EPI_F32);
         }
     }
     if (c.ple_dim > 0) add(g->ple_model, EPI_F32);
     if (c.out_dim > 0) add(g->embed_proj, EPI_F32);
     std::sort(gemms.begin(), gemms.end());
     gemms.erase(std::unique(gemms.begin(), gemms.end()), gemms.end());
-    long sig = an ? gemm_an_units(est) : form == NORM_AHEAD ? 6 : form == NORM_TWO ? 7 : 0;
+    long sig = form == NORM_FUSED ? gemm_an_units(est) : form == NORM_AHEAD ? 6 : 7;
     for (const auto &[N, K, epi] : gemms) {  // at most 14 of them, 3 bits each
         const int small = gemm_small_route(est, N, K, epi, false);
         sig = sig << 3 | (small ? small : gemm_half_tiles(est, N) ? 4 : 0);
     }
-    return sig;
+    return sig << 8 | std::min(split, 255);
 }
 
 // The device entry plans on the device (plan_dev.hip) when the whole batch is one chunk whatever its

@@ -377,13 +377,15 @@ static int launch_an(hipStream_t s, const int *rows, const AnArgs &a, int grid, 
     }
 }
 
-// Whether the projection and its norm_add run as two launches (gemm_s.hip's GEMM, then the row kernel)
-// at a row count: below about a million outputs a workgroup of k_gemm_an reads the whole weight for
-// its 16 rows (0.6-1 MB at the 64 B a clock a CU loads: 5-8 us) while most CUs have none. 768 columns,
-// two launches | one: K = 768 7.1 | 12.5 us at 32 rows, 10.7 | 13.1 at 1024, 15.4 | 13.9 at 2048;
-// K = 1152 7.5 | 15.5, 12.8 | 16.4, 18.4 | 18.2; 512 columns: K = 1024 6.8 | 11.5, 9.9 | 13.2, 13.2 |
-// 13.9; K = 2048 7.8 | 18.2, 14.2 | 21.0, 17.4 | 21.5.
-bool gemm_an_split(int rows, int D) { return (long)rows * D <= 1 << 20; }
+// Whether the projection and its norm_add run as two launches (gemm_s.hip's GEMM, then the row kernel) at a
+// row count: a workgroup of k_gemm_an reads the whole weight for its 16 rows in one serial chain whose
+// length is K, while the two launches pay for 8 more bytes an output, so the line moves with K: up to K
+// rows, and past K = 1152, where k_gemm_ring halves the GEMM's own chain, faster. Two launches | one, us:
+// 768 columns, K = 768 7.6 | 11.5 at 256 rows, 12.6 | 12.9 at 1024, 15.1 | 13.3 at 1360; K = 1152 14.8 | 16.4
+// at 1024, 17.5 | 16.5 at 1360; 512 columns, K = 512 6.6 | 7.5 at 256, 9.0 | 7.9 at 1024, 12.6 | 8.9 at 2048;
+// K = 1024 11.1 | 12.8 at 1024, 13.1 | 13.2 at 1360, 14.9 | 13.7 at 2048; K = 2048 15.1 | 20.8 at 1024,
+// 19.3 | 21.3 at 2048, 21.4 | 22.3 at 3400, 28.2 | 25.3 at 5000.
+bool gemm_an_split(int rows, int K) { return rows <= K + std::max(0, K - 1152); }
 
 bool gemm_fold_fast();
 // rowops.hip: the row kernel with k_gemm_an's byte packing
@@ -432,7 +434,7 @@ static int gemm_add_norm(hipStream_t s, const int8_t *qa, const float *a_scales,
     a.gamma_n = gamma_next; a.x_out = x_out; a.xn_out = xn_out; a.q = q; a.qs = qs; a.y = y;
     a.lda = w->K; a.ldw = w->ld; a.M = M; a.K = w->K; a.eps = eps; a.post_scale = post_scale;
     const int est = dr.ptr && dr.est > 0 && dr.est < M ? dr.est : M;
-    if (engine ? tmp != nullptr : gemm_an_split(est, D)) {
+    if (gemm_an_split(est, w->K) && (!engine || tmp)) {
         // the projection goes through the engine's scratch, y, or x_out beside the residual, which the row
         // kernel then overwrites row by row
         const size_t n = (size_t)M * D;
@@ -453,7 +455,7 @@ static int gemm_add_norm(hipStream_t s, const int8_t *qa, const float *a_scales,
     return fast ? launch_an<768, false, true>(s, dr.ptr, a, grid, uc) : launch_an<768, false, false>(s, dr.ptr, a, grid, uc);
 }
 
-// the engine's: two launches through tmp (M x D floats), or one without it
+// the engine's: two launches, where they are faster, through tmp (M x D floats); one without it
 int launch_gemm_add_norm(hipStream_t s, const int8_t *qa, const float *a_scales, const e2mi_q8w *w, int M,
                          const float *res, const float *gamma_add, float post_scale, const float *gamma_next,
                          float eps, float *x_out, float *xn_out, int8_t *q, float *qs, bool scale, float *tmp) {
