@@ -553,8 +553,9 @@ __global__ __launch_bounds__(512, 1) void k_gemm_sk(const int *rows, GemmArgs p,
 }
 
 // 64 x 128 output tiles between the tiles above and gemm.hip's: A and W stream through an LDS ring of
-// three 128-wide K blocks (24 KB each), loaded two ahead by all eight waves with one barrier a block, so no K
-// is too long and two workgroups share a CU. A wave computes 32 x 32 outputs (4 v_mfma_i32_32x32x32_i8 and 8
+// three 128-wide K blocks (24 KB each), loaded two ahead by all eight waves with one barrier a block, so
+// two workgroups share a CU up to 30 blocks and one holds up to 350 (the activation scales of the whole K
+// stay in LDS, 256 bytes a block). A wave computes 32 x 32 outputs (4 v_mfma_i32_32x32x32_i8 and 8
 // LDS reads a block; k_gemm_s's 64 x 16 read the whole A tile in every wave) and folds a block's products
 // while the next block's fragments arrive. What bounds it is that chain, 0.5 us a block for one workgroup a
 // CU (gemm.hip's 128 x 128 tiles with one wave a SIMD: 1.05). 3072 -> 768, 2520 rows: 31.3 -> 19.1 us
@@ -795,7 +796,7 @@ int gemm_small_route(int M, int N, int K, int epi, bool tok) {
     offer(epi == EPI_F32 && nb * 8448 <= kLds, 3.0 + (nb <= 9 ? 0.69e-3 : 1.0e-3) * nb * (double)tiles(32, 32) * 256 / C, GEMM_SK);
     offer(Small<8, 2, 1>::lds(nb) <= kLds, 1.2 + rounds(tiles(32, 128)) * (2.2 + 0.5 * nb), GEMM_S32);
     offer(Small<8, 4, 1>::lds(nb) <= kLds, 1.2 + rounds(tiles(64, 128)) * (3.4 + 0.85 * nb), GEMM_S64);
-    offer(epi == EPI_F32 && !tok && fr <= (ring_lds(nb) <= kLds / 2 ? 2.0 : 1.0),
+    offer(epi == EPI_F32 && !tok && ring_lds(nb) <= kLds && fr <= (ring_lds(nb) <= kLds / 2 ? 2.0 : 1.0),
           fr <= 1.0 ? 4.2 + 0.52 * nb + 2.4 * fr : 6.4 + 0.77 * nb + fr, GEMM_RING);
     return route;
 }

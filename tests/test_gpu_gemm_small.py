@@ -182,3 +182,15 @@ def test_ring_f32(gpu, oracle, rng, K, N, rows):
                 _same([y], [full[:M]], f"{mode} M={M}, clamped columns")
         finally:
             e2mi.set_gemm_fold(prev)
+
+
+@pytest.mark.parametrize("K", [44800, 44928])  # the last K whose scales fit k_gemm_ring's LDS, and the next
+def test_long_k(gpu, oracle, rng, K):
+    import e2mi
+    M, N = 67, 72
+    qa = rng.integers(-127, 128, (M, K), dtype=np.int8)
+    as_ = rng.uniform(0.001, 0.05, (M, K // 128)).astype(np.float32)
+    w = rng.integers(-127, 128, (N, K), dtype=np.int8)
+    ws = rng.uniform(0.001, 0.02, N).astype(np.float32)
+    y = e2mi.i8_gemm(_t(qa, gpu), _t(as_, gpu), e2mi.DeviceWeight.from_rowmajor(w, ws))
+    assert np.array_equal(y.cpu().numpy().view(np.uint32), oracle.i8_gemm(qa, as_, w, ws).view(np.uint32))
