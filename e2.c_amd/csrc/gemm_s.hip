@@ -771,6 +771,9 @@ NormInScope::~NormInScope() { t_norm = NormIn{}; }
 // - | 21.5 at 2048, 27.0 | 20.6 | - | 22.0 at 3008; 512 -> 512 with the PLE gate's epilogue: 4.7 | 6.1 |
 // 10.9 at 32 rows (32 | 64 | gemm.hip), 6.2 | 7.4 | 12.4 at 2048, 10.3 | 8.8 | 12.9 at 4096; per token
 // 768 -> 1152: 3.4 | 5.1 | 5.7 | 8.0 at 32, 7.9 | 9.7 | 8.0 | 9.0 at 1024, 11.1 | 14.1 | 14.2 | 9.0 at 2048.
+// With eight K-split tiles a CU the large tiles have caught up whatever K is (K-split | gemm.hip: 128 -> 768
+// 7.2 | 6.6 at 3000 rows, 25.3 | 14.3 at 17408; 128 -> 4608 18.9 | 12.0 at 2048; 256 -> 1024 14.4 | 10.7 at
+// 6000; 384 -> 40 53.3 | 34.5 at 262144).
 // The ring up to two workgroups a CU, ring | the best of the others: 768 -> 768 8.0 | 5.7 at 1024 rows, 9.3 |
 // 9.7 at 2048, 9.7 | 10.7 at 2520, 12.6 | 12.8 at 4096; 1152 -> 768 9.7 | 8.5, 10.7 | 12.1, 11.1 | 13.0, 14.8 |
 // 16.1; 2048 -> 512 12.9 | 10.4, 13.6 | 12.7, 13.7 | 21.8, 15.0 | 22.9, 21.6 | 25.7 at 8192; 3072 -> 768 16.6 |
@@ -793,7 +796,9 @@ int gemm_small_route(int M, int N, int K, int epi, bool tok) {
             route = r;
         }
     };
-    offer(epi == EPI_F32 && nb * 8448 <= kLds, 3.0 + (nb <= 9 ? 0.69e-3 : 1.0e-3) * nb * (double)tiles(32, 32) * 256 / C, GEMM_SK);
+    // (per-128 scales: a K-split tile of one to four blocks costs its loads and its exchange more than its blocks)
+    const double sk = tok ? (nb <= 9 ? 0.69 : 1.0) * nb : std::max((nb <= 9 ? 0.69 : 1.1) * nb, 1.5 + 0.3 * nb);
+    offer(epi == EPI_F32 && nb * 8448 <= kLds && (tok || tiles(32, 32) <= 8L * C), 3.0 + 1e-3 * sk * (double)tiles(32, 32) * 256 / C, GEMM_SK);
     offer(Small<8, 2, 1>::lds(nb) <= kLds, 1.2 + rounds(tiles(32, 128)) * (2.2 + 0.5 * nb), GEMM_S32);
     offer(Small<8, 4, 1>::lds(nb) <= kLds, 1.2 + rounds(tiles(64, 128)) * (3.4 + 0.85 * nb), GEMM_S64);
     offer(epi == EPI_F32 && !tok && ring_lds(nb) <= kLds && fr <= (ring_lds(nb) <= kLds / 2 ? 2.0 : 1.0),

@@ -42,3 +42,12 @@ def test_a_route_fits_the_lds(route, epi, tok):
 def test_ring_ends_where_its_scales_fill_the_lds(route):
     assert route(64, 768, 44800) == RING  # 350 blocks: all of the 163,840 bytes
     assert route(64, 768, 44928) == NONE
+
+
+# shapes at which the K-split tiles take longer than the large ones (short K over many rows), and calls
+# of the same widths at which they are the fastest
+@pytest.mark.parametrize("M,N,K", [(17408, 768, 128), (65536, 256, 128), (2000, 4608, 128), (262144, 40, 128),
+                                   (5000, 1024, 256), (262144, 40, 384), (65536, 40, 512)])
+def test_short_k_over_many_rows_takes_the_large_tiles(route, M, N, K):
+    assert route(M, N, K) == NONE
+    assert route(32, N, K) == SK
