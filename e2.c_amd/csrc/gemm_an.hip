@@ -435,11 +435,20 @@ static int gemm_add_norm(hipStream_t s, const int8_t *qa, const float *a_scales,
     a.lda = w->K; a.ldw = w->ld; a.M = M; a.K = w->K; a.eps = eps; a.post_scale = post_scale;
     const int est = dr.ptr && dr.est > 0 && dr.est < M ? dr.est : M;
     if (gemm_an_split(est, w->K) && (!engine || tmp)) {
-        // the projection goes through the engine's scratch, y, or x_out beside the residual, which the row
-        // kernel then overwrites row by row
-        const size_t n = (size_t)M * D;
-        auto apart = [&](const float *t) { return t && (t + n <= res || res + n <= t); };
-        float *t = tmp ? tmp : apart(y) ? y : apart(x_out) ? x_out : nullptr;
+        // the projection goes through the engine's scratch, through y where one is asked for, or through x_out,
+        // which the row kernel then overwrites row by row; y and x_out only beside the inputs, which the
+        // GEMM's and the row kernel's workgroups still read while others write them (k_gemm_an's read a row's
+        // before they write it)
+        const size_t n = (size_t)M * D * 4;
+        auto beside = [&](const float *t, const void *in, size_t bytes) {
+            const uintptr_t a0 = (uintptr_t)t, b0 = (uintptr_t)in;
+            return a0 + n <= b0 || b0 + bytes <= a0;
+        };
+        auto apart = [&](const float *t) {
+            return t && beside(t, res, n) && beside(t, qa, (size_t)M * w->K) &&
+                   beside(t, a_scales, (size_t)M * (w->K / kQBlock) * 4);
+        };
+        float *own = y ? y : x_out, *t = tmp ? tmp : apart(own) ? own : nullptr;
         if (t)
             return e2mi_i8_gemm(s, t, D, qa, a_scales, w, M, 0, D) ||
                            launch_add_norm(s, t, res, gamma_add, post_scale, gamma_next, eps, M, D, x_out, xn_out, q, qs, scale)

@@ -108,6 +108,45 @@ def test_fused_scaled_equals_two_launches(gpu, rng, M, K, gamma_next):
     _both(gpu, rng, 300, K, N=512, gamma_next=gamma_next, post_scale=0.2, inplace=True)
 
 
+def _raw(gpu, case, **over):
+    """The entry point on buffers of the caller's choice: the outputs that were asked for, by name."""
+    import torch
+    import e2mi
+    qa, as_, w, ws, res, ga, gn = case
+    M, K, N = *qa.shape, w.shape[0]
+    W = over.pop("W", None) or e2mi.DeviceWeight.from_rowmajor(w, ws)
+    b = dict(qa=_t(qa, gpu), as_=_t(as_, gpu), res=_t(res, gpu), x=torch.empty((M, N), device=gpu), y=None,
+             q=torch.empty((M, N), dtype=torch.int8, device=gpu), qs=torch.empty((M, N // 128), device=gpu))
+    for k, v in over.items():
+        b[k] = v(b)
+    p = lambda t: None if t is None else t.data_ptr()
+    tga, tgn = _t(ga, gpu), _t(gn, gpu)
+    e2mi.check(e2mi.load().e2mi_i8_gemm_add_norm_quant(
+        torch.cuda.current_stream().cuda_stream, p(b["qa"]), p(b["as_"]), W.ref, M, p(b["res"]), p(tga), p(tgn),
+        EPS, p(b["x"]), None, p(b["q"]), p(b["qs"]), p(b["y"])))
+    torch.cuda.synchronize()
+    return b
+
+
+@pytest.mark.parametrize("M", [7, 333])
+def test_fused_over_its_inputs(gpu, rng, M):
+    """Outputs on the inputs' own memory at row counts that take two launches: y in the residual's place
+    (with x apart from it) is still the projection, and a call whose x lies in the activations' memory
+    (one workgroup's rows) is still computed from them."""
+    import torch
+    case = _case(rng, M, 768)
+    want = _raw(gpu, case, y=lambda b: torch.empty_like(b["res"]))
+    got = _raw(gpu, case, y=lambda b: b["res"])
+    for k in ("x", "y", "q", "qs"):
+        _same(got[k], want[k], f"y over res: {k}")
+    if M <= 16:
+        got = _raw(gpu, case, qa=lambda b: torch.cat([b["qa"].view(-1), torch.zeros(3 * M * D, dtype=torch.int8,
+                                                                                   device=gpu)]).view(4 * M, D),
+                   x=lambda b: b["qa"].view(torch.float32).view(M, D))
+        for k in ("x", "q", "qs"):
+            _same(got[k], want[k], f"x over qa: {k}")
+
+
 def test_fused_fast_fold(gpu, rng):
     import e2mi
     prev = e2mi.load().e2mi_gemm_set_fold(1)
