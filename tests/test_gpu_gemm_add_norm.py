@@ -147,6 +147,28 @@ def test_fused_over_its_inputs(gpu, rng, M):
             _same(got[k], want[k], f"x over qa: {k}")
 
 
+@pytest.mark.parametrize("M", [7, 333, 2100])
+def test_fused_weight_on_4_bytes(gpu, rng, M):
+    """k_gemm_an loads 16 bytes from any 4-byte address; the GEMM of the two launches asks for 16-byte
+    ones, so such a weight (a caller's own e2mi_q8w) keeps the one launch at every row count."""
+    import ctypes as C
+    import torch
+    import e2mi
+    case = _case(rng, M, 768)
+    want = _raw(gpu, case)
+    w, ws = case[2], case[3]
+    buf = torch.zeros(w.size + 16, dtype=torch.int8, device=gpu)
+    buf[4:4 + w.size] = _t(w, gpu).view(-1)
+    tws = _t(ws, gpu)
+
+    class Own:
+        q = e2mi.Q8W(w=buf.data_ptr() + 4, scale=tws.data_ptr(), N=D, K=768, ld=768, out_min=-1e31, out_max=1e31)
+        ref = C.byref(q)
+    got = _raw(gpu, case, W=Own)
+    for k in ("x", "q", "qs"):
+        _same(got[k], want[k], k)
+
+
 def test_fused_fast_fold(gpu, rng):
     import e2mi
     prev = e2mi.load().e2mi_gemm_set_fold(1)
