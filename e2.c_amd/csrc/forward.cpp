@@ -203,7 +203,7 @@ bool gemm_an_fits(int rows);
 int launch_gemm_add_norm(hipStream_t s, const int8_t *qa, const float *a_scales, const e2mi_q8w *w, int M,
                          const float *res, const float *gamma_add, float post_scale, const float *gamma_next,
                          float eps, float *x_out, float *xn_out, int8_t *q, float *qs, bool scale, float *tmp);
-bool gemm_an_split(int rows, int K);
+bool gemm_an_split(int rows, int N, int K);
 
 template <class T>
 static int dalloc(e2mi_engine *g, T **p, size_t count) {
@@ -388,7 +388,7 @@ static int enqueue(e2mi_engine *g, int B, int S, int Mp, bool pk, hipStream_t s,
     const NormForm form = norm_form(g, dev && est > 0 ? est : M);
     const bool an = form == NORM_FUSED;
     // launches of a projection with its norm_add past the first
-    auto an_extra = [&](const e2mi_q8w &w) { return gemm_an_split(dev && est > 0 ? est : M, w.K) ? 1 : 0; };
+    auto an_extra = [&](const e2mi_q8w &w) { return gemm_an_split(dev && est > 0 ? est : M, w.N, w.K) ? 1 : 0; };
     // form ahead: x moves between two buffers, each norm_add reading one and writing the other
     float *x = g->x, *x_other = g->xn;
     if (M <= 0 || M > g->R) {
@@ -714,7 +714,7 @@ static long tile_signature(const e2mi_engine *g, int est) {
     int split = 0;
     auto alone = [&](const e2mi_q8w &w, bool with_an) {
         if (!with_an || form != NORM_FUSED) return true;
-        const bool two = gemm_an_split(est, w.K);
+        const bool two = gemm_an_split(est, w.N, w.K);
         split += two;
         return two;
     };

@@ -380,12 +380,19 @@ static int launch_an(hipStream_t s, const int *rows, const AnArgs &a, int grid, 
 // Whether the projection and its norm_add run as two launches (gemm_s.hip's GEMM, then the row kernel) at a
 // row count: a workgroup of k_gemm_an reads the whole weight for its 16 rows in one serial chain whose
 // length is K, while the two launches pay for 8 more bytes an output, so the line moves with K: up to K
-// rows, and past K = 1152, where k_gemm_ring halves the GEMM's own chain, faster. Two launches | one, us:
-// 768 columns, K = 768 7.6 | 11.5 at 256 rows, 12.6 | 12.9 at 1024, 15.1 | 13.3 at 1360; K = 1152 14.8 | 16.4
-// at 1024, 17.5 | 16.5 at 1360; 512 columns, K = 512 6.6 | 7.5 at 256, 9.0 | 7.9 at 1024, 12.6 | 8.9 at 2048;
-// K = 1024 11.1 | 12.8 at 1024, 13.1 | 13.2 at 1360, 14.9 | 13.7 at 2048; K = 2048 15.1 | 20.8 at 1024,
-// 19.3 | 21.3 at 2048, 21.4 | 22.3 at 3400, 28.2 | 25.3 at 5000.
-bool gemm_an_split(int rows, int K) { return rows <= K + std::max(0, K - 1152); }
+// rows, and past K = 1152, where k_gemm_ring halves the GEMM's own chain, faster, up to the rows that one
+// workgroup of the small tiles a CU covers. A chain of one block (at 512 columns three) is no longer than
+// the second launch. Two launches | one, us: 768 columns, K = 128 6.4 | 5.4 at 1 row, 7.0 | 7.2 at 64, K = 256
+// 7.2 | 8.0 at 100, K = 768 7.6 | 11.5 at 256, 12.6 | 12.9 at 1024, 15.1 | 13.3 at 1360; K = 1152 14.8 | 16.4
+// at 1024, 17.5 | 16.5 at 1360; K = 3840 44.1 | 49.8 at 5000, 60.3 | 51.4 at 6000; 512 columns, K = 256
+// 6.6 | 6.3 at 100, K = 512 6.6 | 7.5 at 256, 9.0 | 7.9 at 1024, 12.6 | 8.9 at 2048; K = 1024 11.1 | 12.8 at
+// 1024, 13.1 | 13.2 at 1360, 14.9 | 13.7 at 2048; K = 2048 15.1 | 20.8 at 1024, 19.3 | 21.3 at 2048, 21.4 | 22.3 at
+// 3400, 28.2 | 25.3 at 5000; K = 4096 30.2 | 40.6 at 4096, 47.1 | 41.5 at 5000; K = 8192 45.9 | 76.5 at 4096, 79.2 |
+// 72.8 at 5000. Measured on 256 CUs; on a part of a chip the rows go with its CUs, as both grids do.
+bool gemm_an_split(int rows, int N, int K) {
+    if (K < (N == 512 ? 512 : 256)) return false;
+    return (long)rows * 256 <= (long)num_cus() * std::min(K + std::max(0, K - 1152), N == 512 ? 4096 : 5120);
+}
 
 bool gemm_fold_fast();
 // rowops.hip: the row kernel with k_gemm_an's byte packing
@@ -435,7 +442,7 @@ static int gemm_add_norm(hipStream_t s, const int8_t *qa, const float *a_scales,
     a.lda = w->K; a.ldw = w->ld; a.M = M; a.K = w->K; a.eps = eps; a.post_scale = post_scale;
     const int est = dr.ptr && dr.est > 0 && dr.est < M ? dr.est : M;
     // (the GEMM asks for a weight on 16 bytes; k_gemm_an's loads take any 4-byte address)
-    if (gemm_an_split(est, w->K) && (!engine || tmp) && aligned16(w->w)) {
+    if (gemm_an_split(est, D, w->K) && (!engine || tmp) && aligned16(w->w)) {
         // the projection goes through the engine's scratch, through y where one is asked for, or through x_out,
         // which the row kernel then overwrites row by row; y and x_out only beside the inputs, which the
         // GEMM's and the row kernel's workgroups still read while others write them (k_gemm_an's read a row's

@@ -1,5 +1,6 @@
-"""Which GEMM kernel a call takes (gemm_small_route, gemm_s.hip; a host function, so no GPU is needed): a
-kernel is offered only where its LDS holds the K of the call."""
+"""Which GEMM kernel a call takes (gemm_small_route, gemm_s.hip) and whether a projection and its norm_add
+run as two launches (gemm_an_split, gemm_an.hip): host functions, so no GPU is needed. A kernel is offered only
+where its LDS holds the K of the call, and no form where it was measured slower than another."""
 import ctypes as C
 
 import pytest
@@ -15,6 +16,15 @@ def route():
     f = e2mi.load()._ZN4e2mi16gemm_small_routeEiiiib
     f.argtypes, f.restype = [C.c_int] * 4 + [C.c_bool], C.c_int
     return lambda M, N, K, epi=F32, tok=False: f(M, N, K, epi, tok)
+
+
+@pytest.fixture(scope="module")
+def split():
+    """Whether a projection of N columns and its norm_add run as two launches (gemm_an.hip)."""
+    import e2mi
+    f = e2mi.load()._ZN4e2mi13gemm_an_splitEiii
+    f.argtypes, f.restype = [C.c_int] * 3, C.c_bool
+    return f
 
 
 def _lds(r, epi, nb):
@@ -51,3 +61,14 @@ def test_ring_ends_where_its_scales_fill_the_lds(route):
 def test_short_k_over_many_rows_takes_the_large_tiles(route, M, N, K):
     assert route(M, N, K) == NONE
     assert route(32, N, K) == SK
+
+
+# both sides of the line, 512 and 768 columns, and the ends of K
+@pytest.mark.parametrize("N,K,two,one", [(768, 768, (1, 768), (769, 17408)), (768, 1152, (1, 1152), (1153,)),
+                                         (512, 512, (33, 512), (513,)), (512, 2048, (1, 2944), (2945, 17408)),
+                                         (512, 4096, (1, 4096), (4200, 5000, 7000)), (512, 8192, (4096,), (5000,)),
+                                         (768, 3840, (5000,), (6000,)), (768, 256, (100,), (257,)),
+                                         (768, 128, (), (1, 64, 128)), (512, 256, (), (1, 100, 256))])
+def test_two_launches_only_where_they_are_faster(split, N, K, two, one):
+    assert all(split(r, N, K) for r in two)
+    assert not any(split(r, N, K) for r in one)
