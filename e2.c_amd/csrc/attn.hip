@@ -1123,11 +1123,15 @@ __global__ __launch_bounds__(256) void k_attn_merge(AttnArgs a, const int32_t *m
 // 1024-2048 89.0 | 108.7 | 175.4; head_dim 512, 1 x 300 36.5 | 21.6 | 19.6 [40], 1 x 2048 158.8 | 95.3 | 87.0 [256],
 // 2 x 700-1500 122.9 | 73.7 | 115.4 [340], 4 x 1024-2048 166.2 | 185.8 | 289.9. At head_dim 256 a sequence of one
 // or two key tiles gains nothing (19 tokens: 7.1 | 7.8 | 7.4).
-static int attn_group_blocks(int rows, int B, int max_len, int H, int D) {
+// Without a work list the grid has every block of max_len for every sequence, and neighbouring query blocks
+// lie on neighbouring XCDs, so the first ones' XCDs get all the short sequences: there the whole grid is counted
+// (3 heads without a list, 128 | 64 us: 12 x 64-512 24.9 | 28.4, 16 x 64-512 23.6 | 31.0; 8 x 64-512 21.7 | 18.4).
+int attn_group_blocks(int rows, int B, int max_len, int H, int D, bool list) {
     if (D == 256 && max_len <= 64) return 0;
     const double C = num_cus();
-    if (H * (rows / 32.0 + B / 2.0) <= 0.8 * C) return 1;
-    return H * (rows / 64.0 + B / 2.0) <= C ? 2 : 0;
+    auto blocks = [&](int q) { return list ? H * ((double)rows / q + B / 2.0) : (double)H * B * ((max_len + q - 1) / q); };
+    if (blocks(32) <= 0.8 * C) return 1;
+    return blocks(64) <= C ? 2 : 0;
 }
 
 template <int D, bool WIN, int QS>
@@ -1226,7 +1230,7 @@ static int attention_packed(const char *who, e2mi_stream stream, const uint16_t 
     const dim3 grid = work ? dim3(n_work) : dim3((max_len + 127) / 128, H, B);
     const DeviceRows dr = device_rows();
     const int rows = dr.ptr && dr.est > 0 ? std::min(dr.est, M) : M;
-    const int qs = merge ? 0 : attn_group_blocks(rows, B, max_len, H, D);
+    const int qs = merge ? 0 : attn_group_blocks(rows, B, max_len, H, D, work != nullptr);
     if (direct && qs) {
         const hipStream_t st = (hipStream_t)stream;
         if (D == 512)
