@@ -23,6 +23,8 @@
 //                  O^T += V^T P^T on int8 MFMA with int32 accumulators folded into f32 once per
 //                  block. S^T = K Q^T as in attn.hip: K tile rows are permuted so a lane's 16
 //                  logits are 16 consecutive keys of its query, exactly its P^T operand bytes.
+#include <algorithm>
+
 #include "common.h"
 
 namespace e2mi {
@@ -161,260 +163,265 @@ constexpr int kI8P = 0, kI8M = 4096, kI8L = kI8M + 1024, kI8X = kI8L + 2048;  //
 constexpr int kI8V = 8 * kI8Buf, kI8S = kI8V + kI8D * 4, kAttnI8Lds = kI8S + kI8X;
 
 template <bool KEEP>
-__global__ __launch_bounds__(256, 2) void k_attn_i8(AttnI8Args a, int n_work) {
+__global__ __launch_bounds__(256, 2) void k_attn_i8(AttnI8Args a, int n_work, int nwg) {
     extern __shared__ __align__(16) unsigned char smem[];
-    int q0 = blockIdx.x * 32, h = blockIdx.y, b = blockIdx.z;
-    if (a.work) {  // work entry i's four blocks on one XCD (i % 8)
-        const int i = (blockIdx.x >> 5) * 8 + (blockIdx.x & 7);
+    int q0 = blockIdx.x * 32, q1 = q0 + 32, h = blockIdx.y, b = blockIdx.z;
+    if (a.work) {  // work entry i's blocks on one XCD (i % 8), dealt to nwg workgroups
+        const int i = (blockIdx.x / (8 * nwg)) * 8 + (blockIdx.x & 7);
         const int item = i < n_work ? a.work[i] : -1;
         if (item < 0) return;
         b = item & 0xffff;
         h = (item >> 16) & 0xf;  // (one part: work_entry(b, h, 0, 1, query block))
-        q0 = (item >> 24) * 128 + ((blockIdx.x >> 3) & 3) * 32;
+        q1 = (item >> 24) * 128 + 128;
+        q0 = q1 - 128 + ((blockIdx.x >> 3) % nwg) * 32;
     }
-    const int Sk = a.seq_len[b];
-    if (q0 >= Sk) return;
-    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, ql = lane & 31;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int HD = a.H * kI8D, kvh = h / (a.H / a.KV);
-    const size_t row0 = (size_t)a.seq_start[b];
-    const int qi = q0 + ql, qc = min(qi, Sk - 1);  // this lane's query
-    // Q^T operand (B of S^T = K Q^T): the query's d = 32 kk + 16 half .. + 16
-    v4i qf[8];
-    {
-        const int8_t *qp = a.q8 + (row0 + qc) * HD + h * kI8D + 16 * half;
+    for (; q0 < min(a.seq_len[b], q1); q0 += 32 * nwg) {
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid), "+s"(b));  // (nothing of a block is kept in registers for the next)
+        const int Sk = a.seq_len[b];
+        const int lane = tid & 63, half = lane >> 5, ql = lane & 31;
+        const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const int HD = a.H * kI8D, kvh = h / (a.H / a.KV);
+        const size_t row0 = (size_t)a.seq_start[b];
+        const int qi = q0 + ql, qc = min(qi, Sk - 1);  // this lane's query
+        // Q^T operand (B of S^T = K Q^T): the query's d = 32 kk + 16 half .. + 16
+        v4i qf[8];
+        {
+            const int8_t *qp = a.q8 + (row0 + qc) * HD + h * kI8D + 16 * half;
 #pragma unroll
-        for (int kk = 0; kk < 8; kk++) qf[kk] = *(const v4i *)(qp + 32 * kk);
-    }
-    const float qs0 = a.qs[(row0 + qc) * a.H * 2 + h * 2], qs1 = a.qs[(row0 + qc) * a.H * 2 + h * 2 + 1];
-    float *vs_l = (float *)(smem + kI8V);
-    vs_l[tid] = a.vs[((size_t)b * a.KV + kvh) * kI8D + tid];
-    // the loads above complete here, under a wait the compiler sees: otherwise its wait would sit
-    // inside a loop and also cover the tile loads in flight
-    __builtin_amdgcn_s_waitcnt(0x0F70);
+            for (int kk = 0; kk < 8; kk++) qf[kk] = *(const v4i *)(qp + 32 * kk);
+        }
+        const float qs0 = a.qs[(row0 + qc) * a.H * 2 + h * 2], qs1 = a.qs[(row0 + qc) * a.H * 2 + h * 2 + 1];
+        float *vs_l = (float *)(smem + kI8V);
+        vs_l[tid] = a.vs[((size_t)b * a.KV + kvh) * kI8D + tid];
+        // the loads above complete here, under a wait the compiler sees: otherwise its wait would sit
+        // inside a loop and also cover the tile loads in flight
+        __builtin_amdgcn_s_waitcnt(0x0F70);
 
-    const int ntiles = (Sk + 31) / 32, nblk = (ntiles + 3) / 4;
-    const uint32_t rowB = (uint32_t)a.KV * kI8D, vpitch = 2u * (uint32_t)a.M;
-    const v4u rK = rsrc_words(a.k8 + row0 * rowB + kvh * kI8D, (uint32_t)Sk * rowB);
-    const v4u rKS = rsrc_words(a.ks + row0 * a.KV + kvh, (uint32_t)Sk * a.KV * 4);
-    const v4u rV = rsrc_words(a.vt8 + (size_t)kvh * kI8D * 2 * a.M, (uint32_t)((size_t)kI8D * 2 * a.M));
-    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const lds_void *)smem);
-    // K: load i fills physical rows rho = 4 i + lane / 16, 16-byte position lane % 16 holding chunk
-    // (lane % 16) ^ (rho % 16), of key 16 ((rho / 4) % 2) + 4 (rho / 8) + rho % 4 = 16 (i % 2) + 4 (i / 2) + lane / 16;
-    // keys past the sequence are out of the buffer's range and read as 0
-    auto issue_k = [&](int g, int buf) __attribute__((always_inline)) {
-        const int k0 = (4 * g + w) * 32;
-        const uint32_t base = lds0 + (uint32_t)((2 * w + buf) * kI8Buf);
+        const int ntiles = (Sk + 31) / 32, nblk = (ntiles + 3) / 4;
+        const uint32_t rowB = (uint32_t)a.KV * kI8D, vpitch = 2u * (uint32_t)a.M;
+        const v4u rK = rsrc_words(a.k8 + row0 * rowB + kvh * kI8D, (uint32_t)Sk * rowB);
+        const v4u rKS = rsrc_words(a.ks + row0 * a.KV + kvh, (uint32_t)Sk * a.KV * 4);
+        const v4u rV = rsrc_words(a.vt8 + (size_t)kvh * kI8D * 2 * a.M, (uint32_t)((size_t)kI8D * 2 * a.M));
+        const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const lds_void *)smem);
+        // K: load i fills physical rows rho = 4 i + lane / 16, 16-byte position lane % 16 holding chunk
+        // (lane % 16) ^ (rho % 16), of key 16 ((rho / 4) % 2) + 4 (rho / 8) + rho % 4 = 16 (i % 2) + 4 (i / 2) + lane / 16;
+        // keys past the sequence are out of the buffer's range and read as 0
+        auto issue_k = [&](int g, int buf) __attribute__((always_inline)) {
+            const int k0 = (4 * g + w) * 32;
+            const uint32_t base = lds0 + (uint32_t)((2 * w + buf) * kI8Buf);
 #pragma unroll
-        for (int i = 0; i < 8; i++)
-            dma16(rK, base + i * 1024, (uint32_t)(k0 + 16 * (i & 1) + 4 * (i >> 1) + (lane >> 4)) * rowB +
-                  (uint32_t)(((lane & 15) ^ ((4 * i + (lane >> 4)) & 15)) << 4), 0u);
-        dma4(rKS, base + kI8Tile, (uint32_t)(k0 + lane) * a.KV * 4, 0u);
-    };
-    // V^T: load i fills rows d = 8 i + lane / 8 of the wave's 64, position lane % 8 holding keys
-    // 16 c .. + 15 of the block, c = (lane % 8) ^ (lane / 8)
-    auto issue_v = [&](int g, int buf) __attribute__((always_inline)) {
-        const uint32_t base = lds0 + (uint32_t)((2 * w + buf) * kI8Buf);
+            for (int i = 0; i < 8; i++)
+                dma16(rK, base + i * 1024, (uint32_t)(k0 + 16 * (i & 1) + 4 * (i >> 1) + (lane >> 4)) * rowB +
+                      (uint32_t)(((lane & 15) ^ ((4 * i + (lane >> 4)) & 15)) << 4), 0u);
+            dma4(rKS, base + kI8Tile, (uint32_t)(k0 + lane) * a.KV * 4, 0u);
+        };
+        // V^T: load i fills rows d = 8 i + lane / 8 of the wave's 64, position lane % 8 holding keys
+        // 16 c .. + 15 of the block, c = (lane % 8) ^ (lane / 8)
+        auto issue_v = [&](int g, int buf) __attribute__((always_inline)) {
+            const uint32_t base = lds0 + (uint32_t)((2 * w + buf) * kI8Buf);
 #pragma unroll
-        for (int i = 0; i < 8; i++)
-            dma16(rV, base + i * 1024, (uint32_t)(64 * w + 8 * i + (lane >> 3)) * vpitch +
-                  (uint32_t)(2 * row0 + 128 * g + (((lane & 7) ^ (lane >> 3)) << 4)), 0u);
-    };
-    // the ring's stream: pass 1's K tiles, then KEEP ? V^T blocks : K tiles and V^T of each block in turn
-    auto issue = [&](int n) __attribute__((always_inline)) {
-        if (n < nblk) return issue_k(n, n & 1);
-        const int m = n - nblk;
-        if (KEEP ? m >= nblk : m >= 2 * nblk) return;
-        if (KEEP) issue_v(m, n & 1);
-        else if (m & 1) issue_v(m >> 1, n & 1);
-        else issue_k(m >> 1, n & 1);
-    };
-    // every wave is past its reads of step n's buffer and its loads of step n + 1 have arrived; step n + 2's
-    // go into the buffer of step n
-    auto step_done = [&](int n) __attribute__((always_inline)) {
+            for (int i = 0; i < 8; i++)
+                dma16(rV, base + i * 1024, (uint32_t)(64 * w + 8 * i + (lane >> 3)) * vpitch +
+                      (uint32_t)(2 * row0 + 128 * g + (((lane & 7) ^ (lane >> 3)) << 4)), 0u);
+        };
+        // the ring's stream: pass 1's K tiles, then KEEP ? V^T blocks : K tiles and V^T of each block in turn
+        auto issue = [&](int n) __attribute__((always_inline)) {
+            if (n < nblk) return issue_k(n, n & 1);
+            const int m = n - nblk;
+            if (KEEP ? m >= nblk : m >= 2 * nblk) return;
+            if (KEEP) issue_v(m, n & 1);
+            else if (m & 1) issue_v(m >> 1, n & 1);
+            else issue_k(m >> 1, n & 1);
+        };
+        // every wave is past its reads of step n's buffer and its loads of step n + 1 have arrived; step n + 2's
+        // go into the buffer of step n
+        auto step_done = [&](int n) __attribute__((always_inline)) {
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            issue(n + 2);
+        };
+        auto sync = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+        unsigned char *const pq8 = smem + kI8S + kI8P;
+        float *ml = (float *)(smem + kI8S + kI8M), *pl = (float *)(smem + kI8S + kI8L);
+
+        // one K tile: S^T (8 MFMAs, two 128-d blocks), folded like the reference's GEMM, keys past the
+        // sequence at -inf. s[r] is key 16 half + r of the tile (K row ql, chunk 2 kk + half).
+        auto scores = [&](const unsigned char *sb, int k0, float (&s)[16]) __attribute__((always_inline)) {
+            v16i acc0 = (v16i){}, acc1 = (v16i){};
+#pragma unroll
+            for (int kk = 0; kk < 8; kk++) {
+                const v4i kf = *(const v4i *)(sb + ql * 256 + (((2 * kk + half) ^ (ql & 15)) << 4));
+                if (kk < 4) acc0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf, qf[kk], acc0, 0, 0, 0);
+                else acc1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf, qf[kk], acc1, 0, 0, 0);
+            }
+            const float *ksl = (const float *)(sb + kI8Tile) + 16 * half;
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const float4 k4 = *(const float4 *)(ksl + 4 * g);
+                const float kv4[4] = {k4.x, k4.y, k4.z, k4.w};
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int r = 4 * g + e;
+                    const float f = __builtin_fmaf((float)acc0[r], __fmul_rn(qs0, kv4[e]), 0.f);
+                    const float x = __builtin_fmaf((float)acc1[r], __fmul_rn(qs1, kv4[e]), f);
+                    s[r] = (k0 + 16 * half + r < Sk) ? x : -INFINITY;
+                }
+            }
+        };
+
+        issue(0);
+        issue(1);
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        issue(n + 2);
-    };
-    auto sync = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-    unsigned char *const pq8 = smem + kI8S + kI8P;
-    float *ml = (float *)(smem + kI8S + kI8M), *pl = (float *)(smem + kI8S + kI8L);
-
-    // one K tile: S^T (8 MFMAs, two 128-d blocks), folded like the reference's GEMM, keys past the
-    // sequence at -inf. s[r] is key 16 half + r of the tile (K row ql, chunk 2 kk + half).
-    auto scores = [&](const unsigned char *sb, int k0, float (&s)[16]) __attribute__((always_inline)) {
-        v16i acc0 = (v16i){}, acc1 = (v16i){};
+        float keep[KEEP ? 4 : 1][16];
+        float mrun = -INFINITY, mfold = -INFINITY, lrun = 0.f, mt[4];
+        int nprev = 0;
+        // the partial sums of the group before (its tiles' maxima in mt), in tile order
+        auto fold = [&](int g) __attribute__((always_inline)) {
 #pragma unroll
-        for (int kk = 0; kk < 8; kk++) {
-            const v4i kf = *(const v4i *)(sb + ql * 256 + (((2 * kk + half) ^ (ql & 15)) << 4));
-            if (kk < 4) acc0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf, qf[kk], acc0, 0, 0, 0);
-            else acc1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf, qf[kk], acc1, 0, 0, 0);
-        }
-        const float *ksl = (const float *)(sb + kI8Tile) + 16 * half;
-#pragma unroll
-        for (int g = 0; g < 4; g++) {
-            const float4 k4 = *(const float4 *)(ksl + 4 * g);
-            const float kv4[4] = {k4.x, k4.y, k4.z, k4.w};
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int r = 4 * g + e;
-                const float f = __builtin_fmaf((float)acc0[r], __fmul_rn(qs0, kv4[e]), 0.f);
-                const float x = __builtin_fmaf((float)acc1[r], __fmul_rn(qs1, kv4[e]), f);
-                s[r] = (k0 + 16 * half + r < Sk) ? x : -INFINITY;
-            }
-        }
-    };
-
-    issue(0);
-    issue(1);
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    float keep[KEEP ? 4 : 1][16];
-    float mrun = -INFINITY, mfold = -INFINITY, lrun = 0.f, mt[4];
-    int nprev = 0;
-    // the partial sums of the group before (its tiles' maxima in mt), in tile order
-    auto fold = [&](int g) __attribute__((always_inline)) {
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            if (t < nprev) {
-                const float mnew = fmaxf(mfold, mt[t]);
-                if (mnew > -INFINITY) {
-                    lrun = (mfold == -INFINITY ? 0.f : lrun * __expf(mfold - mnew)) + pl[(g & 1) * 256 + t * 64 + lane];
-                    mfold = mnew;
+            for (int t = 0; t < 4; t++) {
+                if (t < nprev) {
+                    const float mnew = fmaxf(mfold, mt[t]);
+                    if (mnew > -INFINITY) {
+                        lrun = (mfold == -INFINITY ? 0.f : lrun * __expf(mfold - mnew)) + pl[(g & 1) * 256 + t * 64 + lane];
+                        mfold = mnew;
+                    }
                 }
             }
-        }
-    };
-    auto pass1 = [&](int g, float (&s)[16]) __attribute__((always_inline)) {
-        const int nt = min(4, ntiles - 4 * g);
-        float mloc = -INFINITY;
-        if (w < nt) {
-            scores(smem + (2 * w + (g & 1)) * kI8Buf, (4 * g + w) * 32, s);
+        };
+        auto pass1 = [&](int g, float (&s)[16]) __attribute__((always_inline)) {
+            const int nt = min(4, ntiles - 4 * g);
+            float mloc = -INFINITY;
+            if (w < nt) {
+                scores(smem + (2 * w + (g & 1)) * kI8Buf, (4 * g + w) * 32, s);
 #pragma unroll
-            for (int r = 0; r < 16; r++) mloc = fmaxf(mloc, s[r]);
-            mloc = fmaxf(mloc, xor_lane<32>(mloc));
-            if (half == 0) ml[(g & 1) * 128 + w * 32 + ql] = mloc;
-        }
-        step_done(g);
-        fold(g - 1);
-        float mine = mrun;
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            if (t < nt) {
-                mt[t] = ml[(g & 1) * 128 + t * 32 + ql];
-                mrun = fmaxf(mrun, mt[t]);
-                if (t == w) mine = mrun;
+                for (int r = 0; r < 16; r++) mloc = fmaxf(mloc, s[r]);
+                mloc = fmaxf(mloc, xor_lane<32>(mloc));
+                if (half == 0) ml[(g & 1) * 128 + w * 32 + ql] = mloc;
             }
-        }
-        nprev = nt;
-        if (w < nt) {
-            float ps = 0.f;
+            step_done(g);
+            fold(g - 1);
+            float mine = mrun;
 #pragma unroll
-            for (int r = 0; r < 16; r++) ps += s[r] == -INFINITY ? 0.f : __expf(s[r] - mine);
-            pl[(g & 1) * 256 + w * 64 + lane] = ps;
-        }
-    };
-    if constexpr (KEEP) {
-#pragma unroll
-        for (int g = 0; g < 4; g++)
-            if (g < nblk) pass1(g, keep[g]);
-    } else {
-        for (int g = 0; g < nblk; g++) pass1(g, keep[0]);
-    }
-    sync();
-    fold(nblk - 1);
-    const float ltot = lrun + xor_lane<32>(lrun);
-    const float inv_l = ltot > 0.f ? __fdiv_rn(1.0f, ltot) : 0.f;
-
-    float of[2][16];
-#pragma unroll
-    for (int dt = 0; dt < 2; dt++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) of[dt][r] = 0.f;
-    auto pass2 = [&](int g, float (&s)[16]) __attribute__((always_inline)) {
-        const int nt = min(4, ntiles - 4 * g), nv = KEEP ? nblk + g : nblk + 2 * g + 1;  // this block's V^T step
-        float pv[16], am = 0.f;
-#pragma unroll
-        for (int r = 0; r < 16; r++) pv[r] = 0.f;
-        if (w < nt) {
-            if (!KEEP) scores(smem + (2 * w + ((nv - 1) & 1)) * kI8Buf, (4 * g + w) * 32, s);
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const float e = s[r] == -INFINITY ? 0.f : __expf(s[r] - mrun);
-                pv[r] = __fmul_rn(e, inv_l);
-                am = fmaxf(am, pv[r]);
+            for (int t = 0; t < 4; t++) {
+                if (t < nt) {
+                    mt[t] = ml[(g & 1) * 128 + t * 32 + ql];
+                    mrun = fmaxf(mrun, mt[t]);
+                    if (t == w) mine = mrun;
+                }
             }
+            nprev = nt;
+            if (w < nt) {
+                float ps = 0.f;
+#pragma unroll
+                for (int r = 0; r < 16; r++) ps += s[r] == -INFINITY ? 0.f : __expf(s[r] - mine);
+                pl[(g & 1) * 256 + w * 64 + lane] = ps;
+            }
+        };
+        if constexpr (KEEP) {
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+                if (g < nblk) pass1(g, keep[g]);
+        } else {
+            for (int g = 0; g < nblk; g++) pass1(g, keep[0]);
         }
-        am = fmaxf(am, xor_lane<32>(am));
-        if (half == 0) ml[w * 32 + ql] = am;
-        if (KEEP && g == 0) sync();  // (step nblk - 1 was done in pass 1)
-        else step_done(nv - 1);
-#pragma unroll
-        for (int t = 0; t < 4; t++) am = fmaxf(am, ml[t * 32 + ql]);
-        const QScale ps = qscale(am);
-        v4i mine;
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-            mine[q] = (int)pack4_magic(pv[4 * q], pv[4 * q + 1], pv[4 * q + 2], pv[4 * q + 3], ps.inv);
-        *(v4i *)(pq8 + w * 1024 + lane * 16) = mine;
         sync();
-        v16i acc[2] = {(v16i){}, (v16i){}};
-        const unsigned char *vb = smem + (2 * w + (nv & 1)) * kI8Buf;
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            if (t < nt) {
-                const v4i pq = *(const v4i *)(pq8 + t * 1024 + lane * 16);
-#pragma unroll
-                for (int dt = 0; dt < 2; dt++) {
-                    const v4i vf = *(const v4i *)(vb + (32 * dt + ql) * 128 + (((2 * t + half) ^ (ql & 7)) << 4));
-                    acc[dt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf, pq, acc[dt], 0, 0, 0);
-                }
-            }
-        }
-        // d = 64 w + 32 dt + 8 (r / 4) + 4 half + r % 4
+        fold(nblk - 1);
+        const float ltot = lrun + xor_lane<32>(lrun);
+        const float inv_l = ltot > 0.f ? __fdiv_rn(1.0f, ltot) : 0.f;
+
+        float of[2][16];
 #pragma unroll
         for (int dt = 0; dt < 2; dt++)
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const float4 v4 = *(const float4 *)(vs_l + 64 * w + 32 * dt + 8 * q + 4 * half);
-                const float vv[4] = {v4.x, v4.y, v4.z, v4.w};
+            for (int r = 0; r < 16; r++) of[dt][r] = 0.f;
+        auto pass2 = [&](int g, float (&s)[16]) __attribute__((always_inline)) {
+            const int nt = min(4, ntiles - 4 * g), nv = KEEP ? nblk + g : nblk + 2 * g + 1;  // this block's V^T step
+            float pv[16], am = 0.f;
 #pragma unroll
-                for (int e = 0; e < 4; e++)
-                    of[dt][4 * q + e] = __builtin_fmaf((float)acc[dt][4 * q + e], __fmul_rn(ps.sc, vv[e]), of[dt][4 * q + e]);
+            for (int r = 0; r < 16; r++) pv[r] = 0.f;
+            if (w < nt) {
+                if (!KEEP) scores(smem + (2 * w + ((nv - 1) & 1)) * kI8Buf, (4 * g + w) * 32, s);
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const float e = s[r] == -INFINITY ? 0.f : __expf(s[r] - mrun);
+                    pv[r] = __fmul_rn(e, inv_l);
+                    am = fmaxf(am, pv[r]);
+                }
             }
-        if (!KEEP) step_done(nv);
-    };
-    if constexpr (KEEP) {
+            am = fmaxf(am, xor_lane<32>(am));
+            if (half == 0) ml[w * 32 + ql] = am;
+            if (KEEP && g == 0) sync();  // (step nblk - 1 was done in pass 1)
+            else step_done(nv - 1);
 #pragma unroll
-        for (int g = 0; g < 4; g++)
-            if (g < nblk) pass2(g, keep[g]);
-    } else {
-        for (int g = 0; g < nblk; g++) pass2(g, keep[0]);
-    }
-
-    // a 128-dim block is two waves'
-    float am = 0.f;
+            for (int t = 0; t < 4; t++) am = fmaxf(am, ml[t * 32 + ql]);
+            const QScale ps = qscale(am);
+            v4i mine;
 #pragma unroll
-    for (int dt = 0; dt < 2; dt++)
+            for (int q = 0; q < 4; q++)
+                mine[q] = (int)pack4_magic(pv[4 * q], pv[4 * q + 1], pv[4 * q + 2], pv[4 * q + 3], ps.inv);
+            *(v4i *)(pq8 + w * 1024 + lane * 16) = mine;
+            sync();
+            v16i acc[2] = {(v16i){}, (v16i){}};
+            const unsigned char *vb = smem + (2 * w + (nv & 1)) * kI8Buf;
 #pragma unroll
-        for (int r = 0; r < 16; r++) am = fmaxf(am, fabsf(of[dt][r]));
-    am = fmaxf(am, xor_lane<32>(am));
-    if (half == 0) ml[128 + w * 32 + ql] = am;
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    am = fmaxf(am, ml[128 + (w ^ 1) * 32 + ql]);
-    const QScale qs = qscale(am);
-    if (qi >= Sk) return;  // rows past the sequence belong to the next one
-    const size_t orow = row0 + qi;
+            for (int t = 0; t < 4; t++) {
+                if (t < nt) {
+                    const v4i pq = *(const v4i *)(pq8 + t * 1024 + lane * 16);
 #pragma unroll
-    for (int dt = 0; dt < 2; dt++)
+                    for (int dt = 0; dt < 2; dt++) {
+                        const v4i vf = *(const v4i *)(vb + (32 * dt + ql) * 128 + (((2 * t + half) ^ (ql & 7)) << 4));
+                        acc[dt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf, pq, acc[dt], 0, 0, 0);
+                    }
+                }
+            }
+            // d = 64 w + 32 dt + 8 (r / 4) + 4 half + r % 4
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int d = 64 * w + 32 * dt + 8 * q + 4 * half;
-            *(uint32_t *)(a.cq + orow * HD + h * kI8D + d) =
-                pack4_magic(of[dt][4 * q], of[dt][4 * q + 1], of[dt][4 * q + 2], of[dt][4 * q + 3], qs.inv);
-            if (a.c32)
-                *(float4 *)(a.c32 + orow * HD + h * kI8D + d) =
-                    make_float4(of[dt][4 * q], of[dt][4 * q + 1], of[dt][4 * q + 2], of[dt][4 * q + 3]);
+            for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const float4 v4 = *(const float4 *)(vs_l + 64 * w + 32 * dt + 8 * q + 4 * half);
+                    const float vv[4] = {v4.x, v4.y, v4.z, v4.w};
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        of[dt][4 * q + e] = __builtin_fmaf((float)acc[dt][4 * q + e], __fmul_rn(ps.sc, vv[e]), of[dt][4 * q + e]);
+                }
+            if (!KEEP) step_done(nv);
+        };
+        if constexpr (KEEP) {
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+                if (g < nblk) pass2(g, keep[g]);
+        } else {
+            for (int g = 0; g < nblk; g++) pass2(g, keep[0]);
         }
-    if (half == 0 && !(w & 1)) a.cs[orow * (HD / kQBlock) + h * 2 + (w >> 1)] = qs.sc;
+
+        // a 128-dim block is two waves'
+        float am = 0.f;
+#pragma unroll
+        for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) am = fmaxf(am, fabsf(of[dt][r]));
+        am = fmaxf(am, xor_lane<32>(am));
+        if (half == 0) ml[128 + w * 32 + ql] = am;
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        am = fmaxf(am, ml[128 + (w ^ 1) * 32 + ql]);
+        const QScale qs = qscale(am);
+        const size_t orow = row0 + qi;
+        if (qi < Sk) {  // rows past the sequence belong to the next one
+#pragma unroll
+            for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int d = 64 * w + 32 * dt + 8 * q + 4 * half;
+                    *(uint32_t *)(a.cq + orow * HD + h * kI8D + d) =
+                        pack4_magic(of[dt][4 * q], of[dt][4 * q + 1], of[dt][4 * q + 2], of[dt][4 * q + 3], qs.inv);
+                    if (a.c32)
+                        *(float4 *)(a.c32 + orow * HD + h * kI8D + d) =
+                            make_float4(of[dt][4 * q], of[dt][4 * q + 1], of[dt][4 * q + 2], of[dt][4 * q + 3]);
+                }
+            if (half == 0 && !(w & 1)) a.cs[orow * (HD / kQBlock) + h * 2 + (w >> 1)] = qs.sc;
+        }
+    }
 }
 
 static size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -428,8 +435,15 @@ static int launch_attn_i8(hipStream_t s, const AttnI8Args &a, int B, int max_len
             return -1;
         attr = true;
     }
-    const dim3 grid = a.work ? dim3((n_work + 7) / 8 * 32) : dim3((max_len + 31) / 32, a.H, B);
-    hipLaunchKernelGGL(k_attn_i8<KEEP>, grid, dim3(256), kAttnI8Lds, s, a, n_work);
+    // A work entry has four blocks of 32 queries, fewer where no sequence is that long, each a workgroup's: one
+    // whose block lies past its sequence costs 1-2 us of a CU's slot (300 x 1-66, 3 heads: 71.2 us with four
+    // workgroups an entry, 43.3 with three). From three entries a CU of sequences of at most 128, one
+    // workgroup walks an entry's blocks instead (four | one: 3 heads, 300 x 1-128 86.8 | 65.8; 15 heads, 64 x 8-100
+    // 83.9 | 60.9, 128 x 100-128 220.5 | 216.8; with fewer, 3 heads, 128 x 100-128 50.8 | 55.2).
+    int nwg = std::min(4, (max_len + 31) / 32);
+    if (max_len <= 128 && n_work >= 3 * num_cus()) nwg = 1;
+    const dim3 grid = a.work ? dim3((n_work + 7) / 8 * 8 * nwg) : dim3((max_len + 31) / 32, a.H, B);
+    hipLaunchKernelGGL(k_attn_i8<KEEP>, grid, dim3(256), kAttnI8Lds, s, a, n_work, nwg);
     return check_hip(hipGetLastError(), "attention_i8 launch");
 }
 

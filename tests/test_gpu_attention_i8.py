@@ -226,3 +226,23 @@ def test_attention_i8_kept_scores_match_recomputed(gpu, rng):
         got = e2mi.attention_i8_packed(q, k, v, sd, ld, max_len, H, KV, work=wk)
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("H,KV,B,longest", [(15, 3, 60, 128), (15, 3, 60, 66), (3, 1, 300, 97), (3, 1, 20, 32)])
+def test_attention_i8_short_sequences(gpu, rng, H, KV, B, longest):
+    """Lists of many short sequences, where a workgroup walks an entry's blocks (60 x 15 and 300 x 3 entries) or
+    an entry has fewer than four, against the grid without a list (a workgroup per block), bit for bit; rows
+    outside every sequence stay as they were."""
+    import torch
+    import e2mi
+    lens = [longest, 0, 1, 31, 32, 33, 64] + [int(x) for x in rng.integers(1, longest + 1, B - 7)]
+    lens = [min(n, longest) for n in lens]
+    rowmap, pos, start, plen, M = _packed(rng, e2mi, lens, longest)
+    q, k, v = (_t(x, gpu) for x in _inputs(rng, M, H, KV))
+    sd, ld = _t(start, gpu), _t(plen, gpu)
+    work = e2mi.attention_work(plen, H)
+    work = _t(np.concatenate([work, np.full(37, -1, np.int32)]), gpu)
+    want = e2mi.attention_i8_packed(q, k, v, sd, ld, longest, H, KV)
+    got = e2mi.attention_i8_packed(q, k, v, sd, ld, longest, H, KV, work=work)
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
