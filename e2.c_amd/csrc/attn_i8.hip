@@ -45,13 +45,14 @@ struct I8PrepArgs {
     float *vs;                     // [B][KV][D]
     const int32_t *seq_start, *seq_len;
     int M, H, KV, nch;
-    int nbk, nv;  // B KV, and its workgroups of the first launch (nbk nch)
+    int nbk;      // B KV
+    uint32_t nv;  // V's workgroups of the first launch (nbk nch)
 };
 
 // V's part of the launch: workgroup c B KV + (b, kv) takes the column maxima of rows [64 c, 64 c + 64)
 // of the sequence, thread = dim
-__device__ inline void i8_vmax(const I8PrepArgs &a, int blk) {
-    const int bk = blk % a.nbk, c = blk / a.nbk, b = bk / a.KV, kv = bk % a.KV, d = threadIdx.x;
+__device__ inline void i8_vmax(const I8PrepArgs &a, uint32_t blk) {
+    const int bk = blk % (uint32_t)a.nbk, c = blk / (uint32_t)a.nbk, b = bk / a.KV, kv = bk % a.KV, d = threadIdx.x;
     const int L = a.seq_len[b], r0 = 64 * c;
     if (r0 >= L) return;
     const int r1 = min(L, r0 + 64);
@@ -70,9 +71,10 @@ __device__ inline void i8_vmax(const I8PrepArgs &a, int blk) {
 }
 
 __global__ __launch_bounds__(256) void k_i8_prep(I8PrepArgs a) {
-    if ((int)blockIdx.x < a.nv) return i8_vmax(a, blockIdx.x);
+    const uint32_t blk = blockIdx.x + gridDim.x * blockIdx.y;  // (one row of the grid but for very many workgroups)
+    if (blk < a.nv) return i8_vmax(a, blk);
     const int lane = threadIdx.x & 63;
-    const long item = (long)(blockIdx.x - a.nv) * 4 + (threadIdx.x >> 6);
+    const long item = (long)(blk - a.nv) * 4 + (threadIdx.x >> 6);
     const int per = a.H + a.KV;
     if (item >= (long)a.M * per) return;
     const int row = (int)(item / per), j = (int)(item % per);
@@ -503,10 +505,11 @@ extern "C" int e2mi_attention_i8_packed(e2mi_stream stream, const float *q32, co
     unsigned char *ws = (unsigned char *)workspace;
     I8PrepArgs p = {q32, k32, v32, (int8_t *)(ws + wo.q8), (float *)(ws + wo.qs), (int8_t *)(ws + wo.k8),
                     (float *)(ws + wo.ks), (int8_t *)(ws + wo.vt8), (float *)(ws + wo.vpart),
-                    (float *)(ws + wo.vs), seq_start, seq_len, M, H, KV, (max_len + 63) / 64, B * KV, B * KV * ((max_len + 63) / 64)};
+                    (float *)(ws + wo.vs), seq_start, seq_len, M, H, KV, (max_len + 63) / 64, B * KV, (uint32_t)B * KV * ((max_len + 63) / 64)};
     hipStream_t s = (hipStream_t)stream;
-    const long items = (long)M * (H + KV);
-    hipLaunchKernelGGL(k_i8_prep, dim3((unsigned)(p.nv + (items + 3) / 4)), dim3(256), 0, s, p);
+    // a dimension of a grid takes 2^32 threads: 2^20 workgroups a row where one row would not do
+    const long items = (long)M * (H + KV), prep = p.nv + (items + 3) / 4, row = prep < (1L << 24) ? prep : 1L << 20;
+    hipLaunchKernelGGL(k_i8_prep, dim3((unsigned)row, (unsigned)((prep + row - 1) / row)), dim3(256), 0, s, p);
     hipLaunchKernelGGL(k_i8_vquant, dim3(B * KV, (max_len + 31) / 32), dim3(256), 0, s, p);
     const AttnI8Args a = {p.q8, p.qs, p.k8, p.ks, p.vt8, p.vs, ctx_q, ctx_s, ctx32, seq_start, seq_len, work, M, H, KV};
     return max_len <= kI8Keep ? launch_attn_i8<true>(s, a, B, max_len, n_work) : launch_attn_i8<false>(s, a, B, max_len, n_work);

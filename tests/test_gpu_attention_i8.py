@@ -246,3 +246,21 @@ def test_attention_i8_short_sequences(gpu, rng, H, KV, B, longest):
     got = e2mi.attention_i8_packed(q, k, v, sd, ld, longest, H, KV, work=work)
     torch.cuda.synchronize()
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_attention_i8_prep_past_one_grid_row(gpu, rng):
+    """65,535 sequences (all but the first empty) with a max_len of 16,256: V's column maxima and the Q and K
+    rows together are more workgroups of 256 threads than one dimension of a grid takes. The first
+    sequence's context equals its own call's."""
+    import torch
+    import e2mi
+    B, L, max_len, M = 65535, 70, 16256, 270336
+    q, k, v = (torch.randn((M, D), generator=torch.Generator(device=gpu).manual_seed(i), device=gpu) * 0.3 for i in range(3))
+    start, plen = torch.zeros(B, dtype=torch.int32, device=gpu), torch.zeros(B, dtype=torch.int32, device=gpu)
+    plen[0] = L
+    work = torch.zeros(1, dtype=torch.int32, device=gpu)  # sequence 0, head 0, query block 0
+    assert B * ((max_len + 63) // 64) + M // 2 > 1 << 24
+    got = e2mi.attention_i8_packed(q, k, v, start, plen, max_len, 1, 1, work=work)
+    want = e2mi.attention_i8_packed(q[:256], k[:256], v[:256], start[:1], plen[:1], L, 1, 1)
+    torch.cuda.synchronize()
+    assert all(torch.equal(a[:L], b[:L]) for a, b in zip(got, want))
