@@ -1228,9 +1228,7 @@ static int attention_packed(const char *who, e2mi_stream stream, const uint16_t 
     const bool direct = M % 2 == 0 && (size_t)KV * D * M * 2 < 0x7fffffffu &&
                         (size_t)M * KV * D * 2 < 0x7fffffffu && ((uintptr_t)vt16 & 3) == 0;
     const dim3 grid = work ? dim3(n_work) : dim3((max_len + 127) / 128, H, B);
-    const DeviceRows dr = device_rows();
-    const int rows = dr.ptr && dr.est > 0 ? std::min(dr.est, M) : M;
-    const int qs = merge ? 0 : attn_group_blocks(rows, B, max_len, H, D, work != nullptr);
+    const int qs = merge ? 0 : attn_group_blocks(device_rows().few(M), B, max_len, H, D, work != nullptr);
     if (direct && qs) {
         const hipStream_t st = (hipStream_t)stream;
         if (D == 512)

@@ -162,7 +162,7 @@ struct e2mi_engine {
     std::pair<int, int> slot_shape[kFlagSlots];
     std::map<std::pair<int, int>, int> rows_seen;
     bool packed = true;
-    // (sequences, seq_len, rows, bits: packed 1, split 2, planned on the device 4, tile_signature above)
+    // (sequences, seq_len, rows, bits: packed 1, split 2, planned on the device 4, forward_signature)
     std::map<std::tuple<int, int, int, long>, hipGraphExec_t> graphs;
     bool use_graph = true;
     bool fuse_qkv = true;  // E2MI_NOFUSE=1: the q|k|v GEMM and the norm/RoPE kernel run separately
@@ -371,10 +371,9 @@ constexpr int kAttnPartTiles = 8, kMaxAttnParts = 4;
 // 100, 1899 | 1852 | 2216 at 300; BASELINE geometry 1003 | 1007 | 1226, 1122 | 1120 | 1366, 1455 | 1334 |
 // 1510.
 enum NormForm { NORM_SEPARATE, NORM_FUSED, NORM_AHEAD };
-static NormForm norm_form(const e2mi_engine *g, int rows) {
-    const e2_config &c = g->cfg;
-    if (!g->fuse_an || (c.hidden != 768 && c.hidden != 512) || !gemm_an_fits(rows)) return NORM_SEPARATE;
-    return rows <= 256 ? NORM_AHEAD : NORM_FUSED;
+static NormForm norm_form(const e2_config &c, bool fuse_an, const DeviceRows &dr, int M) {
+    if (!fuse_an || (c.hidden != 768 && c.hidden != 512) || !gemm_an_fits(dr.expected(M))) return NORM_SEPARATE;
+    return dr.few(M) <= 256 ? NORM_AHEAD : NORM_FUSED;
 }
 
 // every kernel of one forward over B sequences of S tokens (M rows: B * S padded, or the packed
@@ -385,10 +384,10 @@ static int enqueue(e2mi_engine *g, int B, int S, int Mp, bool pk, hipStream_t s,
     const DeviceRowsScope dev_rows(dev ? g->d_rows : nullptr, 1, est);
     const e2_config &c = g->cfg;
     const int M = pk ? Mp : B * S, Dm = c.hidden, H = c.n_heads, P = c.ple_dim;
-    const NormForm form = norm_form(g, dev && est > 0 ? est : M);
+    const NormForm form = norm_form(c, g->fuse_an, device_rows(), M);
     const bool an = form == NORM_FUSED;
     // launches of a projection with its norm_add past the first
-    auto an_extra = [&](const e2mi_q8w &w) { return gemm_an_split(dev && est > 0 ? est : M, w.N, w.K) ? 1 : 0; };
+    auto an_extra = [&](const e2mi_q8w &w) { return gemm_an_split(device_rows().few(M), w.N, w.K) ? 1 : 0; };
     // form ahead: x moves between two buffers, each norm_add reading one and writing the other
     float *x = g->x, *x_other = g->xn;
     if (M <= 0 || M > g->R) {
@@ -703,41 +702,45 @@ static int plan_pack(e2mi_engine *g, const uint8_t *valid, int n, int S) {
     return Mp;
 }
 
-// The kernels of a device-planned forward of about `est` rows: for every distinct GEMM of the forward
-// whose kernel follows the row count, which one takes it (gemm_small_route, gemm_half_tiles), and
-// how the projections run their norm_add (fused: in how many row units per workgroup, 1-5, and how many
-// of them in two launches, those of larger K first)
-static long tile_signature(const e2mi_engine *g, int est) {
-    const e2_config &c = g->cfg;
-    const NormForm form = norm_form(g, est);
-    // whether a projection runs as a GEMM of its own, and how many fused ones run in two launches
+// The kernels of a device-planned forward of about `est` rows in M of capacity, as the key of its recording:
+// for every distinct GEMM whose kernel follows the row count, which one takes it (gemm_small_route,
+// gemm_half_tiles), and how the projections run their norm_add (fused: in how many row units per workgroup,
+// 1-5, and how many of them in two launches, those of larger K first)
+long forward_signature(const e2_config &c, bool fuse_an, bool fuse_qkv, int M, int est) {
+    const int planned = 0;  // (any device count: the estimate is what counts here)
+    const DeviceRows dr{&planned, 1, est};
+    const int few = dr.few(M), H = c.n_heads;
+    const bool with_an = fuse_an && (c.hidden == 768 || c.hidden == 512);
+    const NormForm form = norm_form(c, fuse_an, dr, M);
+    // a projection of K columns: whether it runs as a GEMM of its own
     int split = 0;
-    auto alone = [&](const e2mi_q8w &w, bool with_an) {
+    auto alone = [&](int K) {
         if (!with_an || form != NORM_FUSED) return true;
-        const bool two = gemm_an_split(est, w.N, w.K);
+        const bool two = gemm_an_split(few, c.hidden, K);
         split += two;
         return two;
     };
     std::vector<std::tuple<int, int, int>> gemms;  // N, K, epilogue
-    auto add = [&](const e2mi_q8w &w, int epi) { gemms.emplace_back(w.N, w.K, epi); };
-    for (const LayerDev &L : g->layers) {
-        add(L.qkv, L.qkv_fused ? EPI_QKV : EPI_F32);
-        add(L.gu, EPI_GEGLU);
-        if (alone(L.o, L.o_an)) add(L.o, EPI_F32);
-        if (alone(L.down, L.down_an)) add(L.down, EPI_F32);
+    auto add = [&](int N, int K, int epi) { gemms.emplace_back(N, K, epi); };
+    for (int l = 0; l < c.n_layers; l++) {
+        const LayerGeom g = layer_geom(c, l);
+        add((H + 2 * g.KV) * g.D, c.hidden, fuse_qkv && g.D == 256 ? EPI_QKV : EPI_F32);
+        add(2 * c.ffn, c.hidden, EPI_GEGLU);
+        if (alone(H * g.D)) add(c.hidden, H * g.D, EPI_F32);
+        if (alone(c.ffn)) add(c.hidden, c.ffn, EPI_F32);
         if (c.ple_dim > 0) {
-            add(L.ple_gate, EPI_GELUMUL);
-            if (alone(L.ple_proj, L.down_an)) add(L.ple_proj, EPI_F32);
+            add(c.ple_dim, c.hidden, EPI_GELUMUL);
+            if (alone(c.ple_dim)) add(c.hidden, c.ple_dim, EPI_F32);
         }
     }
-    if (c.ple_dim > 0) add(g->ple_model, EPI_F32);
-    if (c.out_dim > 0) add(g->embed_proj, EPI_F32);
+    if (c.ple_dim > 0) add(c.n_layers * c.ple_dim, c.hidden, EPI_F32);
+    if (c.out_dim > 0) add(c.out_dim, c.hidden, EPI_F32);
     std::sort(gemms.begin(), gemms.end());
     gemms.erase(std::unique(gemms.begin(), gemms.end()), gemms.end());
-    long sig = form == NORM_FUSED ? gemm_an_units(est) : form == NORM_AHEAD ? 6 : 7;
-    for (const auto &[N, K, epi] : gemms) {  // at most 14 of them, 3 bits each
-        const int small = gemm_small_route(est, N, K, epi, false);
-        sig = sig << 3 | (small ? small : gemm_half_tiles(est, N) ? 4 : 0);
+    long sig = form == NORM_FUSED ? gemm_an_units(dr.expected(M)) : form == NORM_AHEAD ? 6 : 7;
+    for (const auto &[N, K, epi] : gemms) {  // at most 12 of them, 3 bits each
+        const int small = gemm_small_route(few, N, K, epi, false);
+        sig = sig << 3 | (small ? small : gemm_half_tiles(dr.expected(M), N) ? 4 : 0);
     }
     return sig << 8 | std::min(split, 255);
 }
@@ -1299,7 +1302,7 @@ extern "C" int e2mi_text_embed_batch_device(e2mi_engine *g, const int32_t *ids, 
         const auto seen = g->rows_seen.find(std::make_pair(batch, seq_len));
         const int est = seen != g->rows_seen.end() ? std::min(seen->second, cap) : cap;
         if (launch_plan_packed(s, pa) ||
-            run_shape(g, batch, seq_len, cap, true, s, true, est, tile_signature(g, est)) ||
+            run_shape(g, batch, seq_len, cap, true, s, true, est, forward_signature(g->cfg, g->fuse_an, g->fuse_qkv, cap, est)) ||
             check_hip(hipMemcpyAsync(out, g->out, (size_t)batch * g->dout * 4, hipMemcpyDeviceToDevice, s),
                       "out D2D"))
             return -1;

@@ -1854,18 +1854,11 @@ bool gemm_half_tiles(int M, int N) {
     return r128 <= r256 - 0.3;
 }
 // in a forward planned on the device, for the host's estimate of the planned row count
-static bool half_tiles(const GemmArgs &p) {
-    const int est = p.rows ? device_rows().est : 0;
-    return gemm_half_tiles(est > 0 && est < p.M ? est : p.M, p.N);
-}
+static bool half_tiles(const GemmArgs &p) { return gemm_half_tiles(device_rows().expected(p.M), p.N); }
 
-static int expected_rows(const GemmArgs &p) {
-    const int est = p.rows ? device_rows().est : 0;
-    return est > 0 && est < p.M ? est : p.M;
-}
 // the kernels for few rows (gemm_s.hip) where they are the faster ones
 #define E2MI_TRY_SMALL(epi, tok)                                                                   \
-    if (const int rc = launch_gemm_small(s, p, epi, expected_rows(p), tok)) return rc < 0 ? -1 : 0
+    if (const int rc = launch_gemm_small(s, p, epi, device_rows().few(p.M), tok)) return rc < 0 ? -1 : 0
 
 int launch_gemm_f32(hipStream_t s, GemmArgs p, bool dump, bool tok = false) {
     if (check_args(p, "i8_gemm", !dump && !tok)) return -1;

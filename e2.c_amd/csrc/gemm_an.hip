@@ -440,9 +440,9 @@ static int gemm_add_norm(hipStream_t s, const int8_t *qa, const float *a_scales,
     a.A = qa; a.as = a_scales; a.W = w->w; a.ws = w->scale; a.res = res; a.gamma_a = gamma_add;
     a.gamma_n = gamma_next; a.x_out = x_out; a.xn_out = xn_out; a.q = q; a.qs = qs; a.y = y;
     a.lda = w->K; a.ldw = w->ld; a.M = M; a.K = w->K; a.eps = eps; a.post_scale = post_scale;
-    const int est = dr.ptr && dr.est > 0 && dr.est < M ? dr.est : M;
+    const int est = dr.expected(M);
     // (the GEMM asks for a weight on 16 bytes; k_gemm_an's loads take any 4-byte address)
-    if (gemm_an_split(est, D, w->K) && (!engine || tmp) && aligned16(w->w)) {
+    if (gemm_an_split(dr.few(M), D, w->K) && (!engine || tmp) && aligned16(w->w)) {
         // the projection goes through the engine's scratch, through y where one is asked for, or through x_out,
         // which the row kernel then overwrites row by row; y and x_out only beside the inputs, which the
         // GEMM's and the row kernel's workgroups still read while others write them (k_gemm_an's read a row's

@@ -32,8 +32,8 @@ struct GemmArgs {
     float *q32, *k32, *v32;
     int qH, qKV, qS;
     float eps;
-    // a device row count (a multiple of 256, at most M; k_gemm_p only, which takes it as its own
-    // first argument), or null: M rows
+    // a device row count (a multiple of 256, past M where M is below 256), which the kernels but the
+    // per-token ones take as their own first argument, or null: M rows
     const int *rows;
 };
 
@@ -57,11 +57,12 @@ class NormInScope {
 };
 
 // gemm_s.hip: the kernels for few rows, and which one (0: none) takes an M x N x K GEMM with the
-// epilogue `epi` (tok: per-token activation scales); launch_gemm_small runs it at the expected row
-// count and returns 1, or returns 0 for the caller's kernels and -1 on error
-enum { GEMM_SK = 1, GEMM_S32 = 2, GEMM_S64 = 3, GEMM_RING = 5 };  // (4 is tile_signature's)
+// epilogue `epi` (tok: per-token activation scales); launch_gemm_small runs it, its tiles of the first
+// `few` rows before those of the rest (DeviceRows::few), and returns 1, or returns 0 for the caller's kernels
+// and -1 on error
+enum { GEMM_SK = 1, GEMM_S32 = 2, GEMM_S64 = 3, GEMM_RING = 5 };  // (4 is forward_signature's)
 int gemm_small_route(int M, int N, int K, int epi, bool tok);
-int launch_gemm_small(hipStream_t s, const GemmArgs &p, int epi, int est, bool tok);
+int launch_gemm_small(hipStream_t s, const GemmArgs &p, int epi, int few, bool tok);
 
 #if defined(__HIPCC__)
 // LDS tiles hold 128-byte K slices of consecutive rows with no padding. The LDS has 64 banks of 4

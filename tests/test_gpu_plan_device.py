@@ -151,3 +151,31 @@ def test_reference_geometry_device_plan(gpu):
         ids, valid = random_batch(rng, B, S, cfg.vocab, min_len=100, holes=k == 1)
         d, h = _embed_both(eng, ids, valid, gpu)
         assert np.array_equal(d, h)
+
+
+@pytest.mark.parametrize("geom", ["base", "ref"])
+def test_row_count_moves_within_a_shape(gpu, monkeypatch, geom):
+    """One shape's row count from a few rows to the capacity and back, each forward in the kernels chosen for
+    the call before: the norm_add in the GEMM that reads it (capacity 512, a first call of 40 rows) over
+    masks with more rows than its first tiles cover, the small tiles past the expected rows, the large tiles
+    over a few rows. The device entry equals the host entry, and the host entry the unfused
+    kernels (E2MI_NOFUSE_AN=1), bit for bit."""
+    import e2mi
+    from model_util import reference_small_config, small_config
+    rng = np.random.default_rng(79)
+    cfg = small_config(e2mi, n_layers=2) if geom == "base" else reference_small_config(e2mi, n_layers=6)
+    m = e2mi.Model.synthetic(cfg, 8)
+    monkeypatch.setenv("E2MI_NOFUSE_AN", "1")
+    plain = e2mi.Engine(m, max_rows=8192)
+    monkeypatch.delenv("E2MI_NOFUSE_AN")
+    for B, S, rows in [(4, 128, (20, 20, 512, 19, 300, 300, 40)), (2, 33, (66, 1, 1, 50)), (1, 19, (19, 3, 19)),
+                       (8, 256, (40, 2048, 40, 40, 1100, 1500)), (16, 512, (100, 100, 8000, 5000, 100))]:
+        eng = e2mi.Engine(m, max_rows=8192)
+        ids = rng.integers(0, cfg.vocab, (B, S)).astype(np.int32)
+        for n in rows:
+            valid = np.zeros((B, S), np.uint8)
+            for b in range(B):
+                valid[b, :min(S, n // B + (b < n % B))] = 1
+            d, h = _embed_both(eng, ids, valid, gpu)
+            assert np.array_equal(d, h), (B, S, n)
+            assert np.array_equal(plain.embed_batch(ids, valid), h), (B, S, n, "unfused")
