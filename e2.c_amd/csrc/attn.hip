@@ -1113,25 +1113,28 @@ __global__ __launch_bounds__(256) void k_attn_merge(AttnArgs a, const int32_t *m
     }
 }
 
-// Blocks of 32 (1), 64 (2) or 128 (0) queries by how many of them the sequences have, about H (rows / 32 +
-// B / 2) and H (rows / 64 + B / 2): 32 while those leave a fifth of the CUs idle, 64 while they fit one round
-// of the CUs, one workgroup each; past that the larger K and V^T traffic of small blocks costs more than
-// idle CUs. us per launch at 128 | 64 | 32 queries (32-query blocks in brackets): head_dim 256, 3 heads, 1 x
-// 100 tokens 10.9 | 10.3 | 8.7 [12], 2 x 90-301 18.0 | 15.1 | 13.0 [51], 8 x 64-512 24.7 | 18.2 | 20.1 [237], 16
-// x 64-512 26.1 | 21.4 | 32.8 [459], 32 x 64-512 28.8 | 39.4 | 57.7 [930]; 4 heads, window 512, 1 x 2048 64.8 |
-// 34.6 | 34.5 [256], 2 x 1024-2048 71.5 | 37.6 | 65.6 [464], 4 x 1024-2048 76.3 | 70.9 | 108.3 [864], 8 x
-// 1024-2048 89.0 | 108.7 | 175.4; head_dim 512, 1 x 300 36.5 | 21.6 | 19.6 [40], 1 x 2048 158.8 | 95.3 | 87.0 [256],
-// 2 x 700-1500 122.9 | 73.7 | 115.4 [340], 4 x 1024-2048 166.2 | 185.8 | 289.9. At head_dim 256 a sequence of one
-// or two key tiles gains nothing (19 tokens: 7.1 | 7.8 | 7.4).
+// Blocks of 32 (1), 64 (2) or 128 (0) queries: the smallest whose workgroups, those past their sequence's end
+// among them, are one round of the CUs, one each. A sequence's last work entry of 128 queries is half full on
+// average, so the entries are about H (rows / 128 + B / 2) and the workgroups 128 / q times that. Idle ones count
+// though they exit at once: a shader engine gets every fourth workgroup in turn, the idle ones at regular
+// places, and one with nine busy workgroups for eight CUs makes a second round. us per launch at 128 | 64 | 32
+// queries (workgroups so estimated in brackets): head_dim 256, 3 heads, 1 x 100 tokens 10.9 | 10.3 | 8.7 [-, 9, 18],
+// 2 x 90-301 18.0 | 15.1 | 13.0 [-, 30, 60], 8 x 64-512 21.5 | 18.2 | 16.0 [-, 132, 264], 16 x 64-512 22.6 | 19.5 |
+// 26.1 [-, 252, 504], 32 x 118-142 13.0 | 23.8 | 25.3 [-, 300, 600], 16 x 266-319 17.3 | 27.4 | 33.9 [-, 276, 552];
+// 4 heads, window 512, 1 x 2048 60.0 | 35.8 | 33.8 [-, 132, 264], 20 x 55-66 11.4 | 12.0 | 17.9 [-, 160, 320]; over 1262
+// such shapes 12.6 % less time than 128-query blocks alone, three more than 4 % slower. At head_dim 512 the
+// chain is longer and a little crowding costs less than it saves (1 x 2048 147 | 97 | 81, 12 x 266-319 38.4 |
+// 43.3 | 56.3). At head_dim 256 a sequence of one or two key tiles gains nothing (19 tokens: 7.1 | 7.8 | 7.4).
 // Without a work list the grid has every block of max_len for every sequence, and neighbouring query blocks
 // lie on neighbouring XCDs, so the first ones' XCDs get all the short sequences: there the whole grid is counted
 // (3 heads without a list, 128 | 64 us: 12 x 64-512 24.9 | 28.4, 16 x 64-512 23.6 | 31.0; 8 x 64-512 21.7 | 18.4).
 int attn_group_blocks(int rows, int B, int max_len, int H, int D, bool list) {
     if (D == 256 && max_len <= 64) return 0;
-    const double C = num_cus();
-    auto blocks = [&](int q) { return list ? H * ((double)rows / q + B / 2.0) : (double)H * B * ((max_len + q - 1) / q); };
-    if (blocks(32) <= 0.8 * C) return 1;
-    return blocks(64) <= C ? 2 : 0;
+    auto one_round = [&](int q) {
+        const double entry = D == 512 && q == 64 ? 0.75 : 64.0 / q;  // a sequence's blocks past its rows
+        return H * (list ? (double)rows / q + entry * B : (double)B * ((max_len + q - 1) / q)) <= num_cus();
+    };
+    return one_round(32) ? 1 : one_round(64) ? 2 : 0;
 }
 
 template <int D, bool WIN, int QS>

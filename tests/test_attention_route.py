@@ -18,7 +18,11 @@ def blocks():
 @pytest.mark.parametrize("shape,listed,grid", [((768, 2, 300, 3, 256), 1, 1), ((2304, 8, 512, 3, 256), 2, 2),
                                                ((4352, 12, 512, 3, 256), 2, 0), ((4352, 16, 512, 3, 256), 2, 0),
                                                ((10496, 40, 512, 1, 256), 2, 0), ((10240, 32, 512, 3, 256), 0, 0),
-                                               ((256, 1, 64, 3, 256), 0, 0), ((2048, 1, 2048, 4, 512), 2, 2)])
+                                               ((256, 1, 64, 3, 256), 0, 0), ((2048, 1, 2048, 4, 512), 2, 1),
+                                               # measured slower in 64-query blocks, then in 32-query ones
+                                               ((4352, 32, 142, 3, 256), 0, 0), ((3584, 48, 77, 3, 256), 0, 0),
+                                               ((4864, 16, 319, 3, 256), 0, 2), ((1280, 24, 77, 8, 256), 0, 0),
+                                               ((1280, 20, 66, 4, 256), 2, 1)])
 def test_block_size(blocks, shape, listed, grid):
     assert blocks(*shape, True) == listed
     assert blocks(*shape, False) == grid
