@@ -204,6 +204,8 @@ int launch_gemm_add_norm(hipStream_t s, const int8_t *qa, const float *a_scales,
                          const float *res, const float *gamma_add, float post_scale, const float *gamma_next,
                          float eps, float *x_out, float *xn_out, int8_t *q, float *qs, bool scale, float *tmp);
 bool gemm_an_split(int rows, int N, int K);
+// attn.hip: the packed attention's query block size (1: 32, 2: 64, 0: 128) for B sequences of up to max_len
+int attn_group_blocks(int rows, int B, int max_len, int H, int D, bool list);
 
 template <class T>
 static int dalloc(e2mi_engine *g, T **p, size_t count) {
@@ -702,11 +704,12 @@ static int plan_pack(e2mi_engine *g, const uint8_t *valid, int n, int S) {
     return Mp;
 }
 
-// The kernels of a device-planned forward of about `est` rows in M of capacity, as the key of its recording:
-// for every distinct GEMM whose kernel follows the row count, which one takes it (gemm_small_route,
-// gemm_half_tiles), and how the projections run their norm_add (fused: in how many row units per workgroup,
-// 1-5, and how many of them in two launches, those of larger K first)
-long forward_signature(const e2_config &c, bool fuse_an, bool fuse_qkv, int M, int est) {
+// The kernels of a device-planned forward of B sequences of up to S tokens, about `est` rows in M of capacity,
+// as the key of its recording: for every distinct GEMM whose kernel follows the row count, which one takes it
+// (gemm_small_route, gemm_half_tiles), the attention's block size at each head_dim (attn_group_blocks), and how
+// the projections run their norm_add (fused: in how many row units per workgroup, 1-5, and how many of them in
+// two launches, those of larger K first)
+long forward_signature(const e2_config &c, bool fuse_an, bool fuse_qkv, int B, int S, int M, int est) {
     const int planned = 0;  // (any device count: the estimate is what counts here)
     const DeviceRows dr{&planned, 1, est};
     const int few = dr.few(M), H = c.n_heads;
@@ -742,6 +745,8 @@ long forward_signature(const e2_config &c, bool fuse_an, bool fuse_qkv, int M, i
         const int small = gemm_small_route(few, N, K, epi, false);
         sig = sig << 3 | (small ? small : gemm_half_tiles(dr.expected(M), N) ? 4 : 0);
     }
+    sig = sig << 3 | attn_group_blocks(few, B, S, H, c.head_dim, true);
+    if (c.full_period > 0) sig = sig << 3 | attn_group_blocks(few, B, S, H, c.full_head_dim, true);
     return sig << 8 | std::min(split, 255);
 }
 
@@ -1302,7 +1307,7 @@ extern "C" int e2mi_text_embed_batch_device(e2mi_engine *g, const int32_t *ids, 
         const auto seen = g->rows_seen.find(std::make_pair(batch, seq_len));
         const int est = seen != g->rows_seen.end() ? std::min(seen->second, cap) : cap;
         if (launch_plan_packed(s, pa) ||
-            run_shape(g, batch, seq_len, cap, true, s, true, est, forward_signature(g->cfg, g->fuse_an, g->fuse_qkv, cap, est)) ||
+            run_shape(g, batch, seq_len, cap, true, s, true, est, forward_signature(g->cfg, g->fuse_an, g->fuse_qkv, batch, seq_len, cap, est)) ||
             check_hip(hipMemcpyAsync(out, g->out, (size_t)batch * g->dout * 4, hipMemcpyDeviceToDevice, s),
                       "out D2D"))
             return -1;
