@@ -163,7 +163,15 @@ struct e2mi_engine {
     std::map<std::pair<int, int>, int> rows_seen;
     bool packed = true;
     // (sequences, seq_len, rows, bits: packed 1, split 2, planned on the device 4, forward_signature)
-    std::map<std::tuple<int, int, int, long>, hipGraphExec_t> graphs;
+    // and when each was last launched: the longest unused is dropped at kMaxForwards (a recording holds about
+    // 0.25 MB of host memory; a call that makes one takes 0.25 ms more than one that launches it)
+    struct Recorded {
+        hipGraphExec_t exec;
+        long used;
+    };
+    static constexpr size_t kMaxForwards = 1024;
+    std::map<std::tuple<int, int, int, long>, Recorded> graphs;
+    long launches = 0;
     bool use_graph = true;
     bool fuse_qkv = true;  // E2MI_NOFUSE=1: the q|k|v GEMM and the norm/RoPE kernel run separately
     bool fuse_an = true;   // E2MI_NOFUSE_AN=1: the O and down GEMMs and their norm_add run separately
@@ -604,10 +612,22 @@ static int run_shape(e2mi_engine *g, int B, int S, int Mp, bool pk, hipStream_t 
         const hipError_t ei = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
         (void)hipGraphDestroy(graph);
         if (check_hip(ei, "graph instantiate")) return -1;
-        g->graphs[key] = exec;
+        if (g->graphs.size() >= e2mi_engine::kMaxForwards) {
+            // (calls on another stream have finished, begin_call: only s can still be running it)
+            auto old = std::min_element(g->graphs.begin(), g->graphs.end(),
+                                        [](const auto &a, const auto &b) { return a.second.used < b.second.used; });
+            if (check_hip(hipStreamSynchronize(s), "recording sync")) {
+                (void)hipGraphExecDestroy(exec);
+                return -1;
+            }
+            (void)hipGraphExecDestroy(old->second.exec);
+            g->graphs.erase(old);
+        }
+        g->graphs[key] = {exec, g->launches++};
         return 0;
     }
-    return check_hip(hipGraphLaunch(it->second, s), "graph launch");
+    it->second.used = g->launches++;
+    return check_hip(hipGraphLaunch(it->second.exec, s), "graph launch");
 }
 
 static int validate_batch(const e2mi_engine *g, const int32_t *ids, int batch, int seq_len, bool host_ids) {
@@ -818,7 +838,7 @@ static int set_attention_i8(e2mi_engine *g, bool on) {
             return -1;
     }
     g->attn_i8 = on;
-    for (auto &kv : g->graphs) (void)hipGraphExecDestroy(kv.second);
+    for (auto &kv : g->graphs) (void)hipGraphExecDestroy(kv.second.exec);
     g->graphs.clear();
     return 0;
 }
@@ -830,7 +850,7 @@ extern "C" void e2mi_destroy(e2mi_engine *g) {
     if (!g) return;
     if (g->stream) (void)hipStreamSynchronize(g->stream);
     for (const ProfEv &e : g->pev) (void)hipEventDestroy(e.a), (void)hipEventDestroy(e.b);
-    for (auto &kv : g->graphs) (void)hipGraphExecDestroy(kv.second);
+    for (auto &kv : g->graphs) (void)hipGraphExecDestroy(kv.second.exec);
     for (void *p : g->allocs) (void)hipFree(p);
     if (g->h_ids) (void)hipHostFree(g->h_ids);
     if (g->h_valid) (void)hipHostFree(g->h_valid);
@@ -1447,7 +1467,7 @@ extern "C" int e2mi_set_layer_limit(e2mi_engine *g, int n_layers) {
         return -1;
     }
     g->layer_limit = n_layers;
-    for (auto &kv : g->graphs) (void)hipGraphExecDestroy(kv.second);
+    for (auto &kv : g->graphs) (void)hipGraphExecDestroy(kv.second.exec);
     g->graphs.clear();
     return 0;
 }

@@ -114,3 +114,34 @@ def test_graph_failure_then_recovery(flib, rng, kind, text):
             assert rc == 0 and np.array_equal(out, want)
     finally:
         L.e2mi_destroy(g)
+
+
+def test_recordings_are_bounded(flib, rng):
+    """More shapes (1200) than an engine keeps recordings of (1024): the longest unused one is dropped and recorded
+    again when its shape comes back, the others are launched, and every embedding stays what it was."""
+    L, m, want_eng = flib
+    ids = rng.integers(0, 1000, (3, 400)).astype(np.int32)
+    shapes = [(b, n) for n in range(1, 401) for b in (1, 2, 3)]
+    g = L.e2mi_create_rows(m, 1280)
+    assert g
+
+    def call(i):
+        b, n = shapes[i]
+        c0 = L.e2mi_fault_calls(F_INSTANTIATE)
+        rc, out = _embed(L, g, np.ascontiguousarray(ids[:b, :n]), np.ones((b, n), np.uint8))
+        assert rc == 0, L.e2mi_last_error()
+        return L.e2mi_fault_calls(F_INSTANTIATE) - c0, out
+    try:
+        first = [call(i)[1] for i in range(1200)]
+        for i in (0, 17, 700, 1199):
+            b, n = shapes[i]
+            assert np.array_equal(first[i], want_eng.embed_batch(np.ascontiguousarray(ids[:b, :n]), None))
+        assert call(176)[0] == 0  # the 1024 last are there
+        for i in (175, 3):        # their places are 177's and 178's, 176 was just used
+            made, out = call(i)
+            assert made == 1 and np.array_equal(out, first[i])
+        assert [call(i)[0] for i in (176, 1199, 177, 179)] == [0, 0, 1, 1]
+        for i in (800, 177, 178, 180):
+            assert np.array_equal(call(i)[1], first[i])
+    finally:
+        L.e2mi_destroy(g)
