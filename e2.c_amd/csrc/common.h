@@ -207,5 +207,12 @@ __device__ inline void dma4(v4u r, uint32_t lds, uint32_t voff, uint32_t soff) {
                  : "memory");
 }
 
+// at most N of the wave's vector-memory loads (and stores) still in flight
+template <int N>
+__device__ inline void vm_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+// A workgroup barrier that orders LDS only: __syncthreads() also waits for every global load and store in
+// flight (s_waitcnt vmcnt(0)), which would drain loads issued ahead and finished rows' stores.
+__device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 }  // namespace e2mi
 #endif

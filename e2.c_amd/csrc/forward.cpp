@@ -437,12 +437,12 @@ static int enqueue(e2mi_engine *g, int B, int S, int Mp, bool pk, hipStream_t s,
                              g->x, g->qa, g->as, nullptr));
     // a GEMM whose activations come from the pending norm_add of tmp (form ahead)
     NormIn pend;
-#define RUN_NORMED(name, call)                    \
-    do {                                          \
-        const NormInScope norm_scope(pend);       \
-        RUN(name, call);                          \
-        if (pend.y) std::swap(x, x_other);        \
-        pend.y = nullptr;                         \
+#define RUN_NORMED(name, call)                         \
+    do {                                               \
+        const NormInScope norm_scope(pend);            \
+        RUN(pend.y ? "add_norm+" name : name, call);   \
+        if (pend.y) std::swap(x, x_other);             \
+        pend.y = nullptr;                              \
     } while (0)
     auto ahead = [&](const float *gamma_a, float post_scale, const float *gamma_n) {
         pend = NormIn{g->tmp, x, gamma_a, gamma_n, x_other, post_scale, eps};
@@ -494,7 +494,7 @@ static int enqueue(e2mi_engine *g, int B, int S, int Mp, bool pk, hipStream_t s,
                                g->cq, g->cs, nullptr));
         }
         if (form == NORM_AHEAD) {
-            RUN("o_proj+add_norm", e2mi_i8_gemm(s, g->tmp, Dm, g->cq, g->cs, &L.o, M, 0, Dm));
+            RUN("o_proj", e2mi_i8_gemm(s, g->tmp, Dm, g->cq, g->cs, &L.o, M, 0, Dm));
             ahead(L.ln_attn, 1.0f, L.ln_pre);
         } else if (L.o_an && an) {
             RUN("o_proj+add_norm", launch_gemm_add_norm(s, g->cq, g->cs, &L.o, M, g->x, L.ln_attn, 1.0f, L.ln_pre, eps,
@@ -510,12 +510,12 @@ static int enqueue(e2mi_engine *g, int B, int S, int Mp, bool pk, hipStream_t s,
         const float *gnext = last ? g->final_norm : g->layers[l + 1].ln_in;
         if (form == NORM_AHEAD) {
             // the last norm_add has no GEMM after it that takes it: fused, into g->x and g->xn
-            if (P > 0 || !last) RUN("down+add_norm", e2mi_i8_gemm(s, g->tmp, Dm, g->qg, g->gs, &L.down, M, 0, Dm));
+            if (P > 0 || !last) RUN("down", e2mi_i8_gemm(s, g->tmp, Dm, g->qg, g->gs, &L.down, M, 0, Dm));
             if (P > 0) {
                 ahead(L.ln_ffn, 1.0f, nullptr);
                 RUN_NORMED("ple_gate", e2mi_i8_gemm_gelu_mul(s, g->qg, g->gs, nullptr, g->qa, g->as, &L.ple_gate, M,
                                                              g->ple32 + (size_t)l * P, c.n_layers * P));
-                if (!last) RUN("ple_proj+add_norm", e2mi_i8_gemm(s, g->tmp, Dm, g->qg, g->gs, &L.ple_proj, M, 0, Dm));
+                if (!last) RUN("ple_proj", e2mi_i8_gemm(s, g->tmp, Dm, g->qg, g->gs, &L.ple_proj, M, 0, Dm));
             }
             if (!last) {
                 ahead(P > 0 ? L.ple_norm : L.ln_ffn, P > 0 ? L.layer_scalar : 1.0f, gnext);
@@ -1097,7 +1097,7 @@ static void prof_flush(e2mi_engine *g) {
     snprintf(line, sizeof line, "[e2mi] kernel profile, one call (ms, total %.3f):\n", total);
     std::string text = line;
     for (size_t i = 0; i < names.size(); i++) {
-        snprintf(line, sizeof line, "[e2mi]   %-20s %9.3f ms %6ld calls %8.4f ms/call %5.1f%%\n", names[i].c_str(),
+        snprintf(line, sizeof line, "[e2mi]   %-27s %9.3f ms %6ld calls %8.4f ms/call %5.1f%%\n", names[i].c_str(),
                  ms[i], n[i], ms[i] / n[i], total > 0 ? 100.0 * ms[i] / total : 0.0);
         text += line;
     }

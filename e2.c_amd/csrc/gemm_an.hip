@@ -86,14 +86,6 @@ struct AnShape {
     static_assert(LDS <= 160 * 1024, "LDS budget");
 };
 
-// A workgroup barrier that orders LDS only: __syncthreads() also waits for every global load and
-// store in flight (s_waitcnt vmcnt(0)), which in the epilogue would drain the residual rows loaded
-// ahead and the stores of the rows already normed at every staged unit.
-__device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-template <int N>
-__device__ inline void vm_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-
 template <int D, bool SCALE, int UC, bool FAST>
 __global__ __launch_bounds__(512, 1) void k_gemm_an(const int *rows, AnArgs a) {
     using S = AnShape<D>;

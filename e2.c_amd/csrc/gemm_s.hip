@@ -18,11 +18,6 @@ namespace {
 // activation scales)
 enum { FOLD_EXACT = 0, FOLD_FAST = 1, FOLD_TOK = 2 };
 
-template <int N>
-__device__ inline void vm_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-// a barrier that orders LDS only (__syncthreads() would also wait for the loads in flight)
-__device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 // f16 of an f32 value that is already rounded (the register barrier keeps the compiler from folding
 // the multiply that produced x into the conversion)
 __device__ inline uint32_t f16_rn(float x) {

@@ -45,6 +45,20 @@ def test_profile_reports_stages(model, rng, monkeypatch):
     assert lib.e2mi_profile_text(eng.h).decode() == text
 
 
+def test_profile_names_the_norm_add_of_few_rows(model, rng, monkeypatch):
+    """Up to 256 rows a norm_add runs in the GEMM that reads it: its time is in that GEMM's line, and the
+    projections' lines are theirs alone but for the last, which norms in its epilogue."""
+    e2mi, m = model
+    monkeypatch.setenv("E2MI_PROFILE", "1")
+    eng = e2mi.Engine(m, max_rows=1024)
+    monkeypatch.delenv("E2MI_PROFILE")
+    eng.embed_batch(rng.integers(0, 1000, (1, 19)).astype(np.int32), None)
+    lines = [l.split() for l in e2mi.load().e2mi_profile_text(eng.h).decode().splitlines()[1:]]
+    calls = {f[1]: int(f[4]) for f in lines}
+    assert calls == {"embed": 1, "qkv_norm_rope_gemm": 1, "add_norm+qkv_norm_rope_gemm": 1, "attention": 2, "o_proj": 2,
+                     "add_norm+gate_up_geglu": 2, "down": 1, "down+add_norm": 1, "pool": 1}, calls
+
+
 def test_dump_after_layer_zero(model, oracle, rng, monkeypatch, tmp_path):
     e2mi, m = model
     ids, valid = random_batch(rng, 3, 100, 1000, min_len=30)
