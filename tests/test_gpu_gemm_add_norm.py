@@ -4,6 +4,9 @@ e2mi_i8_gemm then e2mi_add_norm_quant / e2mi_add_norm_scale_quant (the encoder's
 projections and the norm_add after each, text.c:944-953; the reference checkpoint's 512-wide
 projections and its PLE layers' scaled norm_add, text.c:955-961).
 
+Up to a row count that follows K the entry points run the two launches themselves, through y or x_out
+(gemm_an_split); the cases below that line with y test those, test_one_launch_at_few_rows the kernel there.
+
 Bars: every output bit-identical with the two launches (the same per-128 fold, the same row
 arithmetic), which test_gpu_gemm.py and test_gpu_rowops.py pin to the oracle; the projection y also
 bit-exact with the oracle's GEMM directly on a small case. Row counts cover one 16-row unit, ragged
@@ -115,7 +118,7 @@ def _raw(gpu, case, **over):
     qa, as_, w, ws, res, ga, gn = case
     M, K, N = *qa.shape, w.shape[0]
     W = over.pop("W", None) or e2mi.DeviceWeight.from_rowmajor(w, ws)
-    b = dict(qa=_t(qa, gpu), as_=_t(as_, gpu), res=_t(res, gpu), x=torch.empty((M, N), device=gpu), y=None,
+    b = dict(qa=_t(qa, gpu), as_=_t(as_, gpu), res=_t(res, gpu), x=torch.empty((M, N), device=gpu), xn=None, y=None,
              q=torch.empty((M, N), dtype=torch.int8, device=gpu), qs=torch.empty((M, N // 128), device=gpu))
     for k, v in over.items():
         b[k] = v(b)
@@ -123,9 +126,62 @@ def _raw(gpu, case, **over):
     tga, tgn = _t(ga, gpu), _t(gn, gpu)
     e2mi.check(e2mi.load().e2mi_i8_gemm_add_norm_quant(
         torch.cuda.current_stream().cuda_stream, p(b["qa"]), p(b["as_"]), W.ref, M, p(b["res"]), p(tga), p(tgn),
-        EPS, p(b["x"]), None, p(b["q"]), p(b["qs"]), p(b["y"])))
+        EPS, p(b["x"]), p(b["xn"]), p(b["q"]), p(b["qs"]), p(b["y"])))
     torch.cuda.synchronize()
     return b
+
+
+def _split(M, N, K):
+    import ctypes as C
+    import e2mi
+    f = e2mi.load()._ZN4e2mi13gemm_an_splitEiii
+    f.argtypes, f.restype = [C.c_int] * 3, C.c_bool
+    return f(M, N, K)
+
+
+@pytest.mark.parametrize("M,K,N,scale,kw", [
+    (1, 768, 768, None, {}), (16, 768, 768, None, {}), (17, 1152, 768, None, {}), (333, 768, 768, None, {}),
+    (1000, 1152, 768, None, {}), (50, 768, 768, None, dict(gamma_next=False)), (50, 768, 768, None, dict(want_xn=False)),
+    (50, 768, 768, None, dict(quant=False)), (1, 512, 512, None, {}), (50, 1024, 512, None, {}), (2100, 2048, 512, None, {}),
+    (5, 512, 512, 0.7373, {}), (333, 2048, 512, 1.0, dict(gamma_next=False)), (300, 512, 512, 0.2, dict(want_xn=False))])
+def test_one_launch_at_few_rows(gpu, rng, M, K, N, scale, kw):
+    """k_gemm_an where a call with y runs as two launches: x updated in the residual's place and no y leaves the
+    entry point no scratch. Every output against the GEMM and the row kernel called one after the other."""
+    import e2mi
+    assert _split(M, N, K)
+    kw = dict(kw)
+    qa, as_, w, ws, res, ga, gn = _case(rng, M, K, N)
+    W = e2mi.DeviceWeight.from_rowmajor(w, ws)
+    tqa, tas, tga = _t(qa, gpu), _t(as_, gpu), _t(ga, gpu)
+    tgn = _t(gn, gpu) if kw.pop("gamma_next", True) else None
+    kw = dict(dict(want_xn=True, quant=True), **kw)
+    r0, r1 = _t(res, gpu), _t(res, gpu)
+    y = e2mi.i8_gemm(tqa, tas, W)
+    if scale is None:
+        want = e2mi.add_norm_quant(y, r0, tga, tgn, EPS, x_out=r0, **kw)
+        got = e2mi.i8_gemm_add_norm_quant(tqa, tas, W, r1, tga, tgn, EPS, x_out=r1, **kw)
+    else:
+        want = e2mi.add_norm_scale_quant(y, r0, tga, scale, tgn, EPS, x_out=r0, **kw)
+        got = e2mi.i8_gemm_add_norm_scale_quant(tqa, tas, W, r1, tga, scale, tgn, EPS, x_out=r1, **kw)
+    for name, a, b in zip(("x", "xn", "q", "qs"), got, want):
+        assert (a is None) == (b is None), name
+        if a is not None:
+            _same(a, b, name)
+
+
+@pytest.mark.parametrize("M", [7, 333, 2100])  # two launches, then one
+def test_normed_rows_over_the_residual(gpu, rng, M):
+    """xn_out in the residual's place (the engine's last norm_add at few rows): a row's residual is read before
+    its normed row is written."""
+    import torch
+    import e2mi
+    case = _case(rng, M, 768)
+    want = _raw(gpu, case, xn=lambda b: torch.empty_like(b["res"]))
+    for over in (dict(xn=lambda b: b["res"]), dict(x=lambda b: torch.empty_like(b["res"]), y=lambda b: torch.empty_like(b["res"]),
+                                                   xn=lambda b: b["res"])):
+        got = _raw(gpu, case, **over)
+        for k in ("x", "xn", "q", "qs"):
+            _same(got[k], want[k], k)
 
 
 @pytest.mark.parametrize("M", [7, 333])
@@ -260,3 +316,40 @@ def test_engine_fused_equals_unfused_reference_geometry(gpu, rng, monkeypatch):
         fused.embed_batch_device(tid, tv, oa)
         torch.cuda.synchronize()
         assert np.array_equal(_np(oa).view(np.uint32), a.view(np.uint32)), (B, S, "device entry")
+
+
+@pytest.mark.parametrize("geom", ["base", "ref"])
+@pytest.mark.parametrize("fold", ["exact", "fast"])
+def test_engine_at_few_rows_equals_unfused(gpu, rng, monkeypatch, geom, fold):
+    """Up to 256 rows the engine runs each norm_add in the GEMM that reads it, x moving between two buffers: the
+    same embeddings bit for bit as E2MI_NOFUSE_AN=1, through the host and the device entry, at the edges of
+    the 32-row tiles and of the form, with both folds and with every layer as the last."""
+    import sys
+    import torch
+    sys.path.insert(0, __file__.rsplit("/", 1)[0])
+    from model_util import random_batch, reference_small_config, small_config
+    import e2mi
+    layers = 3 if geom == "base" else 7
+    cfg = small_config(e2mi, n_layers=layers) if geom == "base" else reference_small_config(e2mi, n_layers=layers)
+    m = e2mi.Model.synthetic(cfg, 80)
+    prev = e2mi.set_gemm_fold(fold)
+    try:
+        ahead = e2mi.Engine(m, max_rows=2048)
+        monkeypatch.setenv("E2MI_NOFUSE_AN", "1")
+        plain = e2mi.Engine(m, max_rows=2048)
+        monkeypatch.delenv("E2MI_NOFUSE_AN")
+        for B, S in [(1, 1), (1, 8), (1, 19), (1, 33), (1, 100), (3, 64), (1, 256), (1, 257), (8, 32)]:
+            ids, valid = random_batch(rng, B, S, 1000, min_len=S if B == 1 else 1)
+            a, b = ahead.embed_batch(ids, valid), plain.embed_batch(ids, valid)
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), (B, S)
+            out = torch.empty((B, 768), device=gpu)
+            ahead.embed_batch_device(torch.from_numpy(ids).to(gpu), torch.from_numpy(valid).to(gpu), out)
+            torch.cuda.synchronize()
+            assert np.array_equal(_np(out).view(np.uint32), a.view(np.uint32)), (B, S, "device entry")
+        ids = rng.integers(0, 1000, (1, 50)).astype(np.int32)
+        for n in range(1, layers + 1):
+            ahead.set_layer_limit(n)
+            plain.set_layer_limit(n)
+            assert np.array_equal(ahead.embed_batch(ids, None), plain.embed_batch(ids, None)), n
+    finally:
+        e2mi.set_gemm_fold(prev)

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
-BIG = 17408  # rows the large tiles take at every width here
+BIG = 17408  # rows the large tiles take at every width here but (K, N) = (128, 40), which the oracle covers
 
 
 def _t(a, dev):
@@ -182,6 +182,66 @@ def test_ring_f32(gpu, oracle, rng, K, N, rows):
                 _same([y], [full[:M]], f"{mode} M={M}, clamped columns")
         finally:
             e2mi.set_gemm_fold(prev)
+
+
+def _route(M, N, K, epi=0, tok=False):
+    import ctypes as C
+    import e2mi
+    f = e2mi.load()._ZN4e2mi16gemm_small_routeEiiiib
+    f.argtypes, f.restype = [C.c_int] * 4 + [C.c_bool], C.c_int
+    return f(M, N, K, epi, tok)
+
+
+# every f32 kernel by the rule's own word (0: gemm.hip's tiles; K-split, 32 rows, 64 rows, ring), all rows against
+# the oracle bit for bit; the 64-row ones under the fast fold against the large tiles too
+@pytest.mark.parametrize("route,K,N,M", [(1, 128, 40, 513), (1, 128, 40, 4100), (1, 768, 768, 1030), (2, 2560, 512, 257),
+                                         (2, 2048, 256, 2048), (3, 384, 768, 2400), (3, 384, 256, 8149), (3, 512, 1024, 1921),
+                                         (5, 2048, 512, 4096), (0, 384, 768, 6000)])
+def test_f32_routes_against_the_oracle(gpu, oracle, rng, route, K, N, M):
+    import e2mi
+    assert _route(M, N, K) == route
+    qa, as_, w, ws, b, W = _ops(rng, gpu, K, N, True)
+    y = e2mi.i8_gemm(qa[:M], as_[:M], W)
+    want = oracle.i8_gemm(qa[:M].cpu().numpy(), as_[:M].cpu().numpy(), w, ws, bias=b)
+    assert np.array_equal(y.cpu().numpy().view(np.uint32), want.view(np.uint32))
+    if route == 3:
+        assert _route(BIG, N, K) == 0
+        prev = e2mi.set_gemm_fold("fast")
+        try:
+            _same([e2mi.i8_gemm(qa[:M], as_[:M], W)], [e2mi.i8_gemm(qa, as_, W)[:M]], "fast fold")
+        finally:
+            e2mi.set_gemm_fold(prev)
+
+
+@pytest.mark.parametrize("M", [33, 1664])  # 32- and 64-row tiles
+def test_small_epilogues_under_the_fast_fold(gpu, rng, M):
+    import e2mi
+    import torch
+    K, H, KV = 768, 4, 2
+    N = (H + 2 * KV) * 256
+    qa, as_, w, ws, b, W = _ops(rng, gpu, K, N)
+    _, _, _, _, _, Wk = _ops(rng, gpu, K, K)
+    g = torch.Generator(device=gpu).manual_seed(17)
+    mul = torch.randn((BIG, K), generator=g, device=gpu)
+    qg, kg = (torch.rand(256, generator=g, device=gpu) + 0.5 for _ in range(2))
+    cs, sn = (torch.rand((64, 256), generator=g, device=gpu) for _ in range(2))
+    pos = torch.randint(0, 64, (BIG,), generator=g, device=gpu, dtype=torch.int32)
+    for epi, n in ((1, K), (2, N), (3, K), (4, N)):
+        assert _route(M, n, K, epi) != 0 and _route(BIG, n, K, epi) == 0, epi
+
+    def run(m):
+        qkv = e2mi.i8_gemm_qkv(qa[:m], as_[:m], W, H, KV, qg, kg, cs, sn, pos=pos[:m].contiguous(), want_f32=True)
+        return [*e2mi.i8_gemm_q(qa[:m], as_[:m], Wk), *e2mi.i8_gemm_geglu(qa[:m], as_[:m], W),
+                *e2mi.i8_gemm_gelu_mul(qa[:m], as_[:m], Wk, mul[:m]), *qkv]
+
+    exact = run(M)
+    prev = e2mi.set_gemm_fold("fast")
+    try:
+        few, big = run(M), run(BIG)
+    finally:
+        e2mi.set_gemm_fold(prev)
+    _same(few, [o[..., :M] if o.dim() == 4 else o[:M] for o in big], "fast fold")  # (V^T: [1][KV][D][M])
+    assert any(not torch.equal(a, b) for a, b in zip(few, exact))  # (the mode was on)
 
 
 @pytest.mark.parametrize("K", [44800, 44928])  # the last K whose scales fit k_gemm_ring's LDS, and the next
