@@ -164,22 +164,23 @@ constexpr int kI8Keep = 512;
 constexpr int kI8P = 0, kI8M = 4096, kI8L = kI8M + 1024, kI8X = kI8L + 2048;  // bytes, maxima, partial sums
 constexpr int kI8V = 8 * kI8Buf, kI8S = kI8V + kI8D * 4, kAttnI8Lds = kI8S + kI8X;
 
-template <bool KEEP>
+// WALK: a workgroup runs its entry's blocks one after the other (a kernel of its own: the loop costs the others
+// 40 registers and 1-3 %).
+template <bool KEEP, bool WALK>
 __global__ __launch_bounds__(256, 2) void k_attn_i8(AttnI8Args a, int n_work, int nwg) {
     extern __shared__ __align__(16) unsigned char smem[];
-    int q0 = blockIdx.x * 32, q1 = q0 + 32, h = blockIdx.y, b = blockIdx.z;
-    if (a.work) {  // work entry i's blocks on one XCD (i % 8), dealt to nwg workgroups
+    int q0 = blockIdx.x * 32, h = blockIdx.y, b = blockIdx.z;
+    if (WALK || a.work) {  // work entry i's nwg workgroups on one XCD (i % 8)
         const int i = (blockIdx.x / (8 * nwg)) * 8 + (blockIdx.x & 7);
         const int item = i < n_work ? a.work[i] : -1;
         if (item < 0) return;
         b = item & 0xffff;
         h = (item >> 16) & 0xf;  // (one part: work_entry(b, h, 0, 1, query block))
-        q1 = (item >> 24) * 128 + 128;
-        q0 = q1 - 128 + ((blockIdx.x >> 3) % nwg) * 32;
+        q0 = (item >> 24) * 128 + ((blockIdx.x >> 3) % nwg) * 32;
     }
-    for (; q0 < min(a.seq_len[b], q1); q0 += 32 * nwg) {
+    for (const int q1 = q0 + (WALK ? 128 : 32); q0 < min(a.seq_len[b], q1); q0 += 32) {
         int tid = threadIdx.x;
-        asm volatile("" : "+v"(tid), "+s"(b));  // (nothing of a block is kept in registers for the next)
+        if constexpr (WALK) asm volatile("" : "+v"(tid), "+s"(b));  // (nothing of a block is kept in registers for the next)
         const int Sk = a.seq_len[b];
         const int lane = tid & 63, half = lane >> 5, ql = lane & 31;
         const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -423,30 +424,35 @@ __global__ __launch_bounds__(256, 2) void k_attn_i8(AttnI8Args a, int n_work, in
                 }
             if (half == 0 && !(w & 1)) a.cs[orow * (HD / kQBlock) + h * 2 + (w >> 1)] = qs.sc;
         }
+        if constexpr (!WALK) return;
     }
 }
 
 static size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-template <bool KEEP>
-static int launch_attn_i8(hipStream_t s, const AttnI8Args &a, int B, int max_len, int n_work) {
+template <bool KEEP, bool WALK>
+static int launch_attn_i8(hipStream_t s, const AttnI8Args &a, int B, int max_len, int n_work, int nwg) {
     static bool attr = false;
     if (!attr) {
-        if (check_hip(hipFuncSetAttribute((const void *)k_attn_i8<KEEP>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        if (check_hip(hipFuncSetAttribute((const void *)k_attn_i8<KEEP, WALK>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                           kAttnI8Lds), "attention_i8 lds attribute"))
             return -1;
         attr = true;
     }
-    // A work entry has four blocks of 32 queries, fewer where no sequence is that long, each a workgroup's: one
-    // whose block lies past its sequence costs 1-2 us of a CU's slot (300 x 1-66, 3 heads: 71.2 us with four
-    // workgroups an entry, 43.3 with three). From three entries a CU of sequences of at most 128, one
-    // workgroup walks an entry's blocks instead (four | one: 3 heads, 300 x 1-128 86.8 | 65.8; 15 heads, 64 x 8-100
-    // 83.9 | 60.9, 128 x 100-128 220.5 | 216.8; with fewer, 3 heads, 128 x 100-128 50.8 | 55.2).
-    int nwg = std::min(4, (max_len + 31) / 32);
-    if (max_len <= 128 && n_work >= 3 * num_cus()) nwg = 1;
     const dim3 grid = a.work ? dim3((n_work + 7) / 8 * 8 * nwg) : dim3((max_len + 31) / 32, a.H, B);
-    hipLaunchKernelGGL(k_attn_i8<KEEP>, grid, dim3(256), kAttnI8Lds, s, a, n_work, nwg);
+    hipLaunchKernelGGL((k_attn_i8<KEEP, WALK>), grid, dim3(256), kAttnI8Lds, s, a, n_work, nwg);
     return check_hip(hipGetLastError(), "attention_i8 launch");
+}
+// A work entry has four blocks of 32 queries, fewer where no sequence is that long, each a workgroup's: one
+// whose block lies past its sequence costs 1-2 us of a CU's slot (300 x 1-66, 3 heads: 71.2 us with four
+// workgroups an entry, 43.3 with three). From three entries a CU of sequences of at most 128, one
+// workgroup walks an entry's blocks instead (four | one: 3 heads, 300 x 1-128 86.8 | 65.8; 15 heads, 64 x 8-100
+// 83.9 | 60.9, 128 x 100-128 220.5 | 216.8; with fewer, 3 heads, 128 x 100-128 50.8 | 55.2).
+static int launch_attn_i8(hipStream_t s, const AttnI8Args &a, int B, int max_len, int n_work) {
+    if (a.work && max_len <= 128 && n_work >= 3 * num_cus()) return launch_attn_i8<true, true>(s, a, B, max_len, n_work, 1);
+    const int nwg = std::min(4, (max_len + 31) / 32);
+    return max_len <= kI8Keep ? launch_attn_i8<true, false>(s, a, B, max_len, n_work, nwg)
+                              : launch_attn_i8<false, false>(s, a, B, max_len, n_work, nwg);
 }
 
 struct I8Ws {
@@ -512,5 +518,5 @@ extern "C" int e2mi_attention_i8_packed(e2mi_stream stream, const float *q32, co
     hipLaunchKernelGGL(k_i8_prep, dim3((unsigned)row, (unsigned)((prep + row - 1) / row)), dim3(256), 0, s, p);
     hipLaunchKernelGGL(k_i8_vquant, dim3(B * KV, (max_len + 31) / 32), dim3(256), 0, s, p);
     const AttnI8Args a = {p.q8, p.qs, p.k8, p.ks, p.vt8, p.vs, ctx_q, ctx_s, ctx32, seq_start, seq_len, work, M, H, KV};
-    return max_len <= kI8Keep ? launch_attn_i8<true>(s, a, B, max_len, n_work) : launch_attn_i8<false>(s, a, B, max_len, n_work);
+    return launch_attn_i8(s, a, B, max_len, n_work);
 }
