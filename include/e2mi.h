@@ -156,10 +156,12 @@ int e2mi_add_norm_quant(e2mi_stream stream, const float *src, const float *res,
 /* A projection that feeds a norm_add, with the norm_add in its epilogue: y = e2mi_i8_gemm(qa, w)
  * (w: N = D = 768 or 512 rows, K a multiple of 128, no bias or clamp), then
  * e2mi_add_norm_quant(y, res, gamma_add, gamma_next, eps, M, D, x_out, xn_out, q, qs), with the same
- * bits as those two calls and without y in memory (the text tower's O and down projections and the
- * norm_add after each, text.c:944-953; the reference computes them as two passes, so this entry
- * point has no single counterpart). y [M][D] f32 is also written when non-NULL (parity tests).
- * x_out may alias res. */
+ * bits as those two calls (the text tower's O and down projections and the norm_add after each,
+ * text.c:944-953; the reference computes them as two passes, so this entry point has no single
+ * counterpart). y [M][D] f32 is also written when non-NULL. Above a row count that follows K it is one
+ * launch and y goes through no memory of its own. Below, where two launches are faster, the projection goes
+ * through y, or without y through x_out (which is then written twice), where that lies apart from res,
+ * qa and a_scales; elsewhere it stays one launch. x_out, xn_out and y may each alias res. */
 int e2mi_i8_gemm_add_norm_quant(e2mi_stream stream, const int8_t *qa, const float *a_scales,
                                 const e2mi_q8w *w, int M, const float *res, const float *gamma_add,
                                 const float *gamma_next, float eps, float *x_out, float *xn_out,
@@ -448,9 +450,11 @@ int e2mi_stats(e2mi_engine *g, long *calls, long *kernels_last, double *last_ms)
 const char *e2mi_profile_text(const e2mi_engine *g);
 /* Split key ranges in the engine's attention (head_dim-256 layers; e2mi_attention_packed_split): a
  * 128-query block whose keys span more than 8 tiles of 32 is shared out over up to 4 workgroups and
- * merged. mode 0 never (the default), 1 always, 2 only for chunks whose unsplit blocks fill at most
- * half of the device's attention workgroups (few sequences: a single 2048-token document at the
- * reference geometry 5.77 -> 4.87 ms; a full config-4 batch would lose 14 %). E2MI_SPLIT=0|1|auto
+ * merged. mode 0 never (the default), 1 always, 2 only for chunks whose unsplit 128-query blocks fill at
+ * most half of the device's attention workgroups (few sequences). The unsplit attention runs few
+ * sequences in smaller blocks and is the faster one for most of them (one sequence, BASELINE geometry, unsplit
+ * and mode 2: 1.30 and 1.49 ms at 512 tokens, 2.48 and 2.32 at 2048; reference geometry 3.21 and 3.34 at
+ * 2048); a full config-4 batch would lose 14 %. E2MI_SPLIT=0|1|auto
  * sets it at creation. Split results differ from unsplit ones by f16 rounding, so under mode 2 a
  * long sequence's embedding depends on its batch-mates (alone it may split, in a full batch it does
  * not); modes 0 and 1 keep every sequence's embedding independent of the batch, as the reference's
@@ -465,7 +469,8 @@ int e2mi_set_packing(e2mi_engine *g, int on);
 /* Where the device entry plans a packed batch: 1 (the default) on the device (e2mi_plan_device's
  * kernel, whenever the whole batch fits the workspace at any mask, the plan fits the planner's
  * workgroup, and neither the int8 attention, split key ranges nor E2MI_DUMP is on): the call reads
- * nothing back and one recorded forward per (batch, seq_len) serves every mask, its kernels
+ * nothing back and one recorded forward per (batch, seq_len) and choice of kernels (which follow the row
+ * count of the shape's last finished call) serves every mask, its kernels
  * reading the planned row count from device memory; 0 on the host, as e2mi_text_embed_batch does
  * (the mask read back, a forward recorded per packed row count). The embeddings are the same bit
  * for bit. E2MI_DEVICE_PLAN=0 sets 0 at creation. No counterpart in the reference. */
