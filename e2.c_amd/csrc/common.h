@@ -41,8 +41,8 @@ struct DeviceRows {
     // The count at which the kernels and forms for few rows are chosen: at least half of the capacity. Their
     // grids are laid out for the capacity, a workgroup a tile, so that far below it most of a launch is
     // workgroups that find no row, and a batch near the capacity after small ones would run in tiles
-    // for a few rows. BASELINE geometry, 64 x 512 of capacity, us a call at half of the capacity | at the
-    // estimate: 100 valid tokens 1749 | 15069, 10-12 thousand after 100 5720 | 25030.
+    // for a few rows. BASELINE geometry, 64 x 512 of capacity, us a call chosen so | at the estimate alone:
+    // 100 valid tokens 1774 | 15051, a full batch after them 7418 | 24961.
     int few(int M) const {
         const int e = expected(M);
         return e > M / 2 ? e : (M + 1) / 2;
